@@ -102,14 +102,15 @@ def _affine(g, count, rows, cols, bits, scale_mean, scale_std):
     return [words, scales, (scales.float() * -centre).bfloat16()]
 
 
-def _experts(g, desc, count, inter):
-    """The tensors of `count` experts in the order of a blob's slots."""
+def _experts(g, desc, count, inter, small=False):
+    """The tensors of `count` experts in the order of a blob's slots. `small`: down weights that
+    keep a block's output well below the residual, as a trained stack does."""
     H, quant = desc.hidden, desc.quant
     if quant == MXFP4:
         out = []
-        for rows, cols in ((2 * inter, H), (H, inter)):
+        for rows, cols, low in ((2 * inter, H, 119), (H, inter, 112 if small else 119)):
             out += [_bytes(g, (count, rows, cols // 32, 16)),
-                    torch.randint(119, 124, (count, rows, cols // 32), dtype=torch.uint8, device="cuda:0", generator=g),
+                    torch.randint(low, low + 5, (count, rows, cols // 32), dtype=torch.uint8, device="cuda:0", generator=g),
                     _normal(g, (count, rows), 0.02)]
         return out
     if quant == BF16:
@@ -120,11 +121,11 @@ def _experts(g, desc, count, inter):
             for t in _affine(g, count, rows, cols, bits, scale, 0.2 * scale)]
 
 
-def _layer_tensors(desc, seed, part, zipf=0.0):
+def _layer_tensors(desc, seed, part, zipf=0.0, small=False):
     """One layer's weights as separate tensors on the GPU."""
     g = _generator(seed, 100 + part)
     H, E = desc.hidden, desc.experts
-    t = {"experts": _experts(g, desc, E, desc.intermediate)}
+    t = {"experts": _experts(g, desc, E, desc.intermediate, small)}
     if desc.shared_intermediate:
         # The published quantised builds store this router and gate as 8-bit affine rows.
         t["shared"] = _experts(g, desc, 1, desc.shared_intermediate)
@@ -243,7 +244,7 @@ def prepare(case, seed):
     else:
         desc = F.CONFIGS[case["config"]]
         hidden, norms = _block_inputs(desc, seed, case["tokens"], case["layers"])
-        layers = [(_resident(desc, _layer_tensors(desc, seed, i)),
+        layers = [(_resident(desc, _layer_tensors(desc, seed, i, small=True)),
                    {k: _bits(v) if torch.is_tensor(v) else v for k, v in n.items()}, dense)
                   for i, (n, dense) in enumerate(norms)]
         s = {"runner": Runner(ctx, layers), "embedded": hidden, "hidden": torch.empty_like(hidden)}
@@ -317,9 +318,10 @@ def tolerance(case):
     if case["kind"] == "attention":
         return {"rel": 2e-6, "max": 1e-4}
     if case["kind"] == "stack":
-        # Each block rounds its input to bf16: a last bit in one layer flips roundings, and now
-        # and then a near tie of the router, in the next. 2.2e-4 over 4 layers, 1.3e-2 over 24.
-        return {"rel": 1e-3, "max": 5e-2} if case["layers"] <= 4 else {"rel": 3e-2, "max": 0.99}
+        # Each block rounds its input to bf16: a last bit in one layer flips roundings in the next
+        # (2e-4 over 4 layers, 8e-4 over 24), and now and then a near tie of a router: then a
+        # token goes to another expert, 1e-2 to 5e-2.
+        return {"rel": 3e-2, "max": 0.99}
     rel = {MXFP4: 1.5e-4, BF16: 1e-5}.get(F.CONFIGS[case["config"]].quant, 2e-5)
     return {"rel": rel, "max": 40 * rel, "differ": 0.0}
 
@@ -410,7 +412,7 @@ def exact(case, seed):
     for i, (n, dense) in enumerate(norms):
         x = _rmsnorm64(hidden, n["pre_norm"], n["eps"]).bfloat16()
         gemma = desc.router == F.ROUTER_GEMMA
-        y = _layer_64(desc, _layer_tensors(desc, seed, i), x, hidden.bfloat16() if gemma else None)[0]
+        y = _layer_64(desc, _layer_tensors(desc, seed, i, small=True), x, hidden.bfloat16() if gemma else None)[0]
         if gemma:
             both = _rmsnorm64(dense, n["post_dense_norm"], n["eps"]) + _rmsnorm64(y, n["post_expert_norm"], n["eps"])
             hidden = (hidden + _rmsnorm64(both, n["post_norm"], n["eps"])) * n["layer_scalar"].double()
