@@ -161,9 +161,9 @@ struct Scratch {
 constexpr int kSmallT = 16;  // batches up to this size take the decode kernels
 
 int token_tile_nt(const hh_moe_desc &d, int T) {
-  // Prefill work items of 16·nt tokens: MXFP4 32 or 64 (below), BF16 64 once experts
-  // average 64 tokens or more (the weight tile is then read once per 64 tokens), else 32.
-  if (d.quant == HH_QUANT_BF16 && (int64_t)T * d.top_k >= 64 * (int64_t)d.experts) return 4;
+  // Prefill work items of 16·nt tokens: MXFP4 32 or 64 (below), BF16 160 once experts
+  // average 40 tokens or more (the weight tile is then read once per 160 tokens), else 32.
+  if (d.quant == HH_QUANT_BF16 && (int64_t)T * d.top_k >= 40 * (int64_t)d.experts) return 10;
   // MXFP4 without a shared expert, experts averaging 16 or more tokens, rows long enough for the
   // LDS rings: 64-token items for the gate-up (its 256 × 64 tiles skip the MFMAs of padding token
   // tiles, and an expert's rows are read once per 64 tokens); the down product runs the same

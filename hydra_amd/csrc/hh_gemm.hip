@@ -46,6 +46,7 @@
 #include "hh_common.hpp"
 #include "hh_select.hpp"
 #include "hh_logit.hpp"
+#include "hh_mfma.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -53,336 +54,6 @@
 #include <vector>
 
 namespace hh {
-
-enum { PH_UP = 0, PH_DOWN = 1 };
-
-__device__ __forceinline__ f32x4 mfma(const bf16x8 &a, const bf16x8 &b, const f32x4 &c) {
-  return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// Two unsigned integers < 256 → packed bf16 pair (exact: 8 significant bits).
-__device__ __forceinline__ uint32_t u8pair_to_bf16x2(uint32_t lo, uint32_t hi) {
-  uint32_t a = __float_as_uint((float)lo), b = __float_as_uint((float)hi);
-  return (a >> 16) | (b & 0xFFFF0000u);
-}
-
-// 8 4-bit MLX values of one word (low-order first) → bf16 integers.
-__device__ __forceinline__ bf16x8 mlx4_to_bf16(uint32_t w) {
-  u32x4 r;
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    r[k] = u8pair_to_bf16x2((w >> (8 * k)) & 0xF, (w >> (8 * k + 4)) & 0xF);
-  return as_bf16x8(r);
-}
-
-// 8 8-bit MLX values of two words → bf16 integers.
-__device__ __forceinline__ bf16x8 mlx8_to_bf16(uint32_t w0, uint32_t w1) {
-  u32x4 r = {u8pair_to_bf16x2(w0 & 0xFF, (w0 >> 8) & 0xFF),
-             u8pair_to_bf16x2((w0 >> 16) & 0xFF, w0 >> 24),
-             u8pair_to_bf16x2(w1 & 0xFF, (w1 >> 8) & 0xFF),
-             u8pair_to_bf16x2((w1 >> 16) & 0xFF, w1 >> 24)};
-  return as_bf16x8(r);
-}
-
-template <int FMT> struct Fmt;
-
-// ---- MXFP4: 128-column chunks, one 16-byte block per lane -----------------------------------
-template <> struct Fmt<Q_MXFP4> {
-  static constexpr int CHUNK = 128, NB = 4;  // B vectors (16 B) per lane per chunk
-  struct A { u32x4 w; uint32_t s; };
-  struct Row { const uint8_t *w; const uint8_t *s; };
-  __device__ static Row row(const uint8_t *blocks, const uint8_t *scales, int r, int K) {
-    return {blocks + (size_t)r * (K / 2), scales + (size_t)r * (K / 32)};
-  }
-  __device__ static void load(A &a, const Row &rw, int c, int g, int K) {
-    int kb = min(4 * c + g, K / 32 - 1);
-    a.w = *(const u32x4 *)(rw.w + kb * 16);
-    a.s = rw.s[kb];
-  }
-  __device__ static int bcol(int c, int g, int K) { return min(128 * c + 32 * g, K - 32); }
-  __device__ static bool lane_valid(int c, int g, int K) { return 128 * c + 32 * g < K; }
-};
-
-// ---- MXFP4 blocks without their scales (decode kernels stage a tile's scales in LDS) ----------
-constexpr int Q_MXFP4_W = 4;
-// Rows are read through a buffer resource over the whole weight matrix of the expert: the lane's
-// row offset is computed once and a chunk's offset (64 bytes per chunk) goes into the
-// instruction's immediate field, so a stream of chunks costs no address registers. Chunks are
-// not clamped: a lane past K reads the next row (its weights are zeroed by lane_valid) and reads
-// past the matrix return zeros. Streams of this format walk K with stride 1.
-template <> struct Fmt<Q_MXFP4_W> {
-  static constexpr int CHUNK = 128, NB = 4;
-  struct A { u32x4 w; };
-  struct Row {
-    __amdgpu_buffer_rsrc_t rs;
-    int voff;   // row · K/2 + 16·(lane group): the lane's block of chunk 0
-  };
-  __device__ static Row row(const uint8_t *matrix, uint64_t bytes, int r, int K) {
-    Row rw;
-    rw.rs = __builtin_amdgcn_make_buffer_rsrc((void *)matrix, (short)0, (int)bytes, 0x00020000);
-    rw.voff = r * (K / 2) + 16 * ((threadIdx.x & 63) >> 4);
-    return rw;
-  }
-  __device__ static void load(A &a, const Row &rw, int c, int, int) {
-    a.w = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rw.rs, rw.voff + 64 * c, 0, 0));
-  }
-  __device__ static bool lane_valid(int c, int g, int K) { return 128 * c + 32 * g < K; }
-};
-
-// ---- BF16: 128-column chunks; step v (32 columns) of a chunk holds, in lane (g, l16), row l16's
-// columns 128c + 32v + 8g .. +7: a lane's four 16-byte pieces lie 64 bytes apart, so a load of
-// one step reads 64 contiguous bytes of each of 16 rows. K is a multiple of 64: a step lies wholly
-// inside or wholly past K, and steps past K are skipped (uniformly) by every kernel.
-template <> struct Fmt<Q_BF16> {
-  static constexpr int CHUNK = 128, NB = 4, VS = 32;   // VS: B columns between steps
-  struct A { u32x4 w[4]; };
-  struct Row { const uint8_t *w; };
-  __device__ static Row row(const uint8_t *base, int r, int K) { return {base + (size_t)r * K * 2}; }
-  __device__ static void load(A &a, const Row &rw, int c, int g, int K) {
-#pragma unroll
-    for (int s = 0; s < 4; ++s) a.w[s] = *(const u32x4 *)(rw.w + 2 * min(128 * c + 32 * s + 8 * g, K - 8));
-  }
-  __device__ static int bcol(int c, int g, int) { return 128 * c + 8 * g; }
-  __device__ static bool step_ok(int c, int v, int K) { return 128 * c + 32 * v < K; }
-};
-
-// ---- MLX affine: 64-column chunks (one group) ------------------------------------------------
-// The lane's stage also carries its row's group scale and bias (bf16 pair); the D rows' values
-// are fetched from the lanes of those rows by shuffle (affine_sb).
-template <int BITS> struct FmtMLX {
-  static constexpr int CHUNK = 64, NB = 2, VS = 8;
-  struct A { uint32_t w[BITS / 2]; uint32_t sb; };  // 4-bit: 2 words (16 values); 8-bit: 4 words
-  struct Row { const uint8_t *w; const uint16_t *sc, *bi; };
-  __device__ static Row row(const uint8_t *words, const uint8_t *scales, const uint8_t *biases,
-                            int r, int K) {
-    return {words + (size_t)r * (K * BITS / 8), (const uint16_t *)scales + (size_t)r * (K / 64),
-            (const uint16_t *)biases + (size_t)r * (K / 64)};
-  }
-  __device__ static void load(A &a, const Row &rw, int c, int g, int K) {
-    const uint8_t *p = rw.w + (64 * c + 16 * g) * BITS / 8;
-    if constexpr (BITS == 4) {
-      u32x2 v = *(const u32x2 *)p;
-      a.w[0] = v[0]; a.w[1] = v[1];
-    } else {
-      u32x4 v = *(const u32x4 *)p;
-      a.w[0] = v[0]; a.w[1] = v[1]; a.w[2] = v[2]; a.w[3] = v[3];
-    }
-    a.sb = (uint32_t)rw.sc[c] | ((uint32_t)rw.bi[c] << 16);
-  }
-  // The codes only (the group's scale and bias come from elsewhere: MlxSb).
-  __device__ static void load_w(A &a, const Row &rw, int c, int g, int K) {
-    const uint8_t *p = rw.w + (64 * c + 16 * g) * BITS / 8;
-    if constexpr (BITS == 4) {
-      u32x2 v = *(const u32x2 *)p;
-      a.w[0] = v[0]; a.w[1] = v[1];
-    } else {
-      u32x4 v = *(const u32x4 *)p;
-      a.w[0] = v[0]; a.w[1] = v[1]; a.w[2] = v[2]; a.w[3] = v[3];
-    }
-    a.sb = 0u;
-  }
-  __device__ static bf16x8 decode(const A &a, int j) {
-    if constexpr (BITS == 4) return mlx4_to_bf16(a.w[j]);
-    else return mlx8_to_bf16(a.w[2 * j], a.w[2 * j + 1]);
-  }
-  __device__ static int bcol(int c, int g, int) { return 64 * c + 16 * g; }
-};
-template <> struct Fmt<Q_MLX4> : FmtMLX<4> {};
-template <> struct Fmt<Q_MLX8> : FmtMLX<8> {};
-
-template <int FMT> constexpr bool is_mlx() { return FMT == Q_MLX4 || FMT == Q_MLX8; }
-
-// ---- shared pieces of the canonical arithmetic -------------------------------------------------
-
-// Sum of 8 bf16 values of one 16-byte vector, in index order.
-__device__ __forceinline__ float sum8_bf16(const u32x4 &v) {
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    s += bf16_bits_to_f32(v[k] & 0xFFFF);
-    s += bf16_bits_to_f32(v[k] >> 16);
-  }
-  return s;
-}
-
-// One 16-row A tile of a wave: the lane's weight row.
-template <int FMT> struct ATile {
-  typename Fmt<FMT>::Row row;
-};
-
-// Tiles of a wave whose first output row is rb: PH_UP takes RT gate tiles then RT up tiles of
-// intermediates rb + 16q, PH_DOWN RT tiles of hidden rows rb + 16q. Rows past out_dim are
-// clamped into the matrix (their results are never stored).
-// One 16-row A tile: output rows r0 .. r0+15 (lane l16 takes r0 + l16); PH_UP picks the gate
-// (is_up false) or the up matrix.
-template <int PH, int FMT>
-__device__ __forceinline__ ATile<FMT> tile_of(const uint8_t *blob, const ExpertGroup &grp, int r0, bool is_up,
-                                              int K, int l16) {
-  ATile<FMT> t;
-  const int orow = r0 + l16;
-  const int I = grp.inter;
-  if constexpr (FMT == Q_MXFP4) {
-    // GPT-OSS gate_up rows interleave gate and up (ReferenceLayer.swift:11).
-    if (PH == PH_UP) t.row = Fmt<FMT>::row(blob + grp.off[0], blob + grp.off[1], 2 * orow + (is_up ? 1 : 0), K);
-    else t.row = Fmt<FMT>::row(blob + grp.off[3], blob + grp.off[4], orow, K);
-  } else if constexpr (FMT == Q_MXFP4_W) {
-    // The matrix extends to the next sub-tensor of the blob (its scales).
-    if (PH == PH_UP) t.row = Fmt<FMT>::row(blob + grp.off[0], grp.off[1] - grp.off[0], 2 * orow + (is_up ? 1 : 0), K);
-    else t.row = Fmt<FMT>::row(blob + grp.off[3], grp.down_bytes ? grp.down_bytes : grp.off[4] - grp.off[3], orow, K);
-  } else if constexpr (FMT == Q_BF16) {
-    // Gemma gate_up: gate = rows 0..I-1, up = rows I..2I-1 (Gemma4Weights.swift:107-112).
-    if (PH == PH_UP) t.row = Fmt<FMT>::row(blob + grp.off[0], orow + (is_up ? I : 0), K);
-    else t.row = Fmt<FMT>::row(blob + grp.off[1], orow, K);
-  } else {
-    const int mat = (PH == PH_UP) ? (is_up ? 1 : 0) : 2;
-    t.row = Fmt<FMT>::row(blob + grp.off[3 * mat], blob + grp.off[3 * mat + 1], blob + grp.off[3 * mat + 2],
-                          orow, K);
-  }
-  return t;
-}
-
-template <int PH, int FMT, int RT>
-__device__ __forceinline__ void wave_tiles(ATile<FMT> (&t)[(PH == PH_UP ? 2 : 1) * RT],
-                                           const uint8_t *blob, const ExpertGroup &grp, int rb,
-                                           int out_dim, int K, int l16) {
-  constexpr int NM = (PH == PH_UP ? 2 : 1) * RT;
-#pragma unroll
-  for (int m = 0; m < NM; ++m)
-    t[m] = tile_of<PH, FMT>(blob, grp, min(rb + 16 * (m % RT), out_dim - 16), (PH == PH_UP) && (m >= RT), K, l16);
-}
-
-// The MFMA sequence of chunk c for NM A tiles × NT token tiles. `bv(st, hh, v)` returns the
-// lane's 8 B values of token tile st, term hh (x | h_hi, h_lo), step v, at columns
-// Fmt::bcol(c, g, K) + 8v.
-// MLX: `sbf(m)`, when given, returns the (scale | bias << 16) words of D rows 4g .. 4g+3 of tile m
-// for this chunk; otherwise they come from the A operands' rows by shuffles.
-template <int FMT, int NM, int NT, int NH, class BV, class SBF = std::nullptr_t>
-__device__ __forceinline__ void chunk_mfma(f32x4 (&acc)[NM][NT], const typename Fmt<FMT>::A (&w)[NM],
-                                           const ATile<FMT> (&at)[NM], BV bv, int c, int g, int K,
-                                           SBF sbf = nullptr) {
-  using F = Fmt<FMT>;
-  if constexpr (FMT == Q_BF16) {
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      if (!F::step_ok(c, v, K)) break;
-      u32x4 b[NT][NH];
-#pragma unroll
-      for (int st = 0; st < NT; ++st)
-#pragma unroll
-        for (int hh = 0; hh < NH; ++hh) b[st][hh] = bv(st, hh, v);
-#pragma unroll
-      for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int st = 0; st < NT; ++st)
-#pragma unroll
-          for (int hh = 0; hh < NH; ++hh) acc[m][st] = mfma(as_bf16x8(w[m].w[v]), as_bf16x8(b[st][hh]), acc[m][st]);
-    }
-  } else if constexpr (!is_mlx<FMT>()) {
-    const bool ok = F::lane_valid(c, g, K);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      u32x4 b[NT][NH];
-#pragma unroll
-      for (int st = 0; st < NT; ++st)
-#pragma unroll
-        for (int hh = 0; hh < NH; ++hh) b[st][hh] = bv(st, hh, v);
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        bf16x8 av;
-        av = mxfp4_to_bf16(ok ? w[m].w[v] : 0u, e8m0_to_f32(w[m].s));
-#pragma unroll
-        for (int st = 0; st < NT; ++st)
-#pragma unroll
-          for (int hh = 0; hh < NH; ++hh) acc[m][st] = mfma(av, as_bf16x8(b[st][hh]), acc[m][st]);
-      }
-    }
-  } else {
-    // MLX affine, one 64-column group: P = Σ q·x on the bf16 MFMA (steps v = 0, 1: word v of the
-    // lane's codes), G = Σ x on the MFMA with an all-ones A operand (every row of its D holds the
-    // column sums, so each lane gets its column's), then acc += s·P + b·G per D row
-    // (gemma.metal:234-236's factorisation). 4-bit codes enter the MFMA as bf16 (128 + q), two
-    // per instruction pair: ((w >> 4k) & 0x000F000F) | 0x43004300 holds codes k and k+4, so the
-    // B values are paired the same way (x_k, x_{k+4}) and the 128·G term goes into the bias:
-    // acc += s·P' + (b − 128·s)·G.
-    u32x4 b[NT][NH][2];
-#pragma unroll
-    for (int st = 0; st < NT; ++st)
-#pragma unroll
-      for (int hh = 0; hh < NH; ++hh)
-#pragma unroll
-        for (int v = 0; v < 2; ++v) {
-          const u32x4 raw = bv(st, hh, v);
-          if constexpr (FMT == Q_MLX4) {
-            // (x0,x1)(x2,x3)(x4,x5)(x6,x7) → (x0,x4)(x1,x5)(x2,x6)(x3,x7)
-            b[st][hh][v] = u32x4{__builtin_amdgcn_perm(raw[2], raw[0], 0x05040100u),
-                                 __builtin_amdgcn_perm(raw[2], raw[0], 0x07060302u),
-                                 __builtin_amdgcn_perm(raw[3], raw[1], 0x05040100u),
-                                 __builtin_amdgcn_perm(raw[3], raw[1], 0x07060302u)};
-          } else {
-            b[st][hh][v] = raw;
-          }
-        }
-    f32x4 P[NM][NT], G[NT];
-#pragma unroll
-    for (int st = 0; st < NT; ++st) {
-      G[st] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int m = 0; m < NM; ++m) P[m][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-    const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0
-#pragma unroll
-    for (int v = 0; v < 2; ++v) {
-#pragma unroll
-      for (int st = 0; st < NT; ++st)
-#pragma unroll
-        for (int hh = 0; hh < NH; ++hh) G[st] = mfma(as_bf16x8(ones), as_bf16x8(b[st][hh][v]), G[st]);
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        bf16x8 av;
-        if constexpr (FMT == Q_MLX4) {
-          const uint32_t wv = w[m].w[v];
-          u32x4 r;
-#pragma unroll
-          for (int k = 0; k < 4; ++k) r[k] = ((wv >> (4 * k)) & 0x000F000Fu) | 0x43004300u;
-          av = as_bf16x8(r);
-        } else {
-          av = F::decode(w[m], v);
-        }
-#pragma unroll
-        for (int st = 0; st < NT; ++st)
-#pragma unroll
-          for (int hh = 0; hh < NH; ++hh) P[m][st] = mfma(av, as_bf16x8(b[st][hh][v]), P[m][st]);
-      }
-    }
-    // D row 4g + ii is the A row of lane 4g + ii: its scale and bias by shuffle (all four
-    // shuffles issued before the first is used).
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      uint32_t sbs[4];
-      if constexpr (std::is_same_v<SBF, std::nullptr_t>) {
-        const int sbl = (int)w[m].sb;
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) sbs[ii] = (uint32_t)__shfl(sbl, 4 * g + ii);
-      } else {
-        const u32x4 v = sbf(m);
-#pragma unroll
-        for (int ii = 0; ii < 4; ++ii) sbs[ii] = v[ii];
-      }
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) {
-        const uint32_t sbv = sbs[ii];
-        const float sc = bf16_bits_to_f32(sbv & 0xFFFF);
-        const float bi0 = bf16_bits_to_f32(sbv >> 16);
-        const float bi = FMT == Q_MLX4 ? __builtin_fmaf(-128.f, sc, bi0) : bi0;
-#pragma unroll
-        for (int st = 0; st < NT; ++st) {
-          acc[m][st][ii] = __builtin_fmaf(sc, P[m][st][ii], acc[m][st][ii]);
-          acc[m][st][ii] = __builtin_fmaf(bi, G[st][ii], acc[m][st][ii]);
-        }
-      }
-    }
-  }
-}
 
 // Weight stream of one wave over its chunks c = c0, c0 + cs, c0 + 2·cs, ... < nch with a DA-deep
 // register ring: the A operand of the next DA chunks is in flight while a chunk is computed; a
@@ -484,70 +155,6 @@ template <int FMT, int NM, int DA, bool NOSB = false> struct AStream {
     }
   }
 };
-
-// acc = p0 + p1 per element (the two chains of the canonical arithmetic).
-__device__ __forceinline__ f32x4 sum_chains(const f32x4 &p0, const f32x4 &p1) {
-  f32x4 r;
-#pragma unroll
-  for (int ii = 0; ii < 4; ++ii) r[ii] = p0[ii] + p1[ii];
-  return r;
-}
-
-// Activations of 4 intermediates i0..i0+3: bias (GPT-OSS gate_up bias, interleaved like the
-// rows) and the gated activation.
-template <int FMT>
-__device__ __forceinline__ f32x4 up_values(const GemmArgs &a, const uint8_t *blob, const ExpertGroup &grp,
-                                           int i0, const f32x4 &gate, const f32x4 &up) {
-  float gb[4] = {0.f, 0.f, 0.f, 0.f}, ub[4] = {0.f, 0.f, 0.f, 0.f};
-  if (FMT == Q_MXFP4 && a.expert_bias) {
-    const uint16_t *bias = (const uint16_t *)(blob + grp.off[2]);
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-      gb[ii] = bf16_bits_to_f32(bias[2 * (i0 + ii)]);
-      ub[ii] = bf16_bits_to_f32(bias[2 * (i0 + ii) + 1]);
-    }
-  }
-  float gv[4], uv[4], yv[4];
-#pragma unroll
-  for (int ii = 0; ii < 4; ++ii) {
-    gv[ii] = gate[ii] + gb[ii];
-    uv[ii] = up[ii] + ub[ii];
-  }
-  activate_n<4>(a.act, gv, uv, yv, a.alpha, a.limit);
-  return f32x4{yv[0], yv[1], yv[2], yv[3]};
-}
-
-// up_values with the GPT-OSS bias of the 4 intermediates already loaded: 16 bytes from the bias
-// row at element 2·i0, (gate, up) bf16 pairs in order.
-__device__ __forceinline__ f32x4 up_values_mx(const GemmArgs &a, const u32x4 &bias, const f32x4 &gate,
-                                              const f32x4 &up) {
-  float gv[4], uv[4], yv[4];
-#pragma unroll
-  for (int ii = 0; ii < 4; ++ii) {
-    gv[ii] = gate[ii] + bf16_bits_to_f32(bias[ii] & 0xFFFFu);
-    uv[ii] = up[ii] + bf16_bits_to_f32(bias[ii] >> 16);
-  }
-  activate_n<4>(a.act, gv, uv, yv, a.alpha, a.limit);
-  return f32x4{yv[0], yv[1], yv[2], yv[3]};
-}
-
-// Gate-up epilogue of 4 intermediates i0..i0+3 of slot `slot`: bias, activation, bf16 hi/lo.
-template <int FMT>
-__device__ __forceinline__ void up_epilogue(const GemmArgs &a, const uint8_t *blob,
-                                            const ExpertGroup &grp, int i0, int slot,
-                                            const f32x4 &gate, const f32x4 &up) {
-  const f32x4 yv = up_values<FMT>(a, blob, grp, i0, gate, up);
-  uint32_t hi[4], lo[4];
-#pragma unroll
-  for (int ii = 0; ii < 4; ++ii) {
-    const float y = yv[ii];
-    hi[ii] = f32_to_bf16_bits(y);
-    lo[ii] = f32_to_bf16_bits(y - bf16_bits_to_f32(hi[ii]));
-  }
-  const size_t o = (size_t)slot * a.ldh + i0;
-  *(u32x2 *)(a.h_hi + o) = u32x2{hi[0] | (hi[1] << 16), hi[2] | (hi[3] << 16)};
-  *(u32x2 *)(a.h_lo + o) = u32x2{lo[0] | (lo[1] << 16), lo[2] | (lo[3] << 16)};
-}
 
 // Slot values of hidden rows h0..h0+3: routing weight × (product + bias)
 // (write_expert_scaled, dense.metal:131-145).
@@ -941,22 +548,6 @@ __global__ __launch_bounds__(256 * TPW) void up_small(GemmArgs a, RouteArgs ra, 
     }
     if (it == (int)blockIdx.x) HH_TR(1, 4);
   }
-}
-
-// ---- MXFP4 on the scaled MFMA -------------------------------------------------------------------
-typedef int v8i __attribute__((ext_vector_type(8)));
-
-// D += A·B, v_mfma_scale_f32_16x16x128_f8f6f4 with A = 16 rows × 128 K of fp4 e2m1 and B =
-// 128 K × 16 columns of fp8 e4m3. A lane (g, l16): row l16, the 32 values of K block g (low nibble
-// first: exactly one MXFP4 block as stored) and that block's e8m0 scale. B lane (g, l16): column
-// l16, K 16g..16g+15 in bytes 0-15 and K 64+16g..64+16g+15 in bytes 16-31, and the e8m0 scale of
-// K block g. D as the 16x16 bf16 MFMA.
-__device__ __forceinline__ f32x4 smfma(const u32x4 &a, const u32x4 &blo, const u32x4 &bhi, uint32_t sa,
-                                       uint32_t sb, const f32x4 &c) {
-  const v8i av = {(int)a[0], (int)a[1], (int)a[2], (int)a[3], 0, 0, 0, 0};
-  const v8i bv = {(int)blo[0], (int)blo[1], (int)blo[2], (int)blo[3],
-                  (int)bhi[0], (int)bhi[1], (int)bhi[2], (int)bhi[3]};
-  return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 0, 0, (int)sa, 0, (int)sb);
 }
 
 // B operand of chunk c from one term row (bytes, K columns) and its block scales `srow`; columns
@@ -2312,50 +1903,6 @@ template <int PH, int RR, int TT> struct Mx3 {
   static_assert(B_INS % 4 == 0 && BS_DW <= 256 && NTOK <= 64 && S >= 3 && (S - 2) * L <= 63, "loader layout");
 };
 
-// Workgroup barrier without __syncthreads' release fence: the fence would make every wave wait for
-// all of its direct-to-LDS loads (vmcnt(0)) before the barrier; the pipeline orders LDS itself
-// with explicit waits. A compiler memory barrier keeps LDS accesses on their side.
-__device__ __forceinline__ void ring_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
-typedef __attribute__((address_space(3))) void *lds_ptr_t;
-__device__ __forceinline__ void lds_load16(const void *g, uint8_t *l) {
-  __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)l, 16, 0, 0);
-}
-__device__ __forceinline__ void lds_load4(const void *g, uint8_t *l) {
-  __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)l, 4, 0, 0);
-}
-
-// Task ids of one workgroup of a persistent prefill kernel: τ = b, b + G, ... (G a multiple of
-// 8, so τ mod 8 is the workgroup's XCD), skipping tasks past the row tiles or the work items.
-// The 8 XCDs form P row-tile parts × 8/P work-item parts: XCD x takes row tiles of part x mod P
-// and work items of part x / P, work item by work item (each item's row tiles consecutively).
-// An expert's slice of weight rows stays in the XCD's L2 across the expert's consecutive items,
-// and an item's operand rows are fetched by the P XCDs of its item part.
-struct Mx3Tasks {
-  int b, G, RT, nwork, P, rtp, nq, lim;
-  __device__ __forceinline__ Mx3Tasks(int b_, int G_, int RT_, int nwork_, int P_)
-      : b(b_), G(G_), RT(RT_), nwork(nwork_), P(P_ == 1 || P_ == 2 || P_ == 4 ? P_ : 8) {
-    rtp = (RT + P - 1) / P;
-    nq = (nwork + 8 / P - 1) / (8 / P);
-    lim = 8 * rtp * nq;
-  }
-  __device__ __forceinline__ void tile(int tau, int &rt, int &wi) const {
-    const int x = tau & 7, j = tau >> 3, q = j / rtp;
-    rt = (x & (P - 1)) * rtp + (j - q * rtp);
-    wi = (x / P) * nq + q;
-  }
-  __device__ __forceinline__ int first() const { return fix(b); }
-  __device__ __forceinline__ int next(int tau) const { return fix(tau + G); }
-  __device__ __forceinline__ int fix(int tau) const {
-    for (; tau < lim; tau += G) {
-      int rt, wi;
-      tile(tau, rt, wi);
-      if (rt < RT && wi < nwork) return tau;
-    }
-    return lim;
-  }
-};
-
 template <int PH, int RR, int TT>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_mx3(GemmArgs a) {
   using C = Mx3<PH, RR, TT>;
@@ -3076,11 +2623,6 @@ template <int PH, int FMT, int RT, int NT_> struct Ring {
   }
 };
 
-__device__ __forceinline__ void lds_load2(const void *g, uint8_t *l) {
-  __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)l, 2, 0, 0);
-}
-template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-
 template <int PH, int FMT, int RT, int NT_>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_ring(GemmArgs a) {
   using C = Ring<PH, FMT, RT, NT_>;
@@ -3612,7 +3154,10 @@ template <int PH, int TT> static hipError_t launch_mxa(GemmArgs a, hipStream_t s
   return hipGetLastError();
 }
 
+hipError_t launch_prefill(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm);   // hh_prefill.hip
+
 hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &args, hipStream_t s, Timing tm) {
+  if (quant == Q_BF16) return launch_prefill(phase, quant, nt, args, s, tm);
   // Persistent kernels: XCD split into row-tile parts × work-item parts (Mx3Tasks). Measured on
   // the benchmark layers (prefill T = 512..2048) against 8 row-tile parts: BF16 gate-up 832 →
   // 615 µs with 4 or 2 parts, BF16 down 414 → 371 µs with 2; MLX 3-5 % faster with 4; MXFP4

@@ -1,0 +1,234 @@
+// hh_prefill.hip — grouped expert products of the prefill path (T > 16) on gfx950 MFMA: one
+// four-wave workgroup per task (a row tile × a work item), two workgroups per compute unit.
+#include "hh_mfma.hpp"
+
+#include <algorithm>
+#include <mutex>
+
+namespace hh {
+
+// 16 bytes per lane from global memory straight into LDS: base (uniform) + off (per lane) to LDS
+// byte `l` + 16·lane. Written in assembly so that the compiler does not order the wave's own LDS
+// reads after its loads in flight (it would wait for all of them); the kernels wait with wait_vm.
+// The instruction has no register result.
+__device__ __forceinline__ void dma16(const void *base, uint32_t off, uint32_t l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l), "v"(off), "s"(base)
+               : "memory");
+}
+__device__ __forceinline__ void dma16(const void *p, uint32_t l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(p) : "memory");
+}
+// Barrier after the wave's own LDS reads have returned: the next stage may overwrite what they read.
+__device__ __forceinline__ void step_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+__device__ __forceinline__ uint32_t lds_addr(const uint8_t *l) { return (uint32_t)(uintptr_t)(lds_ptr_t)(void *)l; }
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+
+// One task per workgroup; two four-wave workgroups (BF16 160-token items: one of eight waves) per
+// compute unit, so that one's loads, barriers and epilogue pass under the other's MFMAs. Every wave
+// both loads and multiplies: a stage of K columns of the row tile's weights and of the item's
+// token rows goes straight to an S-deep LDS ring, S − 1 stages ahead. Before (one persistent
+// workgroup per compute unit, four loader waves and four MFMA waves) each SIMD had a single MFMA
+// wave, which sat through its own LDS reads and barrier at every stage (with no global traffic at
+// all the BF16 T = 2048 gate-up still took 350 of its 415 us).
+// Weight loads take whole 128-byte pieces of a row with consecutive lanes: 50 B/clk
+// per compute unit from L2, against 15.5 for the MFMA lane order (16 rows × 64 bytes, consecutive
+// lanes on different rows), which the L1 serves a row at a time when the row stride is a multiple
+// of 128 bytes. The XOR of the 16-byte segments by the row keeps the MFMA lanes' LDS reads at full rate.
+// The output tiles' arithmetic is the canonical one (chunk_mfma, prefill equals decode bit for bit).
+//
+// XCD order (Mx3Tasks): two row-tile parts × four item parts, so an item's token rows reach two
+// XCDs' L2: BF16 T = 2048 gate-up 430 us with four parts, 349 with two, 359 with one.
+
+// ---- BF16 -----------------------------------------------------------------------------------------
+// NT token tiles × NM weight tiles of 16 per wave; WT token groups of four waves; SV MFMA steps of
+// 32 columns per stage.
+// Tiles, timed on the 128-expert layer (H 2816, I 704; gate-up / down us at T tokens):
+//   T = 2048 (128 tokens an expert): 64-token items of 128 intermediates 300 / 222, 128-token items
+//     285 / 217, 160-token items 278 / 194 (an expert's weights are read 2.5, 1.5, 1.0 times);
+//     with 32-column stages (64-byte pieces) 349 for the 64-token gate-up;
+//   T = 700 (44 an expert): 160-token 206 / 144, 32-token 243 / 141;
+//   T = 400 (25 an expert): 160-token 195 / 133, 32-token 196 / 112, hence the line at 40;
+//   T = 100 (6 an expert; the weights' 1.03 GB stream at 5.8 TB/s): 32-token gate-up of 64
+//     intermediates 179, of 128 201.
+// The previous kernels: 415 / 284 at T = 2048, 302 / 177 at 700, 189 / 105 at 100.
+template <int PH, int NT_, int RT_, int SV_, int WT_> struct Bf {
+  static constexpr int NT = NT_, NH = PH == PH_UP ? 1 : 2, SV = SV_, WT = WT_;
+  static constexpr int RT = RT_, NM = (PH == PH_UP ? 2 : 1) * RT;   // gate-up: RT gate and RT up tiles
+  static constexpr int NW = 4 * WT;                          // waves
+  static constexpr int ROWS = 64 * RT;                       // output rows per workgroup
+  static constexpr int TB = 1024 * SV;                       // bytes of a 16-row tile
+  static constexpr int A_INS = 4 * NM * SV, B_INS = NH * NT * WT * SV;   // 1 KiB loads per stage
+  static constexpr int APW = A_INS / NW, BPW = (B_INS + NW - 1) / NW;
+  static constexpr int L = APW + BPW;
+  static constexpr int OFF_B = A_INS * 1024;
+  static constexpr int STAGE = OFF_B + B_INS * 1024;
+  static constexpr int S_FIT = (80 * WT * 1024) / STAGE, S = S_FIT > 4 ? 4 : S_FIT;
+  static constexpr int LDS = S * STAGE;
+  static_assert(S >= 2, "ring depth");
+};
+
+template <int PH, int NT_, int RT_, int SV_, int WT_>
+__global__ __launch_bounds__(256 * WT_) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_bf16(GemmArgs a) {
+  using C = Bf<PH, NT_, RT_, SV_, WT_>;
+  constexpr int NM = C::NM, NT = C::NT, NH = C::NH, RT = C::RT, S = C::S, L = C::L, SV = C::SV, WT = C::WT, TB = C::TB;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
+  const int wave = uniform(threadIdx.x >> 6), wr = wave & 3, wt = wave >> 2;
+  const int H = a.hidden, E = a.experts;
+  const int nwork = *a.n_work;
+  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, a.row_tiles, nwork, a.xcd_rows);
+  if ((int)blockIdx.x >= tasks.lim) return;
+  int rt, wi;
+  tasks.tile((int)blockIdx.x, rt, wi);
+  if (rt >= a.row_tiles || wi >= nwork) return;
+  const int4 it = a.work[wi];
+  const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
+  const ExpertGroup &grp = a.grp[e == E ? 1 : 0];
+  const uint8_t *blob = grp.blobs + (e == E ? 0 : (size_t)e * grp.stride);
+  const int I = grp.inter;
+  const int K = PH == PH_UP ? H : I, out_dim = PH == PH_UP ? I : H;
+  const int n = K / (32 * SV);   // stages
+  if (rt * C::ROWS >= out_dim) return;
+  const int rb = rt * C::ROWS + wr * 16 * RT, tb = wt * 16 * NT;
+  const bool active = rb < out_dim && tb < cnt;
+
+  constexpr int RPI = 16 / SV, SEGS = 4 * SV;   // rows per load, 16-byte segments per row
+  const size_t rowb = (size_t)K * 2;
+  const int lr = lane / SEGS;   // row of the load
+  auto swz = [](int r) { return SV == 1 ? (r >> 1) & 3 : r & 7; };
+  const int seg = (lane % SEGS) ^ swz(lr);
+  const uint32_t aoff = (uint32_t)(lr * rowb + 16 * seg);
+  const uint8_t *abase[C::APW];
+#pragma unroll
+  for (int i = 0; i < C::APW; ++i) {
+    const int j = wave * C::APW + i;   // load j of the stage: tile j / SV, rows RPI·(j % SV) ..
+    const int tl = j / SV, w = tl / NM, m = tl % NM;
+    const int r0 = min(rt * C::ROWS + w * 16 * RT + 16 * (m % RT), out_dim - 16) + (PH == PH_UP && m >= RT ? I : 0);
+    abase[i] = blob + grp.off[PH == PH_UP ? 0 : 1] + (r0 + RPI * (j % SV)) * rowb;
+  }
+  const uint8_t *bsrc[C::BPW];
+  uint32_t bdst[C::BPW];
+#pragma unroll
+  for (int i = 0; i < C::BPW; ++i) {
+    const int j = (wave * C::BPW + i) % C::B_INS, hh = j / (NT * WT * SV), tl = j % (NT * WT * SV);
+    const int sl = a.order[pos + min(RPI * tl + lr, cnt - 1)];
+    const uint16_t *row = PH == PH_UP ? a.x + (size_t)(sl / a.slots) * H : (hh ? a.h_lo : a.h_hi) + (size_t)sl * a.ldh;
+    bsrc[i] = (const uint8_t *)row + 16 * seg;
+    bdst[i] = lds_addr(lds) + C::OFF_B + 1024 * j;
+  }
+  int es[NT];
+#pragma unroll
+  for (int st = 0; st < NT; ++st) es[st] = a.order[pos + min(tb + 16 * st + l16, cnt - 1)];
+
+  const uint32_t adst = lds_addr(lds) + wave * C::APW * 1024;
+  int q = 0, qs = 0;   // stages issued, the ring slot of the next
+  auto issue = [&]() {
+    const uint32_t so = (uint32_t)(qs * C::STAGE);
+#pragma unroll
+    for (int i = 0; i < C::APW; ++i) dma16(abase[i] + 64 * SV * q, aoff, adst + so + 1024 * i);
+#pragma unroll
+    for (int i = 0; i < C::BPW; ++i) dma16(bsrc[i] + 64 * SV * q, bdst[i] + so);
+    ++q;
+    qs = qs == S - 1 ? 0 : qs + 1;
+  };
+  for (int u = 0; u < S - 1 && q < n; ++u) issue();
+
+  f32x4 acc[2][NM][NT];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int st = 0; st < NT; ++st) acc[p][m][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int roff = l16 * 64 * SV + 16 * (g ^ swz(l16));   // step v: ^ 64·v
+  int s = 0, ss = 0;   // stage computed, its ring slot
+  auto step = [&](f32x4 (&ac)[NM][NT]) {
+    // Stage s has landed once at most the later issued stages' loads are outstanding.
+    const int later = q - 1 - s;
+    if (later >= S - 2) wait_vm<(S - 2) * L>();
+    else if (S > 3 && later == 1) wait_vm<L>();
+    else wait_vm<0>();
+    step_barrier();
+    if (q < n) issue();
+    const uint8_t *stg = lds + ss * C::STAGE;
+    if (active) {
+#pragma unroll
+      for (int v = 0; v < SV; ++v) {
+        const int ro = roff ^ (64 * v);
+        u32x4 w[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) w[m] = *(const u32x4 *)(stg + (wr * NM + m) * TB + ro);
+#pragma unroll
+        for (int st = 0; st < NT; ++st) {
+          if (st > 0 && tb + 16 * st >= cnt) break;   // token tiles wholly past the item
+#pragma unroll
+          for (int hh = 0; hh < NH; ++hh) {
+            const u32x4 b = *(const u32x4 *)(stg + C::OFF_B + (hh * NT * WT + wt * NT + st) * TB + ro);
+#pragma unroll
+            for (int m = 0; m < NM; ++m) ac[m][st] = mfma(as_bf16x8(w[m]), as_bf16x8(b), ac[m][st]);
+          }
+        }
+      }
+    }
+    ++s;
+    ss = ss == S - 1 ? 0 : ss + 1;
+  };
+  // Chunks of 128 columns: the even ones into chain 0, the odd ones into chain 1.
+  constexpr int SPC = 4 / SV;
+  for (int c0 = 0; c0 < n; c0 += 2 * SPC) {
+    const int n0 = min(n, c0 + SPC), n1 = min(n, c0 + 2 * SPC);
+#pragma unroll 1
+    while (s < n0) step(acc[0]);
+#pragma unroll 1
+    while (s < n1) step(acc[1]);
+  }
+  if (!active) return;
+#pragma unroll
+  for (int st = 0; st < NT; ++st) {
+    if (tb + 16 * st + l16 >= cnt) continue;
+    const float ew = PH == PH_DOWN ? a.slot_w[es[st]] : 0.f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int r0 = rb + 16 * r;
+      if (r0 >= out_dim) continue;
+      if constexpr (PH == PH_UP) {
+        up_epilogue<Q_BF16>(a, nullptr, grp, r0 + 4 * g, es[st], sum_chains(acc[0][r][st], acc[1][r][st]),
+                            sum_chains(acc[0][RT + r][st], acc[1][RT + r][st]));
+      } else {
+        const f32x4 v = sum_chains(acc[0][r][st], acc[1][r][st]);
+        f32x4 o;
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) o[ii] = ew * (v[ii] + 0.f);   // down_value's arithmetic
+        *(f32x4 *)(a.slot_out + (size_t)es[st] * H + r0 + 4 * g) = o;
+      }
+    }
+  }
+}
+
+template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(GemmArgs a, hipStream_t s, Timing tm) {
+  using C = Bf<PH, NT, RT, SV, WT>;
+  static std::once_flag once;
+  std::call_once(once, [] {
+    (void)hipFuncSetAttribute((const void *)prefill_bf16<PH, NT, RT, SV, WT>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+    (void)hipGetLastError();
+  });
+  const int rows = PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
+  a.row_tiles = (rows + C::ROWS - 1) / C::ROWS;
+  a.xcd_rows = 2;
+  const int P = a.xcd_rows;
+  const unsigned blocks = 8u * (unsigned)((a.row_tiles + P - 1) / P) * (unsigned)((a.max_work + 8 / P - 1) / (8 / P));
+  if (blocks == 0) return hipSuccess;
+  hipExtLaunchKernelGGL((prefill_bf16<PH, NT, RT, SV, WT>), dim3(blocks), dim3(256 * WT), C::LDS, s, tm.start, tm.stop, 0, a);
+  return hipGetLastError();
+}
+
+// The tile of each call. BF16 work items hold 160 tokens (nt 10: experts averaging 40 tokens or
+// more) or 32.
+hipError_t launch_prefill(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
+  const bool up = phase == PH_UP;
+  if (quant != Q_BF16) return hipErrorInvalidValue;
+  if (nt == 10) return up ? launch_bf16<PH_UP, 5, 2, 2, 2>(a, s, tm) : launch_bf16<PH_DOWN, 5, 4, 2, 2>(a, s, tm);
+  return up ? launch_bf16<PH_UP, 2, 1, 2, 1>(a, s, tm) : launch_bf16<PH_DOWN, 2, 2, 2, 1>(a, s, tm);
+}
+
+}  // namespace hh

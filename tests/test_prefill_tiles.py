@@ -1,0 +1,41 @@
+"""The prefill products (T > 16) at the edges of their tiles: row tiles past the last row, a last
+stage of one step, token tiles past an item's tokens, experts of more than one work
+item, both item sizes. Against the fp64 oracle, and bit for bit against one-token calls.
+
+Bound: activations travel as a bf16 hi + lo pair (2^-17 of the value each), fp32 sums over at most a
+few hundred columns add less, so rel-L2 stays below 2e-5."""
+import numpy as np
+import pytest
+
+from hydra_amd import formats as F
+from hydra_amd import synth
+
+REL = 2e-5
+
+BF16 = F.GEMMA_BF16.replace(experts=3, top_k=2)
+CASES = {
+    # name: (desc, tokens); 2T/3 tokens an expert
+    "bf16_32_small": (BF16.replace(hidden=64, intermediate=64), 17),      # one stage
+    "bf16_32_ragged": (BF16.replace(hidden=192, intermediate=320), 59),   # 39 an expert: two items of 32
+    "bf16_160_edge": (BF16.replace(hidden=192, intermediate=320), 60),    # 40 an expert: items of 160
+    "bf16_160_two": (BF16.replace(hidden=832, intermediate=192), 300),    # 200 an expert: 160 + 40
+}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(CASES))
+def test_prefill_tiles(name):
+    from hydra_amd.layer import MoELayer
+    from oracle import oracle as O
+    desc, T = CASES[name]
+    print(f"[gpu] prefill tiles {name} T={T}", flush=True)
+    layer = synth.make_layer(desc, seed=11)
+    x = synth.make_tokens(desc.hidden, T, seed=12)
+    L = MoELayer(layer, device=0)
+    y, idx, _ = (t.cpu().numpy() for t in L.forward(x))
+    ry, ridx, _, _ = O.moe_forward(layer, x, nthreads=8)
+    assert np.array_equal(idx, ridx)
+    assert np.linalg.norm(y - ry) / np.linalg.norm(ry) < REL
+    for t in (0, T // 2, T - 1):
+        y1 = L.forward(x[t:t + 1])[0].cpu().numpy()[0]
+        assert np.array_equal(y1.view(np.uint32), y[t].view(np.uint32))
