@@ -2574,406 +2574,6 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-// ---- prefill, BF16 and MLX affine: an LDS ring filled by loader waves -----------------------------
-// 8 waves, one workgroup per compute unit, persistent over the tasks τ = blockIdx, + gridDim, ...
-// (a task = one work item of ≤ 32 tokens × one row tile, in prefill_tile's XCD-aware order).
-// Waves 4-7 load: each stage (SCOLS columns of K) brings, by direct-to-LDS loads, the weight
-// operand of the row tile (per MFMA wave: NM tiles of 16 rows, laid out exactly as that wave's
-// lanes read them), the MLX group scales and biases, and the TOK token rows of the activation
-// (x, or h_hi and h_lo) in 16-byte segments XOR-swizzled by token so the MFMA reads are
-// bank-conflict free. S stages are in flight; the ring runs on across task boundaries (each
-// task's work item and slot ids also travel by direct-to-LDS loads, ahead of its first stage).
-// Waves 0-3 multiply: wave w owns output rows rb .. rb + 16·RT of the tile (gate and up tiles of
-// the same intermediates for gate-up) for all 32 tokens, and reads each stage's operands one
-// stage ahead of its MFMAs. The arithmetic per output element is chunk_mfma's, the decode
-// kernels' bits: two chains over the chunks (even / odd), steps in order.
-template <int PH, int FMT, int RT, int NT_> struct Ring {
-  static constexpr int NT = NT_, TOK = 16 * NT;
-  static constexpr int NM = (PH == PH_UP ? 2 : 1) * RT;
-  static constexpr int NH = PH == PH_UP ? 1 : 2;
-  static constexpr bool MLX = is_mlx<FMT>();
-  // K columns per stage: two MLX groups; BF16 two 32-column steps (128-column stages leave
-  // 64-token tiles too few stages in LDS).
-  static constexpr int SCOLS = MLX ? 128 : 64;
-  static constexpr int SPS = MLX ? 2 : SCOLS / 32;              // MLX groups / BF16 steps per stage
-  static constexpr int SEGS = SCOLS / 8;                        // 16-byte segments per token row
-  static constexpr int RPI = 1024 / (SCOLS * 2);                // token rows per 1 KiB load
-  static constexpr int A_INS = FMT == Q_MLX4 ? 1 : SPS;         // 1 KiB weight loads per tile
-  static constexpr int B_INS = NH * TOK / RPI;                  // 1 KiB operand loads per stage
-  static constexpr int BPW = B_INS / 4;
-  static constexpr int SB_INS = MLX ? 4 : 0;                    // {scale, bias} × 2 groups
-  static constexpr int L = NM * A_INS + BPW + SB_INS;           // loads per loader wave per stage
-  static constexpr int OFF_B = 4 * NM * A_INS * 1024;
-  static constexpr int OFF_SB = OFF_B + B_INS * 1024;
-  static constexpr int STAGE = OFF_SB + (MLX ? 4096 : 0);
-  static constexpr int NO = (TOK + 63) / 64;                    // slot-id registers per lane
-  static constexpr int INFO = 256 + 256 * NO;                   // work item, slot ids
-  static constexpr int S_LDS = (148 * 1024) / STAGE, S_CNT = 3 + 63 / L;
-  static constexpr int S = S_LDS < S_CNT ? (S_LDS < 8 ? S_LDS : 8) : (S_CNT < 8 ? S_CNT : 8);
-  static constexpr int NSLOT = S + 1;                           // task info slots (≤ S tasks ahead)
-  static constexpr int OFF_INFO = S * STAGE;
-  static constexpr int LDS = OFF_INFO + NSLOT * INFO;
-  static constexpr int ROWS = 64 * RT;
-  // The B operand of the next stage is read ahead too, except for wide token tiles (measured
-  // slower there: gate-up 567 → 617 µs).
-  static constexpr bool RA_B = NT <= 2;
-  static_assert(B_INS % 4 == 0 && S >= 3 && NM <= 4 && LDS <= 160 * 1024, "ring layout");
-  __device__ static int swz(int n) {
-    return SEGS == 16 ? (n & 15) : (SEGS == 8 ? ((n >> 1) & 7) : ((n >> 2) & 3));
-  }
-};
-
-template <int PH, int FMT, int RT, int NT_>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_ring(GemmArgs a) {
-  using C = Ring<PH, FMT, RT, NT_>;
-  using F = Fmt<FMT>;
-  constexpr int NM = C::NM, NT = C::NT, NH = C::NH, TOK = C::TOK, S = C::S, L = C::L;
-  constexpr int SCOLS = C::SCOLS, SEGS = C::SEGS, SPS = C::SPS, NO = C::NO;
-  extern __shared__ __align__(16) uint8_t lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, l16 = lane & 15;
-  const int H = a.hidden, E = a.experts;
-  const int RTL = a.row_tiles, rtx = (RTL + 7) >> 3;
-  const int nwork = *a.n_work;
-  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, RTL, nwork, a.xcd_rows);
-  if (tasks.first() >= tasks.lim) return;
-  auto group_of = [&](int e) -> const ExpertGroup & { return a.grp[e == E ? 1 : 0]; };
-  auto k_of = [&](int e) { return PH == PH_UP ? H : group_of(e).inter; };
-  auto nst_of = [&](int e) { return (k_of(e) + SCOLS - 1) / SCOLS; };
-  auto work_of = [&](int tau) {
-    int rt, wi;
-    tasks.tile(min(tau, tasks.lim - 1), rt, wi);
-    return a.work[min(wi, nwork - 1)];
-  };
-  // A task's copy for the MFMA waves: its work item, then its slot ids.
-  auto send_info = [&](int tau, const int4 &w, int slot) {
-    int rt, wi;
-    tasks.tile(tau, rt, wi);
-    uint8_t *info = lds + C::OFF_INFO + C::INFO * slot;
-    lds_load4((const int *)(a.work + wi) + min(lane, 3), info);
-#pragma unroll
-    for (int k = 0; k < NO; ++k) lds_load4(a.order + w.y + min(64 * k + lane, w.z - 1), info + 256 * (k + 1));
-  };
-
-  if (wave >= 4) {
-    // ---- loaders ----
-    const int lw = wave - 4;
-    int tau = tasks.first(), slot = 0;
-    int4 wn = work_of(tau), wnn = work_of(tasks.next(tau));
-    int on[NO];
-#pragma unroll
-    for (int k = 0; k < NO; ++k) on[k] = a.order[wn.y + min(64 * k + lane, wn.z - 1)];
-    int K = 0, nst = 0, ls = 0, q = 0;     // task K, its stages, stage within it, stages issued
-    ATile<FMT> at[NM];
-    const uint16_t *brow[C::BPW];
-    bool more = true;
-    send_info(tau, wn, 0);   // the first task's copy, waited for here
-    wait_vm<0>();
-    auto begin_task = [&]() {
-      const int4 cur = wn;
-      int o[NO];
-#pragma unroll
-      for (int k = 0; k < NO; ++k) o[k] = on[k];
-      int rt, wi;
-      tasks.tile(tau, rt, wi);
-      // The next task's copy goes out a task ahead: it lands long before that task's first stage
-      // is read.
-      const int t1 = tasks.next(tau);
-      if (t1 < tasks.lim) send_info(t1, wnn, slot == C::NSLOT - 1 ? 0 : slot + 1);
-      const int e = cur.x;
-      const ExpertGroup &grp = group_of(e);
-      const uint8_t *blob = grp.blobs + (e == E ? 0 : (size_t)e * grp.stride);
-      K = k_of(e);
-      nst = nst_of(e);
-      const int out_dim = PH == PH_UP ? grp.inter : H;
-      wave_tiles<PH, FMT, RT>(at, blob, grp, rt * C::ROWS + lw * 16 * RT, out_dim, K, l16);
-#pragma unroll
-      for (int i = 0; i < C::BPW; ++i) {
-        const int j = lw * C::BPW + i;
-        const int hh = j / (TOK / C::RPI);
-        const int n = min(C::RPI * (j % (TOK / C::RPI)) + lane / SEGS, cur.z - 1);
-        int sl = 0;
-#pragma unroll
-        for (int k = 0; k < NO; ++k) {
-          const int v = __shfl(o[k], n & 63);
-          if ((n >> 6) == k) sl = v;
-        }
-        brow[i] = PH == PH_UP ? a.x + (size_t)(sl / a.slots) * H : (hh ? a.h_lo : a.h_hi) + (size_t)sl * a.ldh;
-      }
-      // Prefetch: the next task's slot ids, the work item of the one after.
-      wn = wnn;
-#pragma unroll
-      for (int k = 0; k < NO; ++k) on[k] = a.order[wn.y + min(64 * k + lane, wn.z - 1)];
-      wnn = work_of(tasks.next(t1));
-    };
-    auto issue = [&](int s, int st) {
-      uint8_t *stg = lds + st * C::STAGE;
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        uint8_t *dst = stg + (lw * NM + m) * C::A_INS * 1024;
-        const uint8_t *w = at[m].row.w;
-        if constexpr (FMT == Q_BF16) {
-#pragma unroll
-          for (int j = 0; j < SPS; ++j) lds_load16(w + 2 * min(SCOLS * s + 32 * j + 8 * g, K - 8), dst + 1024 * j);
-        } else if constexpr (FMT == Q_MLX4) {
-          lds_load16(w + min(64 * s + 16 * g, K / 2 - 16), dst);
-        } else {
-#pragma unroll
-          for (int p = 0; p < 2; ++p) lds_load16(w + min(128 * s + 64 * p + 16 * g, K - 16), dst + 1024 * p);
-        }
-      }
-      if constexpr (C::MLX) {
-        // Group scales and biases of the wave's rows: lane (m, r) holds tile m's row r (one
-        // dword per lane; tiles past NM repeat the last).
-        typename F::Row r = at[0].row;
-#pragma unroll
-        for (int m = 1; m < NM; ++m)
-          if ((lane >> 4) >= m) r = at[m].row;
-        const int ng = K / 64;
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const int gi = min(2 * s + p, ng - 1);
-          lds_load2(r.sc + gi, stg + C::OFF_SB + lw * 1024 + p * 256);
-          lds_load2(r.bi + gi, stg + C::OFF_SB + lw * 1024 + 512 + p * 256);
-        }
-      }
-#pragma unroll
-      for (int i = 0; i < C::BPW; ++i) {
-        const int j = lw * C::BPW + i;
-        const int n = C::RPI * (j % (TOK / C::RPI)) + lane / SEGS;
-        const int seg = (lane % SEGS) ^ C::swz(n);
-        lds_load16(brow[i] + min(SCOLS * s + 8 * seg, K - 8), stg + C::OFF_B + 1024 * j);
-      }
-    };
-    auto issue_next = [&]() {
-      if (ls == 0) begin_task();
-      issue(ls, q % S);
-      asm volatile("" ::: "memory");   // stages (and task copies) issue in program order
-      ++q;
-      if (++ls == nst) {
-        ls = 0;
-        tau = tasks.next(tau);
-        slot = slot == C::NSLOT - 1 ? 0 : slot + 1;
-        more = tau < tasks.lim;
-      }
-    };
-    for (int u = 0; u < S - 1 && more; ++u) issue_next();
-    if (q >= S - 1) wait_vm<(S - 3) * L>();
-    else wait_vm<0>();
-    for (int step = 0; more || step < q; ++step) {
-      ring_barrier();
-      if (more) {
-        issue_next();
-        wait_vm<(S - 3) * L>();
-      } else {
-        wait_vm<0>();
-      }
-    }
-    return;
-  }
-
-  // ---- MFMA waves ----
-  constexpr int NP = C::MLX ? 2 : 1;
-  struct AOps { typename F::A w[NP][NM]; };
-  struct BOps { u32x4 b[NP][NT][NH][C::MLX ? 2 : SPS]; };
-  auto read_a = [&](int st) {
-    const uint8_t *stg = lds + st * C::STAGE;
-    AOps o;
-#pragma unroll
-    for (int m = 0; m < NM; ++m) {
-      const uint8_t *ab = stg + (wave * NM + m) * C::A_INS * 1024;
-      if constexpr (FMT == Q_BF16) {
-#pragma unroll
-        for (int j = 0; j < SPS; ++j) o.w[0][m].w[j] = *(const u32x4 *)(ab + 1024 * j + 16 * lane);
-      } else {
-#pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          if constexpr (FMT == Q_MLX4) {
-            const u32x2 v = *(const u32x2 *)(ab + 16 * ((2 * p + (g >> 1)) * 16 + l16) + 8 * (g & 1));
-            o.w[p][m].w[0] = v[0];
-            o.w[p][m].w[1] = v[1];
-          } else {
-            const u32x4 v = *(const u32x4 *)(ab + 1024 * p + 16 * lane);
-#pragma unroll
-            for (int k = 0; k < 4; ++k) o.w[p][m].w[k] = v[k];
-          }
-          const uint8_t *sbp = stg + C::OFF_SB + wave * 1024 + p * 256 + 4 * (16 * m + l16);
-          o.w[p][m].sb = (*(const uint32_t *)sbp & 0xFFFFu) | (*(const uint32_t *)(sbp + 512) << 16);
-        }
-      }
-    }
-    return o;
-  };
-  auto read_b = [&](int st) {
-    const uint8_t *stg = lds + st * C::STAGE;
-    BOps o;
-#pragma unroll
-    for (int p = 0; p < NP; ++p)
-#pragma unroll
-      for (int st2 = 0; st2 < NT; ++st2)
-#pragma unroll
-        for (int hh = 0; hh < NH; ++hh)
-#pragma unroll
-          for (int v = 0; v < (C::MLX ? 2 : SPS); ++v) {
-            const int n = 16 * st2 + l16;
-            const int seg = C::MLX ? 8 * p + 2 * g + v : 4 * v + g;
-            o.b[p][st2][hh][v] =
-                *(const u32x4 *)(stg + C::OFF_B + (hh * TOK + n) * (SCOLS * 2) + 16 * (seg ^ C::swz(n)));
-          }
-    return o;
-  };
-
-  // The two chains of the canonical arithmetic. MLX: acc[c & 1] with c static per half-stage.
-  // BF16 (a stage is part of one chunk): acc[0] holds the chain of chunk parity cpar and acc[1] the
-  // other; they trade places when the parity changes (at most once per chunk), so the MFMAs
-  // address fixed registers, and the epilogue's acc[0] + acc[1] is the same sum either way (fp
-  // addition commutes).
-  f32x4 acc[2][NM][NT];
-  int cpar = 0;
-  auto zero = [&]() {
-#pragma unroll
-    for (int p = 0; p < 2; ++p)
-#pragma unroll
-      for (int m = 0; m < NM; ++m)
-#pragma unroll
-        for (int st = 0; st < NT; ++st) acc[p][m][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-    cpar = 0;
-  };
-  zero();
-  int tau = tasks.first(), slot = 0, ls = 0, nst = 0, K = 0, e = 0, ntok = 0, rt = 0;
-  float ew[PH == PH_DOWN ? NT : 1];
-  const ATile<FMT> at_unused[NM] = {};
-  ring_barrier();
-  AOps cur = read_a(0);
-  BOps curb;
-  if constexpr (C::RA_B) curb = read_b(0);
-  for (int step = 0;; ++step) {
-    if (PH == PH_UP) HH_TRS(step, 0);
-    if (ls == 0) {
-      const uint8_t *info = lds + C::OFF_INFO + C::INFO * slot;
-      const int4 it = *(const int4 *)info;
-      e = it.x;
-      ntok = it.z;
-      K = k_of(e);
-      nst = nst_of(e);
-      int wi;
-      tasks.tile(tau, rt, wi);
-      if constexpr (PH == PH_DOWN) {
-#pragma unroll
-        for (int st = 0; st < NT; ++st) ew[st] = a.slot_w[((const int *)(info + 256))[min(16 * st + l16, ntok - 1)]];
-      }
-    }
-    // Is there a stage after this one (this task's next, or the next task's first)?
-    const bool last_stage = ls + 1 == nst;
-    const int tau_n = last_stage ? tasks.next(tau) : tau;
-    const bool more = !last_stage || tau_n < tasks.lim;
-    const int st_n = (step + 1) % S;
-    AOps nxt;
-    BOps nxtb;
-    if (more) {
-      nxt = read_a(st_n);
-      if constexpr (C::RA_B) nxtb = read_b(st_n);
-    }
-    if constexpr (!C::RA_B) curb = read_b(step % S);
-#ifdef HH_TRACE_STEPS
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#endif
-    if (PH == PH_UP) HH_TRS(step, 1);
-    if constexpr (FMT == Q_BF16) {
-      const int c = (SCOLS * ls) >> 7;
-      auto steps = [&](f32x4 (&ac)[NM][NT]) {
-#pragma unroll
-        for (int j = 0; j < SPS; ++j) {
-          const int v = ((SCOLS * ls) & 127) / 32 + j;
-          if (!F::step_ok(c, v, K)) break;
-#pragma unroll
-          for (int m = 0; m < NM; ++m)
-#pragma unroll
-            for (int st = 0; st < NT; ++st)
-#pragma unroll
-              for (int hh = 0; hh < NH; ++hh)
-                ac[m][st] = mfma(as_bf16x8(cur.w[0][m].w[j]), as_bf16x8(curb.b[0][st][hh][j]), ac[m][st]);
-        }
-      };
-      if ((c & 1) != cpar) {
-#pragma unroll
-        for (int m = 0; m < NM; ++m)
-#pragma unroll
-          for (int st = 0; st < NT; ++st) {
-            const f32x4 t = acc[0][m][st];
-            acc[0][m][st] = acc[1][m][st];
-            acc[1][m][st] = t;
-          }
-        cpar ^= 1;
-      }
-      steps(acc[0]);
-    } else {
-      // The (scale | bias) words of D rows 4g .. 4g+3 straight from the stage (16 contiguous
-      // bytes of each), instead of the lane's own row's words moved across lanes by shuffles.
-      const uint8_t *sbb = lds + (step % S) * C::STAGE + C::OFF_SB + wave * 1024 + 16 * g;
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const int c = 2 * ls + p;
-        if (64 * c >= K) break;
-        chunk_mfma<FMT, NM, NT, NH>(acc[c & 1], cur.w[p], at_unused,
-                                    [&](int st, int hh, int v) { return curb.b[p][st][hh][v]; }, c, g, K,
-                                    [&](int m) {
-                                      const u32x4 sv = *(const u32x4 *)(sbb + p * 256 + 64 * m);
-                                      const u32x4 bv = *(const u32x4 *)(sbb + 512 + p * 256 + 64 * m);
-                                      u32x4 r;
-#pragma unroll
-                                      for (int ii = 0; ii < 4; ++ii) r[ii] = (sv[ii] & 0xFFFFu) | (bv[ii] << 16);
-                                      return r;
-                                    });
-      }
-    }
-    if (last_stage) {
-      // ---- epilogue of the task ----
-      const ExpertGroup &grp = group_of(e);
-      const int out_dim = PH == PH_UP ? grp.inter : H;
-      const int rb = rt * C::ROWS + wave * 16 * RT;
-      const int *slots = (const int *)(lds + C::OFF_INFO + C::INFO * slot + 256);   // still this task's
-#pragma unroll
-      for (int st = 0; st < NT; ++st) {
-        if (16 * st + l16 >= ntok) continue;
-        const int es = slots[16 * st + l16];
-#pragma unroll
-        for (int q = 0; q < RT; ++q) {
-          if (rb + 16 * q >= out_dim) continue;
-          if constexpr (PH == PH_UP) {
-            up_epilogue<FMT>(a, nullptr, grp, rb + 16 * q + 4 * g, es,
-                             sum_chains(acc[0][q][st], acc[1][q][st]), sum_chains(acc[0][RT + q][st], acc[1][RT + q][st]));
-          } else {
-            const f32x4 r = sum_chains(acc[0][q][st], acc[1][q][st]);
-            f32x4 o;
-#pragma unroll
-            for (int ii = 0; ii < 4; ++ii) o[ii] = ew[st] * (r[ii] + 0.f);   // down_value's arithmetic
-            *(f32x4 *)(a.slot_out + (size_t)es * H + rb + 16 * q + 4 * g) = o;
-          }
-        }
-      }
-      zero();
-      tau = tau_n;
-      slot = slot == C::NSLOT - 1 ? 0 : slot + 1;
-      ls = 0;
-    } else {
-      ++ls;
-    }
-    if (PH == PH_UP) HH_TRS(step, 2);
-    if (!more) break;
-    ring_barrier();
-    if (PH == PH_UP) HH_TRS(step, 3);
-    cur = nxt;
-    if constexpr (C::RA_B) curb = nxtb;
-  }
-}
-
-// Row tiles per MFMA wave of the ring kernel: gate-up one (a gate and an up tile), down two.
-template <int PH, int FMT> constexpr int ring_rt() {
-  return PH == PH_DOWN ? 2 : 1;
-}
-
 // ---- launch table -----------------------------------------------------------------------------
 typedef void (*GemmKernel)(GemmArgs);
 typedef void (*UpSmallKernel)(GemmArgs, RouteArgs, FuseArgs);
@@ -3042,51 +2642,11 @@ static bool mlx_staged_down(int slots, int imax) {
   return imax <= 64 * (slots > 4 ? mlx_sb_chunks_down<kMaxTopK + 1>() : mlx_sb_chunks_down<4>());
 }
 
-// The ring kernel of a BF16 / MLX phase: 64-token work items (BF16 layers whose experts average
-// 64 or more tokens) or 32-token ones.
-template <int PH, int FMT> static GemmKernel ring_pick(int nt, size_t *lds) {
-  constexpr int RT = ring_rt<PH, FMT>();
-  if constexpr (FMT == Q_BF16) {
-    if (nt > 2) {
-      if (lds) *lds = Ring<PH, FMT, RT, 4>::LDS;
-      return prefill_ring<PH, FMT, RT, 4>;
-    }
-  }
-  if (lds) *lds = Ring<PH, FMT, RT, 2>::LDS;
-  return prefill_ring<PH, FMT, RT, 2>;
-}
-
-template <int PH, int FMT>
-static GemmKernel pick(int nt) {
-  if constexpr (FMT == Q_MXFP4) return nt <= 2 ? prefill_mx2<PH, 1> : prefill_mx2<PH, 2>;
-  else return ring_pick<PH, FMT>(nt, nullptr);
-}
-
-// Output rows per prefill workgroup: intermediates (gate-up) or hidden rows (down). The MXFP4
-// kernel covers 128 weight rows: 64 intermediates of the interleaved gate_up matrix.
+// Output rows per prefill_mx2 workgroup: 64 intermediates of the interleaved gate_up matrix, or 128
+// hidden rows.
 int gemm_rows_per_block(int quant, int phase) {
-  if (quant == Q_MXFP4) return phase == PH_UP ? 64 : 128;
-  return 64 * (phase == PH_UP ? ring_rt<PH_UP, Q_BF16>() : ring_rt<PH_DOWN, Q_BF16>());
-}
-
-static GemmKernel gemm_kernel(int phase, int quant, int nt) {
-  switch (quant) {
-  case Q_MXFP4: return phase == PH_UP ? pick<PH_UP, Q_MXFP4>(nt) : pick<PH_DOWN, Q_MXFP4>(nt);
-  case Q_BF16: return phase == PH_UP ? pick<PH_UP, Q_BF16>(nt) : pick<PH_DOWN, Q_BF16>(nt);
-  case Q_MLX4: return phase == PH_UP ? pick<PH_UP, Q_MLX4>(nt) : pick<PH_DOWN, Q_MLX4>(nt);
-  default: return phase == PH_UP ? pick<PH_UP, Q_MLX8>(nt) : pick<PH_DOWN, Q_MLX8>(nt);
-  }
-}
-
-// Dynamic LDS of the ring kernel of (phase, quant, token tile).
-static size_t ring_lds(int phase, int quant, int nt) {
-  size_t lds = 0;
-  switch (quant) {
-  case Q_BF16: (void)(phase == PH_UP ? ring_pick<PH_UP, Q_BF16>(nt, &lds) : ring_pick<PH_DOWN, Q_BF16>(nt, &lds)); break;
-  case Q_MLX4: (void)(phase == PH_UP ? ring_pick<PH_UP, Q_MLX4>(nt, &lds) : ring_pick<PH_DOWN, Q_MLX4>(nt, &lds)); break;
-  default: (void)(phase == PH_UP ? ring_pick<PH_UP, Q_MLX8>(nt, &lds) : ring_pick<PH_DOWN, Q_MLX8>(nt, &lds)); break;
-  }
-  return lds;
+  (void)quant;
+  return phase == PH_UP ? 64 : 128;
 }
 
 static int device_cus() {
@@ -3157,47 +2717,28 @@ template <int PH, int TT> static hipError_t launch_mxa(GemmArgs a, hipStream_t s
 hipError_t launch_prefill(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm);   // hh_prefill.hip
 
 hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &args, hipStream_t s, Timing tm) {
-  if (quant == Q_BF16) return launch_prefill(phase, quant, nt, args, s, tm);
-  // Persistent kernels: XCD split into row-tile parts × work-item parts (Mx3Tasks). Measured on
-  // the benchmark layers (prefill T = 512..2048) against 8 row-tile parts: BF16 gate-up 832 →
-  // 615 µs with 4 or 2 parts, BF16 down 414 → 371 µs with 2; MLX 3-5 % faster with 4; MXFP4
-  // within ±2 % (its down fetches 18 % fewer bytes with 4).
+  if (quant != Q_MXFP4) return launch_prefill(phase, quant, nt, args, s, tm);
+  // Persistent kernels: XCD split into row-tile parts × work-item parts (Mx3Tasks): MXFP4 within
+  // ±2 % of 8 row-tile parts (its down fetches 18 % fewer bytes with 4).
   GemmArgs a = args;
-  a.xcd_rows = (quant == Q_BF16 && phase == PH_DOWN) ? 2 : 4;
-  if (quant == Q_MXFP4 && use_mxa(phase, a, nt))
+  a.xcd_rows = 4;
+  if (use_mxa(phase, a, nt))
     return nt == 2 ? launch_mxa<PH_UP, 2>(a, s, tm) : launch_mxa<PH_UP, 4>(a, s, tm);
-  if (quant == Q_MXFP4 && nt == 4 && phase == PH_DOWN && a.slots == a.top_k &&
+  if (nt == 4 && phase == PH_DOWN && a.slots == a.top_k &&
       (a.grp[0].inter + 127) / 128 >= Mx3<PH_DOWN, 1, 2>::S)
     return launch_mx3<PH_DOWN, 1, 2>(a, s, tm);
-  if (quant == Q_MXFP4 && use_mx3(phase, a, nt)) {
+  if (use_mx3(phase, a, nt)) {
     if (!mx3_wide(phase, a)) return phase == PH_UP ? launch_mx3<PH_UP, 1, 1>(a, s, tm) : launch_mx3<PH_DOWN, 1, 1>(a, s, tm);
     return phase == PH_UP ? launch_mx3<PH_UP, 2, 1>(a, s, tm) : launch_mx3<PH_DOWN, 2, 1>(a, s, tm);
-  }
-  if (quant != Q_MXFP4) {
-    // BF16 / MLX: the persistent ring kernel, one workgroup per compute unit.
-    static std::once_flag once;
-    std::call_once(once, [] {
-      for (int ph = 0; ph < 2; ++ph)
-        for (int q : {Q_BF16, Q_MLX4, Q_MLX8})
-          for (int nt : {2, 4}) {
-            (void)hipFuncSetAttribute((const void *)gemm_kernel(ph, q, nt), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                      160 * 1024);
-            (void)hipGetLastError();
-          }
-    });
-    if (a.max_work == 0) return hipSuccess;
-    hipExtLaunchKernelGGL(gemm_kernel(phase, quant, nt), dim3(device_cus()), dim3(512), ring_lds(phase, quant, nt), s,
-                          tm.start, tm.stop, 0, a);
-    return hipGetLastError();
   }
   // prefill_tile: 8 XCDs × ⌈row_tiles / 8⌉ row tiles × work items.
   const unsigned blocks = 8u * (unsigned)((a.row_tiles + 7) / 8) * (unsigned)a.max_work;
   if (blocks == 0) return hipSuccess;
-  const bool mx = quant == Q_MXFP4;
-  // MXFP4: 8 waves, the weight rows' scales (128 rows × K/32 bytes) in dynamic LDS.
-  const size_t lds = mx ? (size_t)128 * ((phase == PH_UP ? a.hidden : a.ldh) / 32) : 0;
-  hipExtLaunchKernelGGL(gemm_kernel(phase, quant, nt), dim3(blocks), dim3(mx ? 512 : 256), lds, s, tm.start,
-                        tm.stop, 0, a);
+  // 8 waves, the weight rows' scales (128 rows × K/32 bytes) in dynamic LDS.
+  const size_t lds = (size_t)128 * ((phase == PH_UP ? a.hidden : a.ldh) / 32);
+  GemmKernel k = phase == PH_UP ? (nt <= 2 ? prefill_mx2<PH_UP, 1> : prefill_mx2<PH_UP, 2>)
+                                : (nt <= 2 ? prefill_mx2<PH_DOWN, 1> : prefill_mx2<PH_DOWN, 2>);
+  hipExtLaunchKernelGGL(k, dim3(blocks), dim3(512), lds, s, tm.start, tm.stop, 0, a);
   return hipGetLastError();
 }
 

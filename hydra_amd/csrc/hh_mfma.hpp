@@ -16,8 +16,8 @@ __device__ __forceinline__ f32x4 mfma(const bf16x8 &a, const bf16x8 &b, const f3
 
 // Two unsigned integers < 256 → packed bf16 pair (exact: 8 significant bits).
 __device__ __forceinline__ uint32_t u8pair_to_bf16x2(uint32_t lo, uint32_t hi) {
-  uint32_t a = __float_as_uint((float)lo), b = __float_as_uint((float)hi);
-  return (a >> 16) | (b & 0xFFFF0000u);
+  const uint32_t a = __float_as_uint((float)lo), b = __float_as_uint((float)hi);
+  return __builtin_amdgcn_perm(b, a, 0x07060302u);   // the upper halves
 }
 
 // 8 4-bit MLX values of one word (low-order first) → bf16 integers.
@@ -462,9 +462,6 @@ struct Mx3Tasks {
   }
 };
 
-__device__ __forceinline__ void lds_load2(const void *g, uint8_t *l) {
-  __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)l, 2, 0, 0);
-}
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 }  // namespace hh

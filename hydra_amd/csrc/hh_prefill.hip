@@ -18,6 +18,13 @@ __device__ __forceinline__ void dma16(const void *base, uint32_t off, uint32_t l
 __device__ __forceinline__ void dma16(const void *p, uint32_t l) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(p) : "memory");
 }
+// 4 (2) bytes per lane to LDS byte `l` + 4·lane.
+__device__ __forceinline__ void dma4(const void *p, uint32_t l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(l), "v"(p) : "memory");
+}
+__device__ __forceinline__ void dma2(const void *p, uint32_t l) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" ::"s"(l), "v"(p) : "memory");
+}
 // Barrier after the wave's own LDS reads have returned: the next stage may overwrite what they read.
 __device__ __forceinline__ void step_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 __device__ __forceinline__ uint32_t lds_addr(const uint8_t *l) { return (uint32_t)(uintptr_t)(lds_ptr_t)(void *)l; }
@@ -30,7 +37,7 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // workgroup per compute unit, four loader waves and four MFMA waves) each SIMD had a single MFMA
 // wave, which sat through its own LDS reads and barrier at every stage (with no global traffic at
 // all the BF16 T = 2048 gate-up still took 350 of its 415 us).
-// Weight loads take whole 128-byte pieces of a row with consecutive lanes: 50 B/clk
+// Weight loads take whole 128-byte (4-bit MLX: 64-byte) pieces of a row with consecutive lanes: 50 B/clk
 // per compute unit from L2, against 15.5 for the MFMA lane order (16 rows × 64 bytes, consecutive
 // lanes on different rows), which the L1 serves a row at a time when the row stride is a multiple
 // of 128 bytes. The XOR of the 16-byte segments by the row keeps the MFMA lanes' LDS reads at full rate.
@@ -205,6 +212,265 @@ __global__ __launch_bounds__(256 * WT_) __attribute__((amdgpu_waves_per_eu(2, 2)
   }
 }
 
+// ---- MLX affine -----------------------------------------------------------------------------------
+// A stage is two 64-column groups. Bound by VALU work where experts have many tokens: per group and wave, 14
+// operations to expand a 16-row tile's 4-bit codes (24 for 8-bit), and eight per tile and token tile
+// to scale the group's partial sums; the MFMAs take a third of that. Two things keep the rest small:
+// the group scales become fp32 once per row (one row per lane, through LDS) instead of in every
+// lane of the 16 that share a D row (48 operations per group, T = 1024 gate-up 151 -> 135 us), and the
+// lane's LDS offsets are formed once. 256-expert layer (H 2048, I 512), gate-up / down us:
+//   4-bit T = 1024 135 / 112 (before: 227 / 160), T = 333 110 / 67 (158 / 104), T = 60 85 / 53 (125 / 85);
+//   8-bit T = 333 137 / 79 (170 / 99), T = 1024 176 / 126 (237 / 154).
+// RT: 4-bit gate-up tiles of 128 intermediates 135, of 64 157 (an operand pair is expanded for half
+// the rows); 4-bit down tiles of 192 rows 112, of 256 115 (spills), of 128 120; 8-bit down tiles of 128
+// rows 79 at T = 333, of 64 115; wider 8-bit tiles leave one stage in LDS.
+template <int PH, int BITS, int RT_, int NT_> struct Ml {
+  static constexpr int NT = NT_, NH = PH == PH_UP ? 1 : 2;
+  static constexpr int RT = RT_, NM = (PH == PH_UP ? 2 : 1) * RT;
+  static constexpr int ROWS = 64 * RT;
+  static constexpr int AK = BITS / 4;                        // KiB of a 16-row tile per stage
+  static constexpr int APW = NM * AK, BPW = NH * NT;         // 1 KiB loads per wave per stage
+  static constexpr int L = APW + BPW + 2;
+  static constexpr int OFF_B = 4 * APW * 1024;
+  static constexpr int OFF_SB = OFF_B + 4 * BPW * 1024;      // per wave: scale words, bias words of 64 rows
+  static constexpr int STAGE = OFF_SB + 4 * 512;
+  static constexpr int S_FIT = (76 * 1024) / STAGE, S = S_FIT > 4 ? 4 : S_FIT;
+  static constexpr int OFF_F = S * STAGE;                    // per wave: [group][scale, bias][64 rows] fp32
+  static constexpr int LDS = OFF_F + 4 * 1024;
+  static_assert(S >= 2 && NM <= 4, "ring depth");
+};
+
+template <int PH, int BITS, int RT_, int NT_>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_mlx(GemmArgs a) {
+  using C = Ml<PH, BITS, RT_, NT_>;
+  constexpr int NM = C::NM, NT = C::NT, NH = C::NH, RT = C::RT, S = C::S, L = C::L, AK = C::AK;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int H = a.hidden, E = a.experts;
+  const int nwork = *a.n_work;
+  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, a.row_tiles, nwork, a.xcd_rows);
+  if ((int)blockIdx.x >= tasks.lim) return;
+  int rt, wi;
+  tasks.tile((int)blockIdx.x, rt, wi);
+  if (rt >= a.row_tiles || wi >= nwork) return;
+  const int4 it = a.work[wi];
+  const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
+  const ExpertGroup &grp = a.grp[e == E ? 1 : 0];
+  const uint8_t *blob = grp.blobs + (e == E ? 0 : (size_t)e * grp.stride);
+  const int I = grp.inter;
+  const int K = PH == PH_UP ? H : I, out_dim = PH == PH_UP ? I : H;
+  const int ng = K / 64, n = (ng + 1) / 2;   // groups; stages of two
+  if (rt * C::ROWS >= out_dim) return;
+  const int rb = rt * C::ROWS + wave * 16 * RT;
+  const bool active = rb < out_dim;
+
+  constexpr int SEGS = 4 * AK, RPI = 16 / AK;   // 16-byte segments per weight row, rows per load
+  const int rowb = K * BITS / 8;
+  auto aswz = [](int r) { return AK == 1 ? (r >> 1) & 3 : r & 7; };
+  const int lr = lane / SEGS, seg = (lane % SEGS) ^ aswz(lr);
+  // The last stage of an odd group count has one group: lanes past it repeat that group's bytes.
+  const uint32_t aoff = (uint32_t)(lr * rowb + 16 * seg);
+  const uint32_t aoff_t = (ng & 1) ? (uint32_t)(lr * rowb + 16 * (seg & (SEGS / 2 - 1))) : aoff;
+  const uint8_t *abase[C::APW];
+#pragma unroll
+  for (int i = 0; i < C::APW; ++i) {
+    const int m = i / AK, mat = PH == PH_UP ? (m >= RT ? 1 : 0) : 2;
+    const int r0 = min(rb + 16 * (m % RT), out_dim - 16);
+    abase[i] = blob + grp.off[3 * mat] + (size_t)(r0 + RPI * (i % AK)) * rowb;
+  }
+  // Lane 16m + r: the two groups' scales (biases) of row r of tile m, one dword.
+  const uint8_t *ssrc, *zsrc;
+  {
+    const int m = min(lane >> 4, NM - 1), mat = PH == PH_UP ? (m >= RT ? 1 : 0) : 2;
+    const size_t r = min(rb + 16 * (m % RT), out_dim - 16) + l16;
+    ssrc = blob + grp.off[3 * mat + 1] + r * ng * 2;
+    zsrc = blob + grp.off[3 * mat + 2] + r * ng * 2;
+  }
+  // Operand load j of the stage: 4 token rows of 256 bytes.
+  const uint8_t *bsrc[C::BPW];
+  uint32_t bdst[C::BPW];
+  int btail[C::BPW];
+#pragma unroll
+  for (int i = 0; i < C::BPW; ++i) {
+    const int j = wave * C::BPW + i, hh = j / (4 * NT), tl = j % (4 * NT);
+    const int tn = 4 * tl + (lane >> 4), sl = a.order[pos + min(tn, cnt - 1)];
+    const uint16_t *row = PH == PH_UP ? a.x + (size_t)(sl / a.slots) * H : (hh ? a.h_lo : a.h_hi) + (size_t)sl * a.ldh;
+    const int sg = l16 ^ (tn & 15);
+    bsrc[i] = (const uint8_t *)row + 16 * sg;
+    btail[i] = (ng & 1) && sg >= 8 ? 128 : 0;
+    bdst[i] = lds_addr(lds) + C::OFF_B + 1024 * j;
+  }
+  int es[NT];
+#pragma unroll
+  for (int st = 0; st < NT; ++st) es[st] = a.order[pos + min(16 * st + l16, cnt - 1)];
+
+  const uint32_t adst = lds_addr(lds) + wave * C::APW * 1024;
+  const uint32_t sdst = lds_addr(lds) + C::OFF_SB + wave * 512;
+  int q = 0, qs = 0;
+  auto issue = [&]() {
+    const uint32_t so = (uint32_t)(qs * C::STAGE);
+    const bool tail = q == n - 1;
+    const uint32_t ao = tail ? aoff_t : aoff;
+#pragma unroll
+    for (int i = 0; i < C::APW; ++i) dma16(abase[i] + 64 * AK * q, ao, adst + so + 1024 * i);
+#pragma unroll
+    for (int i = 0; i < C::BPW; ++i) dma16(bsrc[i] + (256 * q - (tail ? btail[i] : 0)), bdst[i] + so);
+    // A dword holds groups 2q and 2q + 1; the last stage of an odd count reads its group alone.
+    if (tail && (ng & 1)) {
+      dma2(ssrc + 4 * q, sdst + so);
+      dma2(zsrc + 4 * q, sdst + so + 256);
+    } else {
+      dma4(ssrc + 4 * q, sdst + so);
+      dma4(zsrc + 4 * q, sdst + so + 256);
+    }
+    ++q;
+    qs = qs == S - 1 ? 0 : qs + 1;
+  };
+  for (int u = 0; u < S - 1 && q < n; ++u) issue();
+
+  f32x4 acc[2][NM][NT];
+#pragma unroll
+  for (int p = 0; p < 2; ++p)
+#pragma unroll
+    for (int m = 0; m < NM; ++m)
+#pragma unroll
+      for (int st = 0; st < NT; ++st) acc[p][m][st] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // The lane's offsets in a stage: its codes (group 1: ^ 32 · AK), its operand segments (group, step: ^ 128, ^ 16).
+  const uint32_t alo = wave * NM * AK * 1024 + 64 * AK * l16 +
+                       (BITS == 4 ? 16 * ((g >> 1) ^ aswz(l16)) + 8 * (g & 1) : 16 * (g ^ aswz(l16)));
+  const uint32_t blo = C::OFF_B + 256 * l16 + 16 * ((2 * g) ^ l16);
+  float *fsb = (float *)(lds + C::OFF_F) + 256 * wave + lane;
+  const float *fsr = (const float *)(lds + C::OFF_F) + 256 * wave + 4 * g;
+  int ss = 0;
+#pragma unroll 1
+  for (int s = 0; s < n; ++s) {
+    const int later = q - 1 - s;
+    if (later >= S - 2) wait_vm<(S - 2) * L>();
+    else if (S > 3 && later == 1) wait_vm<L>();
+    else wait_vm<0>();
+    step_barrier();
+    if (q < n) issue();
+    const uint8_t *stg = lds + ss * C::STAGE;
+    ss = ss == S - 1 ? 0 : ss + 1;
+    if (!active) continue;
+    {
+      // The wave's 64 rows, one per lane: scale and bias of both groups as fp32 (the 4-bit bias
+      // less 128 scales), written for the D rows' reads below. Every lane would otherwise convert
+      // the values of its four D rows of each tile.
+      const uint32_t sw = *(const uint32_t *)(stg + C::OFF_SB + wave * 512 + 4 * lane);
+      const uint32_t zw = *(const uint32_t *)(stg + C::OFF_SB + wave * 512 + 256 + 4 * lane);
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const float sc = __uint_as_float(p ? sw & 0xFFFF0000u : sw << 16);
+        const float z = __uint_as_float(p ? zw & 0xFFFF0000u : zw << 16);
+        fsb[128 * p] = sc;
+        fsb[128 * p + 64] = BITS == 4 ? __builtin_fmaf(-128.f, sc, z) : z;
+      }
+      __builtin_amdgcn_wave_barrier();
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      if (2 * s + p >= ng) break;   // an odd group count's last stage has one
+      // Codes of group 2s + p as bf16 (chunk_mfma's forms); its scales and biases of D rows 4g .. 4g + 3.
+      u32x4 av[NM][2];
+      f32x4 sc[NM], bi[NM];
+#pragma unroll
+      for (int m = 0; m < NM; ++m) {
+        const uint8_t *tile = stg + m * AK * 1024;
+        if constexpr (BITS == 4) {
+          const u32x2 c = *(const u32x2 *)(tile + (alo ^ (32 * p)));
+#pragma unroll
+          for (int v = 0; v < 2; ++v)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) av[m][v][k] = ((c[v] >> (4 * k)) & 0x000F000Fu) | 0x43004300u;
+        } else {
+          const u32x4 c = *(const u32x4 *)(tile + (alo ^ (64 * p)));
+#pragma unroll
+          for (int v = 0; v < 2; ++v) av[m][v] = __builtin_bit_cast(u32x4, mlx8_to_bf16(c[2 * v], c[2 * v + 1]));
+        }
+        sc[m] = *(const f32x4 *)(fsr + 128 * p + 16 * m);
+        bi[m] = *(const f32x4 *)(fsr + 128 * p + 64 + 16 * m);
+      }
+      const u32x4 ones = {0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u};   // bf16 1.0
+#pragma unroll
+      for (int st = 0; st < NT; ++st) {
+        if (st > 0 && 16 * st >= cnt) break;   // token tiles wholly past the item
+        u32x4 b[NH][2];
+#pragma unroll
+        for (int hh = 0; hh < NH; ++hh)
+#pragma unroll
+          for (int v = 0; v < 2; ++v) {
+            const u32x4 r = *(const u32x4 *)(stg + (hh * NT + st) * 4096 + (blo ^ (128 * p + 16 * v)));
+            if constexpr (BITS == 4) {
+              // (x0,x1)(x2,x3)(x4,x5)(x6,x7) → (x0,x4)(x1,x5)(x2,x6)(x3,x7), the codes' pairing
+              b[hh][v] = u32x4{__builtin_amdgcn_perm(r[2], r[0], 0x05040100u), __builtin_amdgcn_perm(r[2], r[0], 0x07060302u),
+                               __builtin_amdgcn_perm(r[3], r[1], 0x05040100u), __builtin_amdgcn_perm(r[3], r[1], 0x07060302u)};
+            } else {
+              b[hh][v] = r;
+            }
+          }
+        f32x4 G = {0.f, 0.f, 0.f, 0.f}, P[NM];
+#pragma unroll
+        for (int m = 0; m < NM; ++m) P[m] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+          for (int hh = 0; hh < NH; ++hh) {
+            G = mfma(as_bf16x8(ones), as_bf16x8(b[hh][v]), G);
+#pragma unroll
+            for (int m = 0; m < NM; ++m) P[m] = mfma(as_bf16x8(av[m][v]), as_bf16x8(b[hh][v]), P[m]);
+          }
+#pragma unroll
+        for (int m = 0; m < NM; ++m)
+#pragma unroll
+          for (int ii = 0; ii < 4; ++ii) {
+            acc[p][m][st][ii] = __builtin_fmaf(sc[m][ii], P[m][ii], acc[p][m][st][ii]);
+            acc[p][m][st][ii] = __builtin_fmaf(bi[m][ii], G[ii], acc[p][m][st][ii]);
+          }
+      }
+    }
+  }
+  if (!active) return;
+#pragma unroll
+  for (int st = 0; st < NT; ++st) {
+    if (16 * st + l16 >= cnt) continue;
+    const float ew = PH == PH_DOWN ? a.slot_w[es[st]] : 0.f;
+#pragma unroll
+    for (int r = 0; r < RT; ++r) {
+      const int r0 = rb + 16 * r;
+      if (r0 >= out_dim) continue;
+      if constexpr (PH == PH_UP) {
+        up_epilogue<Q_BF16>(a, nullptr, grp, r0 + 4 * g, es[st], sum_chains(acc[0][r][st], acc[1][r][st]),
+                            sum_chains(acc[0][RT + r][st], acc[1][RT + r][st]));
+      } else {
+        const f32x4 v = sum_chains(acc[0][r][st], acc[1][r][st]);
+        f32x4 o;
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) o[ii] = ew * (v[ii] + 0.f);   // down_value's arithmetic
+        *(f32x4 *)(a.slot_out + (size_t)es[st] * H + r0 + 4 * g) = o;
+      }
+    }
+  }
+}
+
+template <int PH, int BITS, int RT, int NT> static hipError_t launch_mlx(GemmArgs a, hipStream_t s, Timing tm) {
+  using C = Ml<PH, BITS, RT, NT>;
+  static std::once_flag once;
+  std::call_once(once, [] {
+    (void)hipFuncSetAttribute((const void *)prefill_mlx<PH, BITS, RT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+    (void)hipGetLastError();
+  });
+  const int rows = PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
+  a.row_tiles = (rows + C::ROWS - 1) / C::ROWS;
+  a.xcd_rows = 2;
+  const int P = a.xcd_rows;
+  const unsigned blocks = 8u * (unsigned)((a.row_tiles + P - 1) / P) * (unsigned)((a.max_work + 8 / P - 1) / (8 / P));
+  if (blocks == 0) return hipSuccess;
+  hipExtLaunchKernelGGL((prefill_mlx<PH, BITS, RT, NT>), dim3(blocks), dim3(256), C::LDS, s, tm.start, tm.stop, 0, a);
+  return hipGetLastError();
+}
+
 template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(GemmArgs a, hipStream_t s, Timing tm) {
   using C = Bf<PH, NT, RT, SV, WT>;
   static std::once_flag once;
@@ -223,9 +489,11 @@ template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(
 }
 
 // The tile of each call. BF16 work items hold 160 tokens (nt 10: experts averaging 40 tokens or
-// more) or 32.
+// more) or 32; the MLX formats' always 32.
 hipError_t launch_prefill(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
   const bool up = phase == PH_UP;
+  if (quant == Q_MLX4) return up ? launch_mlx<PH_UP, 4, 2, 2>(a, s, tm) : launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
+  if (quant == Q_MLX8) return up ? launch_mlx<PH_UP, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
   if (quant != Q_BF16) return hipErrorInvalidValue;
   if (nt == 10) return up ? launch_bf16<PH_UP, 5, 2, 2, 2>(a, s, tm) : launch_bf16<PH_DOWN, 5, 4, 2, 2>(a, s, tm);
   return up ? launch_bf16<PH_UP, 2, 1, 2, 1>(a, s, tm) : launch_bf16<PH_DOWN, 2, 2, 2, 1>(a, s, tm);

@@ -1,5 +1,5 @@
 """The prefill products (T > 16) at the edges of their tiles: row tiles past the last row, a last
-stage of one step, token tiles past an item's tokens, experts of more than one work
+stage of one step or one group, token tiles past an item's tokens, experts of more than one work
 item, both item sizes. Against the fp64 oracle, and bit for bit against one-token calls.
 
 Bound: activations travel as a bf16 hi + lo pair (2^-17 of the value each), fp32 sums over at most a
@@ -13,12 +13,18 @@ from hydra_amd import synth
 REL = 2e-5
 
 BF16 = F.GEMMA_BF16.replace(experts=3, top_k=2)
+MLX4 = F.QWEN_35B_A3B_Q4.replace(experts=3, top_k=2)
 CASES = {
     # name: (desc, tokens); 2T/3 tokens an expert
     "bf16_32_small": (BF16.replace(hidden=64, intermediate=64), 17),      # one stage
     "bf16_32_ragged": (BF16.replace(hidden=192, intermediate=320), 59),   # 39 an expert: two items of 32
     "bf16_160_edge": (BF16.replace(hidden=192, intermediate=320), 60),    # 40 an expert: items of 160
     "bf16_160_two": (BF16.replace(hidden=832, intermediate=192), 300),    # 200 an expert: 160 + 40
+    "mlx4_one_group": (MLX4.replace(hidden=64, intermediate=64, shared_intermediate=64), 17),
+    "mlx4_odd_groups": (MLX4.replace(hidden=320, intermediate=192, shared_intermediate=320), 100),
+    "mlx4_even_groups": (MLX4.replace(hidden=640, intermediate=384, shared_intermediate=0), 49),
+    "mlx8_one_group": (MLX4.replace(quant=F.QUANT_MLX8, hidden=64, intermediate=64, shared_intermediate=0), 50),
+    "mlx8_odd_groups": (MLX4.replace(quant=F.QUANT_MLX8, hidden=448, intermediate=320, shared_intermediate=192), 70),
 }
 
 
