@@ -21,7 +21,6 @@ hipError_t launch_small(int quant, GemmArgs a, const RouteArgs &ra, hipStream_t 
                         Timing tm_down, const FuseArgs *fr = nullptr);
 bool fused_router_fits(int quant, int H, int E, int router, int T);
 int fused_router_flags(int T, int E);
-int gemm_rows_per_block(int quant, int phase);
 size_t decode_fused_lds(const GemmArgs &a, int T);
 bool decode_fused_fits(int H, int I, int E, int K, int shared_inter);
 int decode_fused_flags(int T, int E, int K, int I);
@@ -164,10 +163,9 @@ int token_tile_nt(const hh_moe_desc &d, int T) {
   // Prefill work items of 16·nt tokens: MXFP4 32 or 64 (below), BF16 160 once experts
   // average 40 tokens or more (the weight tile is then read once per 160 tokens), else 32.
   if (d.quant == HH_QUANT_BF16 && (int64_t)T * d.top_k >= 40 * (int64_t)d.experts) return 10;
-  // MXFP4 without a shared expert, experts averaging 16 or more tokens, rows long enough for the
-  // LDS rings: 64-token items for the gate-up (its 256 × 64 tiles skip the MFMAs of padding token
-  // tiles, and an expert's rows are read once per 64 tokens); the down product runs the same
-  // segments as 32-token items (Scratch::half_down).
+  // MXFP4 without a shared expert, experts averaging 16 or more tokens (rows below 1024 columns: not
+  // measured): 64-token items for the gate-up (an expert's rows are read once per 64 tokens); the
+  // down product runs the same segments as 32-token items (Scratch::half_down).
   if (d.quant == HH_QUANT_MXFP4 && d.shared_intermediate == 0 && (int64_t)T * d.top_k >= 16 * (int64_t)d.experts &&
       d.hidden >= 1024 && d.intermediate >= 1024)
     return 4;
@@ -203,9 +201,8 @@ Scratch plan(const hh_moe_desc &d, int T) {
   s.work = take(sizeof(int4) * (size_t)s.max_work);
   s.n_work = take(sizeof(int32_t));
   s.dcount = take((size_t)A >= (size_t)hh::DB_MIN_ASSIGN ? sizeof(int32_t) * hh::DB_MAX * E : 0);
-  // MXFP4 batches of 64-token items: the down product takes 32-token items of 256 rows, which
-  // re-read the three activation terms half as often per row as 128-row tiles (a 256 × 64 tile
-  // does not fit the register file).
+  // MXFP4 batches of 64-token items: the down product takes 32-token items (three operand terms:
+  // a 64-token stage leaves its ring one slot).
   s.half_down = d.quant == HH_QUANT_MXFP4 && s.nt == 4 && !shared;
   s.max_work_half = s.half_down ? std::min(E, A) + (A + s.tile_tokens / 2 - 1) / (s.tile_tokens / 2) : 0;
   s.work_half = take(sizeof(int4) * (size_t)s.max_work_half);
@@ -579,12 +576,8 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
     ctx->dispatches += fr ? 2 : 3;
     return HH_OK;
   }
-  int rows = hh::gemm_rows_per_block(d->quant, 0);
-  g.row_tiles = (s.ldh + rows - 1) / rows;
   if ((rc = phase_timing(ctx, &tm, noalloc))) return rc;
   HH_HIP(hh::launch_gemm(0, d->quant, s.nt, g, ctx->stream, tm));
-  rows = hh::gemm_rows_per_block(d->quant, 1);
-  g.row_tiles = (d->hidden + rows - 1) / rows;
   if ((rc = phase_timing(ctx, &tm, noalloc))) return rc;
   if (s.half_down) {
     hh::GemmArgs gd = g;
@@ -1145,8 +1138,6 @@ int hh_expert_gemm(hh_ctx *ctx, const hh_matrix *m, const float *x, int32_t T, f
   if (T <= kSmallT) {
     HH_HIP(hh::launch_down_small(q, g, topk, T, ctx->stream, hh::Timing{}));
   } else {
-    const int rows = hh::gemm_rows_per_block(q, 1);
-    g.row_tiles = (R + rows - 1) / rows;
     g.max_work = items;
     HH_HIP(hh::launch_gemm(1, q, 2, g, ctx->stream, hh::Timing{}));
   }

@@ -26,9 +26,7 @@
 //     tokens' x rows staged in LDS. down_small computes 16 hidden rows of one token for all of
 //     its slots (one wave per slot) and sums them in rank order in the epilogue: no slot buffer,
 //     no combine launch.
-//   prefill_gemm (T > 16): a work list of (expert, first position, ≤ 16·NT tokens) from the
-//     device-side dispatch; 4 waves on different row tiles share the B chunk staged in LDS;
-//     slot values go to slot_out and combine_kernel sums them in rank order.
+//   T > 16: hh_prefill.hip.
 //
 // MFMA operand mapping (16x16x32, lane l, lane group g = l/16): A lane l supplies row l%16,
 // B lane l supplies token column l%16, each with 8 consecutive K values; D lane l holds rows
@@ -175,18 +173,6 @@ __device__ __forceinline__ f32x4 down_value(const GemmArgs &a, const uint8_t *bl
   return o;
 }
 
-// Prefill block order: hardware places block b on XCD b % 8. XCD x takes the row tiles
-// [x·rtx, x·rtx + rtx) (rtx = ⌈row_tiles / 8⌉) and walks the work items in order, an item's row
-// tiles consecutively: the item's activation operand is fetched about once per XCD and reused
-// from its L2 by the item's row tiles, and an expert's weight rows by its consecutive items.
-// (Row-tile-major order re-read every item's operand from HBM once per row tile.)
-__device__ __forceinline__ void prefill_tile(int b, int row_tiles, int &rt, int &wi) {
-  const int rtx = (row_tiles + 7) >> 3;
-  const int x = b & 7, j = b >> 3;
-  wi = j / rtx;
-  rt = x * rtx + (j - wi * rtx);
-}
-
 // Copies vectors v ∈ [base, base + threads·NB) ∩ [0, n) with `threads` threads (thread index
 // `id`): the loads of the batch are all issued before any store, so a batch costs one memory
 // latency (a load-store loop would wait for each load in turn, and, completion being in order,
@@ -216,16 +202,8 @@ static __device__ uint64_t hh_trace_buf[3 * kTraceBlocks * kTracePoints];
     if (threadIdx.x == 0 && blockIdx.x < kTraceBlocks)                                         \
       hh_trace_buf[((kern) * kTraceBlocks + blockIdx.x) * kTracePoints + (point)] = wall_clock64(); \
   } while (0)
-// Per-step stamps (core clock) of MFMA wave 0 of workgroup 0 of the MXFP4 prefill gate-up:
-// hh_trace_buf[2][step][point], steps < kTraceBlocks.
-#define HH_TRS(step, point)                                                                      \
-  do {                                                                                           \
-    if (threadIdx.x == 0 && blockIdx.x == 0 && (step) < kTraceBlocks)                            \
-      hh_trace_buf[(2 * kTraceBlocks + (step)) * kTracePoints + (point)] = clock64();            \
-  } while (0)
 #else
 #define HH_TR(kern, point) do {} while (0)
-#define HH_TRS(step, point) do {} while (0)
 #endif
 
 // ---- decode prologue -----------------------------------------------------------------------------
@@ -550,41 +528,11 @@ __global__ __launch_bounds__(256 * TPW) void up_small(GemmArgs a, RouteArgs ra, 
   }
 }
 
-// B operand of chunk c from one term row (bytes, K columns) and its block scales `srow`; columns
-// at or past K read as zero and their blocks' scales as 2^0, so only finite values meet the zeroed
-// weights of a tail chunk.
+// B operand of a chunk: the two 16-byte halves of the lane's K columns and their block's scale.
 struct MxB {
   u32x4 lo, hi;
   uint32_t s;
 };
-__device__ __forceinline__ MxB mx_b(const uint8_t *row, const uint8_t *srow, int c, int g, int K) {
-  const int k0 = 128 * c + 16 * g;
-  MxB b;
-  b.lo = *(const u32x4 *)(row + k0);
-  b.hi = *(const u32x4 *)(row + k0 + 64);
-  b.s = srow[4 * c + g];
-  if (k0 >= K) b.lo = u32x4{0u, 0u, 0u, 0u};
-  if (k0 + 64 >= K) b.hi = u32x4{0u, 0u, 0u, 0u};
-  if (128 * c + 32 * g >= K) b.s = 127u;
-  return b;
-}
-
-// One chunk of the canonical MXFP4 arithmetic: acc += A·B_t for the terms t in order.
-template <int NM, int NT, int NTERM, class BF>
-__device__ __forceinline__ void chunk_mx(f32x4 (&acc)[NM][NT], const u32x4 (&w)[NM], const uint32_t (&sa)[NM], BF bf,
-                                         int c, int g, int K) {
-  const bool ok = Fmt<Q_MXFP4>::lane_valid(c, g, K);
-#pragma unroll
-  for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-    for (int st = 0; st < NT; ++st) {
-      const MxB b = bf(st, t);
-#pragma unroll
-      for (int m = 0; m < NM; ++m)
-        acc[m][st] = smfma(ok ? w[m] : u32x4{0u, 0u, 0u, 0u}, b.lo, b.hi, sa[m] & 0xFFu, b.s, acc[m][st]);
-    }
-}
-
 // The operands of one chunk that come from LDS, read unmasked: the B operand of every term and
 // the e8m0 scale of the wave's weight block.
 template <int NTERM> struct MxOps {
@@ -605,9 +553,9 @@ __device__ __forceinline__ MxOps<NTERM> mx_ops(const uint8_t *brow, int RS, int 
   o.sa = my_sc[min(4 * c + g, nsb - 1)];
   return o;
 }
-// chunk_mx for one tile and one token tile with pre-read operands, which come from rows staged by
-// MxStage (zero past K, scales 2^0 there): the same values mx_b's masks give. Lanes whose weight
-// block lies past K take zero weights, as in chunk_mx.
+// One chunk of the canonical MXFP4 arithmetic, acc += A·B_t for the terms t in order, for one tile and
+// one token tile with pre-read operands, which come from rows staged by MxStage (zero past K,
+// scales 2^0 there). Lanes whose weight block lies past K take zero weights.
 // `full`: the chunk lies wholly inside K (no lane needs the test).
 template <int NTERM>
 __device__ __forceinline__ void chunk_mx1(f32x4 &acc, const u32x4 &w, const MxOps<NTERM> &o, int c, int g, int K,
@@ -1621,233 +1569,6 @@ __global__ __launch_bounds__(256, 2) void decode_mx(GemmArgs a, RouteArgs ra, Fu
   }
 }
 
-// ---- prefill, MXFP4, producer/consumer workgroups ----------------------------------------------------
-// 8 waves: waves 4-7 load, waves 0-3 multiply. Per 128-column chunk the loaders bring the chunk of
-// the workgroup's 128 weight rows (8 KiB of fp4 blocks) and of the pass's NTOK token operands
-// (NTERM fp8 terms × 128 B each, XOR-swizzled by token, plus their block scales) into a
-// double-buffered LDS stage, keeping R chunks in flight in their registers; the weight rows' e8m0
-// scales for the whole K are staged once. One barrier per chunk. The MFMA waves form a 2 × 2
-// grid of 64 rows × 16·NTW tokens (4 row tiles × NTW token tiles each). Weight rows are the
-// matrix's consecutive rows: for gate_up (gate/up interleaved, ReferenceLayer.swift:11) a tile
-// holds 8 intermediates' gate and up rows, so each lane pairs gate and up in its own D fragment,
-// and a wave's 64 rows are one 32-intermediate block of the activation terms. Per output
-// element the arithmetic is the canonical one (the decode kernels' bits).
-template <int PH, int NTW>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4, 4))) void prefill_mx2(GemmArgs a) {
-  constexpr int NTERM = (PH == PH_UP) ? NTX : NTH;
-  constexpr int NTOK = 32 * NTW;            // tokens per pass
-  constexpr int MR = 128;                   // weight rows per workgroup
-  constexpr int AV = MR * 4;                // 16-byte weight vectors per chunk
-  constexpr int BV = NTERM * NTOK * 8;      // 16-byte operand vectors per chunk
-  constexpr int BS = NTERM * NTOK;          // operand scale dwords per chunk
-  constexpr int APL = AV / 256;             // per loader thread
-  constexpr int BPL = (BV + 255) / 256;
-  // Loader ring depth (chunks in flight), within the 128 registers that let two workgroups
-  // share a compute unit.
-  constexpr int R = (APL + BPL) * 4 * 3 <= 80 ? 3 : 2;
-  static_assert(AV % 256 == 0 && BS <= 256, "loader assignment");
-  __shared__ __align__(16) u32x4 sA[2][AV];
-  __shared__ __align__(16) u32x4 sB[2][BV];
-  __shared__ uint32_t sBs[2][BS];
-  __shared__ float sBias[MR];                       // bias of the workgroup's weight rows
-  extern __shared__ __align__(16) uint8_t sAS[];   // [MR][K/32] weight scales
-
-  int rt, wi;
-  prefill_tile(blockIdx.x, a.row_tiles, rt, wi);
-  if (rt >= a.row_tiles || wi >= *a.n_work) return;
-  const int4 item = a.work[wi];
-  const int e = item.x, pos0 = item.y, nitem = item.z;
-  const int gsel = (e == a.experts) ? 1 : 0;
-  const ExpertGroup &grp = a.grp[gsel];
-  const uint8_t *blob = grp.blobs + (gsel ? 0 : (size_t)e * grp.stride);
-  const int I = grp.inter, H = a.hidden;
-  const int out_dim = (PH == PH_UP) ? 2 * I : H;    // weight rows of the matrix
-  const int K = (PH == PH_UP) ? H : I;
-  const int r0 = rt * MR;
-  if (r0 >= out_dim) return;
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, l16 = lane & 15;
-  const int nch = (K + 127) / 128, nsb = K / 32;
-  const uint8_t *wblk = blob + grp.off[PH == PH_UP ? 0 : 3];
-  const uint8_t *wsc = blob + grp.off[PH == PH_UP ? 1 : 4];
-  const int ld = PH == PH_UP ? a.xld : a.hld;
-  const uint8_t *qbase = PH == PH_UP ? a.xq : a.hq;
-  const uint8_t *sbase = PH == PH_UP ? a.xs : a.hs;
-
-  // Weight scales of the valid rows (16-row granular), whole K, and the rows' biases.
-  const int vrows = min(MR, out_dim - r0);
-  for (int v = tid; v < vrows * nsb / 16; v += 512)
-    *(u32x4 *)(sAS + 16 * v) = *(const u32x4 *)(wsc + (size_t)r0 * nsb + 16 * v);
-  if (tid < MR) {
-    const uint16_t *bias = (const uint16_t *)(blob + grp.off[PH == PH_UP ? 2 : 5]);
-    sBias[tid] = a.expert_bias ? bf16_bits_to_f32(bias[min(r0 + tid, out_dim - 1)]) : 0.f;
-  }
-
-  for (int t0 = 0; t0 < nitem; t0 += NTOK) {
-    const int ntok = min(NTOK, nitem - t0);
-    auto slot_of = [&](int n) { return a.order[pos0 + t0 + min(n, ntok - 1)]; };
-    if (wave >= 4) {
-      // ---- loaders ----
-      const int lt = tid - 256;
-      const uint8_t *asrc[APL];
-      int ag[APL];
-      const uint8_t *bsrc[BPL];
-      const uint8_t *ssrc;
-#pragma unroll
-      for (int k = 0; k < APL; ++k) {
-        // Vector v = (tile j, lane i): row 16j + i%16, block g = i/16 of the chunk.
-        const int v = lt + 256 * k, j = v >> 6, i = v & 63;
-        const int r = min(r0 + 16 * j + (i & 15), out_dim - 1);
-        asrc[k] = wblk + (size_t)r * (K / 2);
-        ag[k] = i >> 4;
-      }
-#pragma unroll
-      for (int k = 0; k < BPL; ++k) {
-        const int v = min(lt + 256 * k, BV - 1);
-        const int tt = v / (NTOK * 8), sl = v % (NTOK * 8), n = sl >> 3, sg = (sl & 7) ^ (n & 7);
-        const int row = PH == PH_UP ? slot_of(n) / a.slots : slot_of(n);
-        bsrc[k] = qbase + ((size_t)row * NTERM + tt) * ld + 16 * sg;
-      }
-      {
-        const int v = min(lt, BS - 1), tt = v / NTOK, n = v % NTOK;
-        const int row = PH == PH_UP ? slot_of(n) / a.slots : slot_of(n);
-        ssrc = sbase + ((size_t)row * NTERM + tt) * (ld / 32);
-      }
-      u32x4 ra[R][APL], rb[R][BPL];
-      uint32_t rs[R];
-      auto issue = [&](int u, int c) {
-        const int cc = min(c, nch - 1);
-#pragma unroll
-        for (int k = 0; k < APL; ++k) ra[u][k] = *(const u32x4 *)(asrc[k] + 16 * min(4 * cc + ag[k], nsb - 1));
-#pragma unroll
-        for (int k = 0; k < BPL; ++k) rb[u][k] = *(const u32x4 *)(bsrc[k] + 128 * cc);
-        rs[u] = *(const uint32_t *)(ssrc + 4 * cc);
-      };
-      auto put = [&](int u, int buf) {
-#pragma unroll
-        for (int k = 0; k < APL; ++k) sA[buf][lt + 256 * k] = ra[u][k];
-#pragma unroll
-        for (int k = 0; k < BPL; ++k)
-          if (lt + 256 * k < BV) sB[buf][lt + 256 * k] = rb[u][k];
-        if (lt < BS) sBs[buf][lt] = rs[u];
-      };
-#pragma unroll
-      for (int u = 0; u < R; ++u) issue(u, u);
-      for (int c0 = 0; c0 < nch; c0 += R) {
-#pragma unroll
-        for (int u = 0; u < R; ++u) {
-          const int c = c0 + u;
-          if (c < nch) {
-            put(u, c & 1);
-            __syncthreads();
-            issue(u, c + R);
-          }
-        }
-      }
-    } else {
-      // ---- MFMA waves ----
-      const int wr = wave & 1, wt = wave >> 1;
-      const int rw = r0 + 64 * wr;              // first weight row of this wave
-      // Epilogue operands fetched now, off the critical path: slot ids and routing weights.
-      int eslot[NTW];
-      float ew[NTW];
-#pragma unroll
-      for (int st = 0; st < NTW; ++st) {
-        eslot[st] = slot_of(16 * NTW * wt + 16 * st + l16);
-        ew[st] = PH == PH_DOWN ? a.slot_w[eslot[st]] : 0.f;
-      }
-      f32x4 acc[4][NTW];
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int st = 0; st < NTW; ++st) acc[j][st] = f32x4{0.f, 0.f, 0.f, 0.f};
-      auto compute = [&](int c) {
-        const int buf = c & 1;
-        const bool ok = 128 * c + 32 * g < K;
-        u32x4 w[4];
-        uint32_t sa[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          w[j] = ok ? sA[buf][(4 * wr + j) * 64 + lane] : u32x4{0u, 0u, 0u, 0u};
-          sa[j] = sAS[(64 * wr + 16 * j + l16) * nsb + min(4 * c + g, nsb - 1)];
-        }
-#pragma unroll
-        for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-          for (int st = 0; st < NTW; ++st) {
-            const int n = 16 * NTW * wt + 16 * st + l16;
-            const int k0 = 128 * c + 16 * g;
-            u32x4 blo = sB[buf][(t * NTOK + n) * 8 + (g ^ (n & 7))];
-            u32x4 bhi = sB[buf][(t * NTOK + n) * 8 + ((4 + g) ^ (n & 7))];
-            uint32_t bs = (sBs[buf][t * NTOK + n] >> (8 * g)) & 0xFFu;
-            if (k0 >= K) blo = u32x4{0u, 0u, 0u, 0u};
-            if (k0 + 64 >= K) bhi = u32x4{0u, 0u, 0u, 0u};
-            if (!ok) bs = 127u;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc[j][st] = smfma(w[j], blo, bhi, sa[j], bs, acc[j][st]);
-          }
-      };
-      for (int c = 0; c < nch; ++c) {
-        __syncthreads();
-        compute(c);
-      }
-      // ---- epilogue ----
-      if (rw < out_dim) {
-#pragma unroll
-        for (int st = 0; st < NTW; ++st) {
-          const int n = 16 * NTW * wt + 16 * st + l16;
-          const int slot = eslot[st];
-          if constexpr (PH == PH_UP) {
-            // Tile j, lane group g: rows rw + 16j + 4g + {0..3} = (gate, up) of intermediates
-            // rw/2 + 8j + 2g + {0, 1}.
-            float v[8], gv[8], uv[8];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const f32x4 d = acc[j][st];
-              const float *bb = sBias + 64 * wr + 16 * j + 4 * g;
-              gv[2 * j] = d[0] + bb[0];
-              uv[2 * j] = d[1] + bb[1];
-              gv[2 * j + 1] = d[2] + bb[2];
-              uv[2 * j + 1] = d[3] + bb[3];
-            }
-            activate_n<8>(a.act, gv, uv, v, a.alpha, a.limit);
-            uint32_t hq[NTH][2], sb[NTH];
-            quant_block<NTH>(v, hq, sb);
-            if (n < ntok) {
-              const int i0 = rw / 2;
-#pragma unroll
-              for (int t = 0; t < NTH; ++t) {
-                uint8_t *row = a.hq + ((size_t)slot * NTH + t) * a.hld + i0 + 2 * g;
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-                  *(uint16_t *)(row + 8 * j) = (uint16_t)(hq[t][j >> 1] >> (16 * (j & 1)));
-                if (g == 0) a.hs[((size_t)slot * NTH + t) * (a.hld / 32) + i0 / 32] = (uint8_t)sb[t];
-              }
-            }
-          } else {
-            if (n < ntok) {
-              const float wgt = ew[st];
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const int h0 = rw + 16 * j + 4 * g;
-                const f32x4 r = acc[j][st];
-                const float *bb = sBias + 64 * wr + 16 * j + 4 * g;
-                f32x4 o;
-#pragma unroll
-                for (int ii = 0; ii < 4; ++ii) o[ii] = wgt * (r[ii] + bb[ii]);   // down_value's arithmetic
-                *(f32x4 *)(a.slot_out + (size_t)slot * H + h0) = o;
-              }
-            }
-          }
-        }
-      }
-    }
-    __syncthreads();   // the next pass restages the buffers
-  }
-}
-
 #ifndef HH_GEMM_KERNELS_ONLY
 // y[t][j] = Σ_r slot[t·slots + r][j] in rank order (sum_expert_slices, dense.metal:147; the
 // shared expert's slot comes last as in QwenReferenceLayer.swift:399-404).
@@ -1871,711 +1592,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const float *slot_out, int
 }
 #endif
 
-// ---- prefill, MXFP4: persistent pipeline with direct-to-LDS loads -----------------------------
-// One 512-thread workgroup per compute unit takes tasks τ = blockIdx.x, + gridDim.x, ... in
-// prefill_tile order (a task: 128 weight rows × one work item of ≤ 32 tokens). Waves 4-7 load,
-// waves 0-3 multiply (2×2: 64 rows × 16 tokens each). The loaders stream every task's 128-column
-// chunks (weight blocks, the rows' block scales, the tokens' fp8 terms and their scales) straight
-// into a ring of S LDS stages with global_load_lds, S−1 chunks ahead of the MFMA waves and across
-// task boundaries, so neither a chunk's memory latency nor a task's start is waited for. Each
-// loader wave issues at least L loads per chunk, so "the oldest chunk has landed" is the fixed wait
-// vmcnt((S−2)·L); the task switches' extra loads (work item and slot ids, fetched into LDS one and
-// two tasks ahead) only make that wait stricter. The arithmetic per output element is
-// prefill_mx2's: one chain over the chunks, the terms in order.
-// RR: 128-row halves of the weight tile (MR = 128·RR rows); TT: 32-token halves of the token tile.
-template <int PH, int RR, int TT> struct Mx3 {
-  static constexpr int NTERM = PH == PH_UP ? NTX : NTH;
-  static constexpr int NTOK = 32 * TT, MR = 128 * RR;
-  static constexpr int B_INS = NTERM * NTOK / 8;            // 1 KB operand loads per chunk
-  static constexpr int BPW = B_INS / 4;                     // per loader wave
-  static constexpr int BS_DW = NTERM * NTOK;                // operand scale dwords per chunk
-  static constexpr int L = 2 * RR + BPW + 1 + 1;            // loads per loader wave per chunk
-  static constexpr int OFF_B = 8192 * RR;                   // after 8·RR weight tiles of 1 KB
-  static constexpr int OFF_BS = OFF_B + B_INS * 1024;
-  static constexpr int OFF_SC = OFF_BS + 256 * ((BS_DW + 63) / 64);
-  static constexpr int STAGE = OFF_SC + 512 * RR;           // + MR rows × 4 block-scale bytes
-  static constexpr int S_FIT = (150 * 1024 - 1792) / STAGE;
-  static constexpr int S = S_FIT > 8 ? 8 : S_FIT;
-  static constexpr int OFF_INFO = S * STAGE;                // [3][64] work item (4 dwords used)
-  static constexpr int OFF_ORDER = OFF_INFO + 3 * 256;      // [3][64] slot ids (32 used)
-  static constexpr int OFF_JUNK = OFF_ORDER + 3 * 256;      // sink of loads no stage needs
-  static constexpr int LDS = OFF_JUNK + 256;
-  static_assert(B_INS % 4 == 0 && BS_DW <= 256 && NTOK <= 64 && S >= 3 && (S - 2) * L <= 63, "loader layout");
-};
-
-template <int PH, int RR, int TT>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_mx3(GemmArgs a) {
-  using C = Mx3<PH, RR, TT>;
-  constexpr int NTERM = C::NTERM, NTOK = C::NTOK, S = C::S, L = C::L;
-  extern __shared__ __align__(16) uint8_t lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, l16 = lane & 15;
-  const ExpertGroup &grp = a.grp[0];
-  const int I = grp.inter, H = a.hidden;
-  const int out_dim = PH == PH_UP ? 2 * I : H;
-  const int K = PH == PH_UP ? H : I;
-  const int nch = (K + 127) / 128, nsb = K / 32;
-  const int ld = PH == PH_UP ? a.xld : a.hld;
-  const uint8_t *qbase = PH == PH_UP ? a.xq : a.hq;
-  const uint8_t *sbase = PH == PH_UP ? a.xs : a.hs;
-  const int RT = a.row_tiles, rtx = (RT + 7) >> 3;
-  const int nwork = *a.n_work;
-  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, RT, nwork, a.xcd_rows);
-  // Number of chunks this workgroup computes.
-  int nsteps = 0;
-  for (int tau = tasks.first(); tau < tasks.lim; tau = tasks.next(tau)) nsteps += nch;
-  if (nsteps == 0) return;
-  uint8_t *info = lds + C::OFF_INFO, *order = lds + C::OFF_ORDER, *junk = lds + C::OFF_JUNK;
-  auto item_of = [&](int slot) { return *(const int4 *)(info + 256 * slot); };
-
-  if (wave >= 4) {
-    // ---- loaders ----
-    const int lw = wave - 4;
-    // Work item (lanes 0-3) and slot ids (lanes 0-31) of a task into its LDS slot (other lanes
-    // repeat valid entries). Every loader wave fetches them (the same values), so each one's own
-    // vmcnt tells it they have landed.
-    auto fetch_info = [&](int tau, int slot) {
-      int rt, wi;
-      tasks.tile(min(tau, tasks.lim - 1), rt, wi);
-      lds_load4((const int *)(a.work + min(wi, nwork - 1)) + min(lane, 3), info + 256 * slot);
-    };
-    auto fetch_order = [&](int slot) {
-      const int4 it = item_of(slot);
-      lds_load4(a.order + it.y + min(lane, it.z - 1), order + 256 * slot);
-    };
-    // Per-task source pointers.
-    const uint8_t *asrc[2 * RR], *bsrc[C::BPW], *bssrc, *scsrc;
-    auto start_task = [&](int tau, int slot) {
-      int rt, wi;
-      tasks.tile(tau, rt, wi);
-      const int4 it = item_of(slot);
-      const int r0 = rt * C::MR;
-      const uint8_t *blob = grp.blobs + (size_t)it.x * grp.stride;
-      const uint8_t *wblk = blob + grp.off[PH == PH_UP ? 0 : 3];
-      const uint8_t *wsc = blob + grp.off[PH == PH_UP ? 1 : 4];
-      const int *ord = (const int *)(order + 256 * slot);
-      auto row_of = [&](int n) {
-        const int sl = ord[min(n, it.z - 1)];
-        return PH == PH_UP ? sl / a.slots : sl;
-      };
-#pragma unroll
-      for (int k = 0; k < 2 * RR; ++k) {
-        const int j = 2 * RR * lw + k;   // 16-row tile of the chunk
-        asrc[k] = wblk + (size_t)min(r0 + 16 * j + l16, out_dim - 1) * (K / 2);
-      }
-#pragma unroll
-      for (int k = 0; k < C::BPW; ++k) {
-        const int v = (lw * C::BPW + k) * 64 + lane;
-        const int t = v / (NTOK * 8), sl = v % (NTOK * 8), n = sl >> 3, sg = (sl & 7) ^ (n & 7);
-        bsrc[k] = qbase + ((size_t)row_of(n) * NTERM + t) * ld + 16 * sg;
-      }
-      {
-        const int d = min(lw * 64 + lane, C::BS_DW - 1), t = d / NTOK, n = d % NTOK;
-        bssrc = sbase + ((size_t)row_of(n) * NTERM + t) * (ld / 32);
-      }
-      // Block scales: one row's 4 bytes of a chunk per lane (4-byte loads from 2-byte-aligned
-      // rows are exact; a 2-byte direct-to-LDS load would write a whole dword per lane).
-      scsrc = wsc + (size_t)min(r0 + min(lw, 2 * RR - 1) * 64 + lane, out_dim - 1) * nsb;
-    };
-    // Chunk c of the current task into stage st.
-    auto issue = [&](int c, int st) {
-      uint8_t *stg = lds + st * C::STAGE;
-#pragma unroll
-      for (int k = 0; k < 2 * RR; ++k)
-        lds_load16(asrc[k] + 16 * min(4 * c + g, nsb - 1), stg + 1024 * (2 * RR * lw + k));
-#pragma unroll
-      for (int k = 0; k < C::BPW; ++k) lds_load16(bsrc[k] + 128 * c, stg + C::OFF_B + 1024 * (lw * C::BPW + k));
-      lds_load4(bssrc + 4 * c, lw * 64 < C::BS_DW ? stg + C::OFF_BS + 256 * lw : junk);
-      lds_load4(scsrc + 4 * c, lw < 2 * RR ? stg + C::OFF_SC + 256 * lw : junk);
-    };
-    // Prologue: work items of the first two tasks and the first task's slot ids, then the first
-    // S−1 chunks.
-    int tq[3];   // task ids: issuing, next, the one after
-    tq[0] = tasks.first();
-    tq[1] = tasks.next(tq[0]);
-    tq[2] = tasks.next(tq[1]);
-    fetch_info(tq[0], 0);
-    fetch_info(tq[1], 1);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    fetch_order(0);
-    fetch_order(1);
-    fetch_info(tq[2], 2);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    int slot = 0, lc = 0;
-    start_task(tq[0], 0);
-    int q = 0;   // chunks issued
-    auto issue_next = [&]() {
-      issue(lc, q % S);
-      ++q;
-      if (++lc == nch) {
-        lc = 0;
-        // Next task: its work item and slot ids have landed (fetched ≥ one task ago).
-        tq[0] = tq[1];
-        tq[1] = tq[2];
-        tq[2] = tasks.next(tq[2]);
-        slot = slot == 2 ? 0 : slot + 1;
-        if (tq[0] < tasks.lim) {
-          start_task(tq[0], slot);
-          const int s1 = slot == 2 ? 0 : slot + 1, s2 = s1 == 2 ? 0 : s1 + 1;
-          fetch_order(s1);            // slot ids of the next task (its work item landed)
-          fetch_info(tq[2], s2);      // work item of the task after it
-        }
-      }
-    };
-    // At every barrier the chunk being computed and the next one (whose operands the MFMA waves
-    // read ahead) have landed: after issuing chunk q, wait until at most S−3 chunks' loads are
-    // outstanding.
-    for (int u = 0; u < S - 1 && q < nsteps; ++u) issue_next();
-    if (q >= S - 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 3) * L) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    for (int step = 0; step < nsteps; ++step) {
-      ring_barrier();
-      if (q < nsteps) {
-        issue_next();
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 3) * L) : "memory");
-      } else {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-    }
-    return;
-  }
-
-  // ---- MFMA waves ----
-  // Wave (wr, wt): weight rows r0 + 64·RR·wr + 16j (j < 4·RR), tokens 16·TT·wt + 16·tt + l16.
-  const int wr = wave & 1, wt = wave >> 1;
-  constexpr int NJ = 4 * RR;
-  f32x4 acc[NJ][TT];
-#pragma unroll
-  for (int j = 0; j < NJ; ++j)
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) acc[j][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int tau = tasks.first(), slot = 0, c = 0;
-  int ntok = 0, r0 = 0;
-  int eslot[TT];
-  float ew[TT];
-  uint16_t braw[NJ][4];   // bias bits of the lane's rows, loaded at the task's start, used at its end
-  auto task_begin = [&]() {
-    int rt, wi;
-    tasks.tile(tau, rt, wi);
-    const int4 it = item_of(slot);
-    r0 = rt * C::MR;
-    ntok = __builtin_amdgcn_readfirstlane(it.z);
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      eslot[tt] = ((const int *)(order + 256 * slot))[min(16 * TT * wt + 16 * tt + l16, ntok - 1)];
-      ew[tt] = PH == PH_DOWN ? a.slot_w[eslot[tt]] : 0.f;
-    }
-    // Unconditional loads (a branch on expert_bias would make the compiler wait for them here).
-    const uint16_t *bp = (const uint16_t *)(grp.blobs + (size_t)it.x * grp.stride + grp.off[PH == PH_UP ? 2 : 5]);
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int ii = 0; ii < 4; ++ii) braw[j][ii] = bp[min(r0 + 64 * RR * wr + 16 * j + 4 * g + ii, out_dim - 1)];
-  };
-  // Operands of a chunk, read from its stage one step ahead of its MFMAs (raw: the chunk's masks
-  // are applied at use).
-  struct Ops {
-    u32x4 w[NJ], blo[NTERM][TT], bhi[NTERM][TT];
-    uint32_t sa[NJ], bs[NTERM][TT];
-  };
-  auto read_ops = [&](int st) {
-    const uint8_t *stg = lds + st * C::STAGE;
-    Ops o;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      o.w[j] = *(const u32x4 *)(stg + 1024 * (NJ * wr + j) + 16 * lane);
-      o.sa[j] = stg[C::OFF_SC + 4 * (64 * RR * wr + 16 * j + l16) + g];
-    }
-    const u32x4 *sb = (const u32x4 *)(stg + C::OFF_B);
-#pragma unroll
-    for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        const int n = 16 * TT * wt + 16 * tt + l16;
-        o.blo[t][tt] = sb[(t * NTOK + n) * 8 + (g ^ (n & 7))];
-        o.bhi[t][tt] = sb[(t * NTOK + n) * 8 + ((4 + g) ^ (n & 7))];
-        o.bs[t][tt] = (((const uint32_t *)(stg + C::OFF_BS))[t * NTOK + n] >> (8 * g)) & 0xFFu;
-      }
-    return o;
-  };
-  ring_barrier();
-  Ops cur = read_ops(0);
-  for (int step = 0; step < nsteps; ++step) {
-    if (c == 0) task_begin();
-    Ops nxt;
-    if (step + 1 < nsteps) nxt = read_ops((step + 1) % S);
-    if (128 * (c + 1) <= K) {
-      // A whole chunk (every chunk but a partial last one): no lane masks.
-#pragma unroll
-      for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[j][tt] = smfma(cur.w[j], cur.blo[t][tt], cur.bhi[t][tt], cur.sa[j], cur.bs[t][tt], acc[j][tt]);
-    } else {
-      const bool ok = 128 * c + 32 * g < K;
-      const int k0 = 128 * c + 16 * g;
-#pragma unroll
-      for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-        for (int tt = 0; tt < TT; ++tt) {
-          // Lanes past K take zero weights; their scale byte may be any byte of the blob, so 2^0
-          // (the product is the same signed zero).
-          const u32x4 blo = k0 >= K ? u32x4{0u, 0u, 0u, 0u} : cur.blo[t][tt];
-          const u32x4 bhi = k0 + 64 >= K ? u32x4{0u, 0u, 0u, 0u} : cur.bhi[t][tt];
-          const uint32_t bs = ok ? cur.bs[t][tt] : 127u;
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[j][tt] = smfma(ok ? cur.w[j] : u32x4{0u, 0u, 0u, 0u}, blo, bhi, ok ? cur.sa[j] : 127u, bs, acc[j][tt]);
-        }
-    }
-    const bool more = step + 1 < nsteps;
-    if (++c < nch) {
-      if (more) ring_barrier();
-      cur = nxt;
-      continue;
-    }
-    // ---- epilogue of the task ----
-    c = 0;
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      if (16 * TT * wt + 16 * tt >= ntok) break;   // padding tiles (also wt > 0 past the tokens)
-      const int n = 16 * TT * wt + 16 * tt + l16;
-#pragma unroll
-      for (int h = 0; h < RR; ++h) {
-        const int rw = r0 + 64 * RR * wr + 64 * h;   // a 64-row block: 32 intermediates of gate-up
-        if (rw >= out_dim) continue;
-        float bias[4][4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-          for (int ii = 0; ii < 4; ++ii) bias[j][ii] = a.expert_bias ? bf16_bits_to_f32(braw[4 * h + j][ii]) : 0.f;
-        if constexpr (PH == PH_UP) {
-          float v[8], gv[8], uv[8];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const f32x4 d = acc[4 * h + j][tt];
-            gv[2 * j] = d[0] + bias[j][0];
-            uv[2 * j] = d[1] + bias[j][1];
-            gv[2 * j + 1] = d[2] + bias[j][2];
-            uv[2 * j + 1] = d[3] + bias[j][3];
-          }
-          activate_n<8>(a.act, gv, uv, v, a.alpha, a.limit);
-          uint32_t hq[NTH][2], sbq[NTH];
-          quant_block<NTH>(v, hq, sbq);
-          if (n < ntok) {
-            const int i0 = rw / 2;
-#pragma unroll
-            for (int t = 0; t < NTH; ++t) {
-              uint8_t *row = a.hq + ((size_t)eslot[tt] * NTH + t) * a.hld + i0 + 2 * g;
-#pragma unroll
-              for (int j = 0; j < 4; ++j) *(uint16_t *)(row + 8 * j) = (uint16_t)(hq[t][j >> 1] >> (16 * (j & 1)));
-              if (g == 0) a.hs[((size_t)eslot[tt] * NTH + t) * (a.hld / 32) + i0 / 32] = (uint8_t)sbq[t];
-            }
-          }
-        } else {
-          if (n < ntok) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const int h0 = rw + 16 * j + 4 * g;
-              f32x4 o;
-#pragma unroll
-              for (int ii = 0; ii < 4; ++ii) o[ii] = ew[tt] * (acc[4 * h + j][tt][ii] + bias[j][ii]);   // down_value's arithmetic
-              *(f32x4 *)(a.slot_out + (size_t)eslot[tt] * H + h0) = o;
-            }
-          }
-        }
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) acc[j][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    tau = tasks.next(tau);
-    slot = slot == 2 ? 0 : slot + 1;
-    if (more) ring_barrier();
-    cur = nxt;
-  }
-}
-
-// ---- prefill, MXFP4: weight rows in registers, token operand through an LDS ring -----------------
-// prefill_mx3's persistent task order and loader protocol, with the weight operand taken out of
-// LDS: each MFMA wave owns 64 distinct weight rows of the task's 256-row tile (one 32-intermediate
-// block of gate-up) and streams them straight into a DA-deep register ring that runs across task
-// boundaries (the wave reads the next task's work item from the loaders' LDS copy when its stream
-// crosses into it). The loaders only stage the 32 tokens' fp8 terms, their scales and the weight
-// rows' block scales, so a stage is ~9 KB and the ring holds S = 12 of them: with the weight
-// rows in the register file, about twice as many bytes are in flight per compute unit as when
-// everything passes through LDS. Per output element the arithmetic is the canonical one.
-// TT: 16-token tiles per wave (the whole token tile): 2 (32-token work items) or 4 (64).
-#ifndef HH_MXA_DA
-#define HH_MXA_DA 4
-#endif
-#ifndef HH_MXA_RA
-#define HH_MXA_RA 1
-#endif
-template <int PH, int TT_ = 2> struct MxA {   // PH_UP (down's three terms leave too few registers)
-  static constexpr int NTERM = PH == PH_UP ? NTX : NTH;
-  static constexpr int TT = TT_, NTOK = 16 * TT, MR = 256, NJ = 4;
-  // RA: an even step also reads the next step's operands (32-token items; 64-token items leave
-  // no registers for a second set). DA: the weight ring's depth in chunks.
-  static constexpr bool RA = TT == 2 && HH_MXA_RA;
-  static constexpr int DA = TT == 2 ? HH_MXA_DA : 2;
-  static constexpr int B_INS = NTERM * NTOK / 8;            // 1 KB operand loads per chunk
-  static constexpr int BPW = B_INS / 4;                     // per loader wave
-  static constexpr int BS_DW = NTERM * NTOK;                // operand scale dwords per chunk
-  static constexpr int L = BPW + 1 + 1;                     // loads per loader wave per chunk
-  static constexpr int OFF_BS = B_INS * 1024;
-  static constexpr int OFF_SC = OFF_BS + 256 * ((BS_DW + 63) / 64);
-  static constexpr int STAGE = OFF_SC + 4 * 256;            // + 256 rows × 4 block-scale bytes
-  static constexpr int S = TT == 2 ? 12 : 8;
-  static constexpr int OFF_INFO = S * STAGE;                // [3][64] work item (4 dwords used)
-  static constexpr int OFF_ORDER = OFF_INFO + 3 * 256;      // [3][64] slot ids (NTOK used)
-  static constexpr int OFF_BIAS = OFF_ORDER + 3 * 256;      // [3][256] bf16 bias of the tile's rows
-  static constexpr int OFF_JUNK = OFF_BIAS + 3 * 512;       // sink of loads no stage needs
-  static constexpr int LDS = OFF_JUNK + 256;
-  static_assert(B_INS % 4 == 0 && BS_DW <= 256 && (S - 2) * L <= 63 && DA % 2 == 0 && LDS <= 160 * 1024, "loader layout");
-};
-
-template <int PH, int TT_>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_mxa(GemmArgs a) {
-  using C = MxA<PH, TT_>;
-  constexpr int NTERM = C::NTERM, NTOK = C::NTOK, S = C::S, L = C::L, NJ = C::NJ, DA = C::DA;
-  extern __shared__ __align__(16) uint8_t lds[];
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int g = lane >> 4, l16 = lane & 15;
-  const ExpertGroup &grp = a.grp[0];
-  const int I = grp.inter, H = a.hidden;
-  const int out_dim = PH == PH_UP ? 2 * I : H;
-  const int K = PH == PH_UP ? H : I;
-  const int nch = (K + 127) / 128, nsb = K / 32;
-  const int ld = PH == PH_UP ? a.xld : a.hld;
-  const uint8_t *qbase = PH == PH_UP ? a.xq : a.hq;
-  const uint8_t *sbase = PH == PH_UP ? a.xs : a.hs;
-  const int RT = a.row_tiles, rtx = (RT + 7) >> 3;
-  const int nwork = *a.n_work;
-  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, RT, nwork, a.xcd_rows);
-  int nsteps = 0;
-  for (int tau = tasks.first(); tau < tasks.lim; tau = tasks.next(tau)) nsteps += nch;
-  if (nsteps == 0) return;
-  uint8_t *info = lds + C::OFF_INFO, *order = lds + C::OFF_ORDER, *junk = lds + C::OFF_JUNK;
-  auto item_of = [&](int slot) { return *(const int4 *)(info + 256 * slot); };
-
-  if (wave >= 4) {
-    // ---- loaders (prefill_mx3's, without the weight blocks) ----
-    const int lw = wave - 4;
-    auto fetch_info = [&](int tau, int slot) {
-      int rt, wi;
-      tasks.tile(min(tau, tasks.lim - 1), rt, wi);
-      lds_load4((const int *)(a.work + min(wi, nwork - 1)) + min(lane, 3), info + 256 * slot);
-    };
-    // Slot ids and the tile rows' bias of a task whose work item has landed.
-    auto fetch_order = [&](int tau, int slot) {
-      const int4 it = item_of(slot);
-      lds_load4(a.order + it.y + min(lane, it.z - 1), order + 256 * slot);
-      int rt, wi;
-      tasks.tile(min(tau, tasks.lim - 1), rt, wi);
-      const uint8_t *bp = grp.blobs + (size_t)it.x * grp.stride + grp.off[PH == PH_UP ? 2 : 5];
-#pragma unroll
-      for (int k = 0; k < 2; ++k)
-        lds_load4(bp + 2 * min(rt * C::MR + 2 * (64 * k + lane), out_dim - 2), lds + C::OFF_BIAS + 512 * slot + 256 * k);
-    };
-    const uint8_t *bsrc[C::BPW], *bssrc, *scsrc;
-    auto start_task = [&](int tau, int slot) {
-      int rt, wi;
-      tasks.tile(tau, rt, wi);
-      const int4 it = item_of(slot);
-      const int r0 = rt * C::MR;
-      const uint8_t *wsc = grp.blobs + (size_t)it.x * grp.stride + grp.off[PH == PH_UP ? 1 : 4];
-      const int *ord = (const int *)(order + 256 * slot);
-      auto row_of = [&](int n) {
-        const int sl = ord[min(n, it.z - 1)];
-        return PH == PH_UP ? sl / a.slots : sl;
-      };
-#pragma unroll
-      for (int k = 0; k < C::BPW; ++k) {
-        const int v = (lw * C::BPW + k) * 64 + lane;
-        const int t = v / (NTOK * 8), sl = v % (NTOK * 8), n = sl >> 3, sg = (sl & 7) ^ (n & 7);
-        bsrc[k] = qbase + ((size_t)row_of(n) * NTERM + t) * ld + 16 * sg;
-      }
-      {
-        const int d = min(lw * 64 + lane, C::BS_DW - 1), t = d / NTOK, n = d % NTOK;
-        bssrc = sbase + ((size_t)row_of(n) * NTERM + t) * (ld / 32);
-      }
-      // Block scales of rows r0 + 64·lw + lane: one row's 4 bytes of a chunk per lane.
-      scsrc = wsc + (size_t)min(r0 + lw * 64 + lane, out_dim - 1) * nsb;
-    };
-    auto issue = [&](int c, int st) {
-      uint8_t *stg = lds + st * C::STAGE;
-#pragma unroll
-      for (int k = 0; k < C::BPW; ++k) lds_load16(bsrc[k] + 128 * c, stg + 1024 * (lw * C::BPW + k));
-      lds_load4(bssrc + 4 * c, lw * 64 < C::BS_DW ? stg + C::OFF_BS + 256 * lw : junk);
-      lds_load4(scsrc + 4 * c, stg + C::OFF_SC + 256 * lw);
-    };
-    int tq[3];
-    tq[0] = tasks.first();
-    tq[1] = tasks.next(tq[0]);
-    tq[2] = tasks.next(tq[1]);
-    fetch_info(tq[0], 0);
-    fetch_info(tq[1], 1);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    fetch_order(tq[0], 0);
-    fetch_order(tq[1], 1);
-    fetch_info(tq[2], 2);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    int slot = 0, lc = 0;
-    start_task(tq[0], 0);
-    int q = 0;
-    auto issue_next = [&]() {
-      issue(lc, q % S);
-      ++q;
-      if (++lc == nch) {
-        lc = 0;
-        tq[0] = tq[1];
-        tq[1] = tq[2];
-        tq[2] = tasks.next(tq[2]);
-        slot = slot == 2 ? 0 : slot + 1;
-        if (tq[0] < tasks.lim) {
-          start_task(tq[0], slot);
-          const int s1 = slot == 2 ? 0 : slot + 1, s2 = s1 == 2 ? 0 : s1 + 1;
-          fetch_order(tq[1], s1);
-          fetch_info(tq[2], s2);
-        }
-      }
-    };
-    // One barrier per two chunks: at barrier k chunks 2k and 2k+1 have landed; after it the
-    // slots of chunks 2k−2 and 2k−1 (computed before it) take chunks 2k+S−2 and 2k+S−1.
-    for (int u = 0; u < S - 2 && q < nsteps; ++u) issue_next();
-    if (q >= S - 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 4) * L) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    const int nbar = (nsteps + 1) / 2;
-    for (int k = 0; k < nbar; ++k) {
-      ring_barrier();
-      if (q + 2 <= nsteps) {
-        issue_next();
-        issue_next();
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 4) * L) : "memory");
-      } else {
-        while (q < nsteps) issue_next();
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      }
-    }
-    return;
-  }
-
-  // ---- MFMA waves: rows 64·wave .. +63 of the tile (NJ = 4 tiles of 16), every token ----
-  constexpr int TT = C::TT;
-  f32x4 acc[NJ][TT];
-#pragma unroll
-  for (int j = 0; j < NJ; ++j)
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) acc[j][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // Weight stream: chunk qa (of this workgroup's flat chunk sequence) of the load task.
-  int la_tau = tasks.first(), la_slot = 0, la_c = 0;
-  const uint8_t *arow[NJ];
-  auto la_rows = [&]() {
-    int rt, wi;
-    tasks.tile(la_tau, rt, wi);
-    const int4 it = item_of(la_slot);
-    const uint8_t *wblk = grp.blobs + (size_t)it.x * grp.stride + grp.off[PH == PH_UP ? 0 : 3];
-#pragma unroll
-    for (int j = 0; j < NJ; ++j)
-      arow[j] = wblk + (size_t)min(rt * C::MR + 64 * wave + 16 * j + l16, out_dim - 1) * (K / 2);
-  };
-  u32x4 ar[DA][NJ];
-  // Unconditional: past the last task the stream re-reads the last task's rows (never used). A
-  // load under a branch becomes a copy at the merge, which waits for the data: the ring would be
-  // one chunk deep.
-  auto load_a = [&](u32x4 (&dst)[NJ]) {
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) dst[j] = *(const u32x4 *)(arow[j] + 16 * min(4 * la_c + g, nsb - 1));
-    if (la_tau >= tasks.lim) return;
-    if (++la_c == nch) {
-      la_c = 0;
-      la_tau = tasks.next(la_tau);
-      la_slot = la_slot == 2 ? 0 : la_slot + 1;
-      if (la_tau < tasks.lim) la_rows();
-    }
-  };
-  int tau = tasks.first(), slot = 0, c = 0;
-  int ntok = 0, r0 = 0;
-  int eslot[TT];
-  float ew[TT];
-  auto task_begin = [&]() {
-    int rt, wi;
-    tasks.tile(tau, rt, wi);
-    const int4 it = item_of(slot);
-    r0 = rt * C::MR;
-    ntok = __builtin_amdgcn_readfirstlane(it.z);
-#pragma unroll
-    for (int tt = 0; tt < TT; ++tt) {
-      eslot[tt] = ((const int *)(order + 256 * slot))[min(16 * tt + l16, ntok - 1)];
-      ew[tt] = PH == PH_DOWN ? a.slot_w[eslot[tt]] : 0.f;
-    }
-  };
-  struct Ops {
-    u32x4 blo[NTERM][TT], bhi[NTERM][TT];
-    uint32_t sa[NJ], bs[NTERM][TT];
-  };
-  auto read_ops = [&](int st) {
-    const uint8_t *stg = lds + st * C::STAGE;
-    Ops o;
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) o.sa[j] = stg[C::OFF_SC + 4 * (64 * wave + 16 * j + l16) + g];
-    const u32x4 *sb = (const u32x4 *)stg;
-#pragma unroll
-    for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        const int n = 16 * tt + l16;
-        o.blo[t][tt] = sb[(t * NTOK + n) * 8 + (g ^ (n & 7))];
-        o.bhi[t][tt] = sb[(t * NTOK + n) * 8 + ((4 + g) ^ (n & 7))];
-        o.bs[t][tt] = (((const uint32_t *)(stg + C::OFF_BS))[t * NTOK + n] >> (8 * g)) & 0xFFu;
-      }
-    return o;
-  };
-  ring_barrier();   // the loaders' first task copies have landed
-  la_rows();
-#pragma unroll
-  for (int u = 0; u < DA; ++u) load_a(ar[u]);
-  bool done = false;
-  // Barrier k lands chunks 2k and 2k + 1: with RA an even step reads its own operands and the
-  // next (odd) step's, whose LDS latency then passes under the even step's MFMAs. DA is even and
-  // k0 a multiple of DA, so the parity of `step` is that of the unrolled copy u.
-  Ops nx;
-  for (int k0 = 0; !done; k0 += DA) {
-#pragma unroll
-    for (int u = 0; u < DA; ++u) {
-      const int step = k0 + u;
-      if (PH == PH_UP) HH_TRS(step, 0);
-      if (c == 0) task_begin();
-      Ops cur;
-      if (C::RA && (u & 1)) {
-        cur = nx;
-      } else {
-        cur = read_ops(step % S);
-        if (C::RA) nx = read_ops((step + 1) % S);   // past the last step: a stage no step reads
-      }
-#ifdef HH_TRACE_STEPS
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#endif
-      if (PH == PH_UP) HH_TRS(step, 1);
-      const bool more = step + 1 < nsteps;
-      if (128 * (c + 1) > K) {
-        // A partial last chunk: lanes past K take zero weights and operand terms; their scale
-        // bytes may be any bytes, so 2^0 (the product is the same signed zero). Masked in place.
-        const bool ok = 128 * c + 32 * g < K;
-        const int kk = 128 * c + 16 * g;
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) {
-          if (!ok) ar[u][j] = u32x4{0u, 0u, 0u, 0u};
-          if (!ok) cur.sa[j] = 127u;
-        }
-#pragma unroll
-        for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-          for (int tt = 0; tt < TT; ++tt) {
-            if (kk >= K) cur.blo[t][tt] = u32x4{0u, 0u, 0u, 0u};
-            if (kk + 64 >= K) cur.bhi[t][tt] = u32x4{0u, 0u, 0u, 0u};
-            if (!ok) cur.bs[t][tt] = 127u;
-          }
-      }
-      // Token tiles wholly past the item's tokens (padding) are skipped: never stored.
-#pragma unroll
-      for (int tt = 0; tt < TT; ++tt) {
-        if (tt > 0 && 16 * tt >= ntok) break;
-#pragma unroll
-        for (int t = 0; t < NTERM; ++t)
-#pragma unroll
-          for (int j = 0; j < NJ; ++j)
-            acc[j][tt] = smfma(ar[u][j], cur.blo[t][tt], cur.bhi[t][tt], cur.sa[j], cur.bs[t][tt], acc[j][tt]);
-      }
-      if (PH == PH_UP) HH_TRS(step, 2);
-      load_a(ar[u]);   // the chunk DA ahead into the slot just consumed
-      if (PH == PH_UP) HH_TRS(step, 3);
-      if (++c == nch) {
-        // ---- epilogue of the task ----
-        c = 0;
-        const int rw = r0 + 64 * wave;   // a 64-row block: 32 intermediates of gate-up
-        if (rw < out_dim) {
-          // The tile rows' bias from the task's LDS copy (rows past out_dim: another row's, never
-          // stored).
-          const uint8_t *bl = lds + C::OFF_BIAS + 512 * slot;
-          float bias[NJ][4];
-#pragma unroll
-          for (int j = 0; j < NJ; ++j) {
-            const u32x2 bw = *(const u32x2 *)(bl + 2 * (64 * wave + 16 * j + 4 * g));
-#pragma unroll
-            for (int ii = 0; ii < 4; ++ii)
-              bias[j][ii] = a.expert_bias ? bf16_bits_to_f32((bw[ii >> 1] >> (16 * (ii & 1))) & 0xFFFFu) : 0.f;
-          }
-#pragma unroll
-          for (int tt = 0; tt < TT; ++tt) {
-            if (16 * tt >= ntok) break;   // padding tiles
-            const int n = 16 * tt + l16;
-            if constexpr (PH == PH_UP) {
-              float v[8], gv[8], uv[8];
-#pragma unroll
-              for (int j = 0; j < 4; ++j) {
-                const f32x4 d = acc[j][tt];
-                gv[2 * j] = d[0] + bias[j][0];
-                uv[2 * j] = d[1] + bias[j][1];
-                gv[2 * j + 1] = d[2] + bias[j][2];
-                uv[2 * j + 1] = d[3] + bias[j][3];
-              }
-              activate_n<8>(a.act, gv, uv, v, a.alpha, a.limit);
-              uint32_t hq[NTH][2], sbq[NTH];
-              quant_block<NTH>(v, hq, sbq);
-              // Each lane's 8 contiguous bytes of every term (one store each).
-              uint32_t he[NTH][2];
-#pragma unroll
-              for (int t = 0; t < NTH; ++t) transpose_pieces(hq[t][0], hq[t][1], g, he[t][0], he[t][1]);
-              if (n < ntok) {
-                const int i0 = rw / 2;
-#pragma unroll
-                for (int t = 0; t < NTH; ++t) {
-                  uint8_t *row = a.hq + ((size_t)eslot[tt] * NTH + t) * a.hld + i0;
-                  *(u32x2 *)(row + 8 * g) = u32x2{he[t][0], he[t][1]};
-                  if (g == 0) a.hs[((size_t)eslot[tt] * NTH + t) * (a.hld / 32) + i0 / 32] = (uint8_t)sbq[t];
-                }
-              }
-            } else {
-              if (n < ntok) {
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                  const int h0 = rw + 16 * j + 4 * g;
-                  f32x4 o;
-#pragma unroll
-                  for (int ii = 0; ii < 4; ++ii) o[ii] = ew[tt] * (acc[j][tt][ii] + bias[j][ii]);   // down_value's arithmetic
-                  *(f32x4 *)(a.slot_out + (size_t)eslot[tt] * H + h0) = o;
-                }
-              }
-            }
-          }
-        }
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-          for (int tt = 0; tt < TT; ++tt) acc[j][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-        tau = tasks.next(tau);
-        slot = slot == 2 ? 0 : slot + 1;
-      }
-      if (!more) {
-        done = true;
-        break;
-      }
-      if (PH == PH_UP) HH_TRS(step, 4);
-      if (step & 1) ring_barrier();   // one barrier per two chunks
-      if (PH == PH_UP) HH_TRS(step, 5);
-    }
-  }
-}
-
 // ---- launch table -----------------------------------------------------------------------------
-typedef void (*GemmKernel)(GemmArgs);
 typedef void (*UpSmallKernel)(GemmArgs, RouteArgs, FuseArgs);
 typedef void (*DownSmallKernel)(GemmArgs, const int32_t *);
 
@@ -2640,106 +1657,6 @@ template <int FMT> static DownSmallKernel down_small_k(int slots, bool one, bool
 static bool mlx_staged_up(int hidden) { return hidden <= 64 * kMlxSbChunks; }
 static bool mlx_staged_down(int slots, int imax) {
   return imax <= 64 * (slots > 4 ? mlx_sb_chunks_down<kMaxTopK + 1>() : mlx_sb_chunks_down<4>());
-}
-
-// Output rows per prefill_mx2 workgroup: 64 intermediates of the interleaved gate_up matrix, or 128
-// hidden rows.
-int gemm_rows_per_block(int quant, int phase) {
-  (void)quant;
-  return phase == PH_UP ? 64 : 128;
-}
-
-static int device_cus() {
-  static int ncu = 0;
-  if (!ncu) {
-    int dev = 0;
-    (void)hipGetDevice(&dev);
-    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 8) ncu = 256;
-    ncu &= ~7;   // prefill_tile's order assumes 8 | gridDim for persistent grids
-  }
-  return ncu;
-}
-
-// Whether prefill_mx3 takes a phase: MXFP4 without a shared expert, work items of 32 tokens, and
-// rows of at least S chunks (task switches are prefetched one task ahead inside the chunk ring).
-// Gate-up over batches of 64 or more work items takes 256-row tiles (twice the products per staged
-// byte); down, and smaller batches, 128-row tiles (down's deeper ring measured faster).
-template <int PH, int RR, int TT> static bool mx3_fits(const GemmArgs &a) {
-  const int K = PH == PH_UP ? a.hidden : a.grp[0].inter;
-  return (K + 127) / 128 >= Mx3<PH, RR, TT>::S;
-}
-static bool mx3_wide(int phase, const GemmArgs &a) { return a.max_work >= 64; }
-static bool use_mx3(int phase, const GemmArgs &a, int nt) {
-  if (a.slots != a.top_k || nt != 2) return false;
-  if (!mx3_wide(phase, a)) return phase == PH_UP ? mx3_fits<PH_UP, 1, 1>(a) : mx3_fits<PH_DOWN, 1, 1>(a);
-  return phase == PH_UP ? mx3_fits<PH_UP, 2, 1>(a) : mx3_fits<PH_DOWN, 2, 1>(a);
-}
-
-template <int PH, int RR, int TT> static hipError_t launch_mx3(GemmArgs a, hipStream_t s, Timing tm) {
-  static std::once_flag once;
-  std::call_once(once, [] {
-    (void)hipFuncSetAttribute((const void *)prefill_mx3<PH, RR, TT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    (void)hipGetLastError();
-  });
-  // Row tiles of this variant: MR weight rows (MR / 2 intermediates of the interleaved gate_up).
-  constexpr int rows = PH == PH_UP ? Mx3<PH, RR, TT>::MR / 2 : Mx3<PH, RR, TT>::MR;
-  a.row_tiles = ((PH == PH_UP ? a.ldh : a.hidden) + rows - 1) / rows;
-  hipExtLaunchKernelGGL(prefill_mx3<PH, RR, TT>, dim3(device_cus()), dim3(512), Mx3<PH, RR, TT>::LDS, s, tm.start,
-                        tm.stop, 0, a);
-  return hipGetLastError();
-}
-
-// Whether prefill_mxa takes a phase: gate-up of MXFP4 layers without a shared expert, 32-token
-// work items in batches of 64 or more, or 64-token ones; rows of at least S chunks (a wave's
-// weight stream reads the next task's copy, which the loaders rewrite S chunks later). Down's three
-// operand terms leave too few registers for the weight ring.
-static bool use_mxa(int phase, const GemmArgs &a, int nt) {
-  if (phase != PH_UP || a.slots != a.top_k) return false;
-  if (nt == 2) return a.max_work >= 64 && (a.hidden + 127) / 128 >= MxA<PH_UP, 2>::S;
-  return nt == 4 && (a.hidden + 127) / 128 >= MxA<PH_UP, 4>::S;
-}
-
-template <int PH, int TT> static hipError_t launch_mxa(GemmArgs a, hipStream_t s, Timing tm) {
-  static std::once_flag once;
-  std::call_once(once, [] {
-    (void)hipFuncSetAttribute((const void *)prefill_mxa<PH, TT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                              160 * 1024);
-    (void)hipGetLastError();
-  });
-  constexpr int rows = PH == PH_UP ? MxA<PH, TT>::MR / 2 : MxA<PH, TT>::MR;
-  a.row_tiles = ((PH == PH_UP ? a.ldh : a.hidden) + rows - 1) / rows;
-  hipExtLaunchKernelGGL(prefill_mxa<PH, TT>, dim3(device_cus()), dim3(512), MxA<PH, TT>::LDS, s, tm.start, tm.stop, 0,
-                        a);
-  return hipGetLastError();
-}
-
-hipError_t launch_prefill(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm);   // hh_prefill.hip
-
-hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &args, hipStream_t s, Timing tm) {
-  if (quant != Q_MXFP4) return launch_prefill(phase, quant, nt, args, s, tm);
-  // Persistent kernels: XCD split into row-tile parts × work-item parts (Mx3Tasks): MXFP4 within
-  // ±2 % of 8 row-tile parts (its down fetches 18 % fewer bytes with 4).
-  GemmArgs a = args;
-  a.xcd_rows = 4;
-  if (use_mxa(phase, a, nt))
-    return nt == 2 ? launch_mxa<PH_UP, 2>(a, s, tm) : launch_mxa<PH_UP, 4>(a, s, tm);
-  if (nt == 4 && phase == PH_DOWN && a.slots == a.top_k &&
-      (a.grp[0].inter + 127) / 128 >= Mx3<PH_DOWN, 1, 2>::S)
-    return launch_mx3<PH_DOWN, 1, 2>(a, s, tm);
-  if (use_mx3(phase, a, nt)) {
-    if (!mx3_wide(phase, a)) return phase == PH_UP ? launch_mx3<PH_UP, 1, 1>(a, s, tm) : launch_mx3<PH_DOWN, 1, 1>(a, s, tm);
-    return phase == PH_UP ? launch_mx3<PH_UP, 2, 1>(a, s, tm) : launch_mx3<PH_DOWN, 2, 1>(a, s, tm);
-  }
-  // prefill_tile: 8 XCDs × ⌈row_tiles / 8⌉ row tiles × work items.
-  const unsigned blocks = 8u * (unsigned)((a.row_tiles + 7) / 8) * (unsigned)a.max_work;
-  if (blocks == 0) return hipSuccess;
-  // 8 waves, the weight rows' scales (128 rows × K/32 bytes) in dynamic LDS.
-  const size_t lds = (size_t)128 * ((phase == PH_UP ? a.hidden : a.ldh) / 32);
-  GemmKernel k = phase == PH_UP ? (nt <= 2 ? prefill_mx2<PH_UP, 1> : prefill_mx2<PH_UP, 2>)
-                                : (nt <= 2 ? prefill_mx2<PH_DOWN, 1> : prefill_mx2<PH_DOWN, 2>);
-  hipExtLaunchKernelGGL(k, dim3(blocks), dim3(512), lds, s, tm.start, tm.stop, 0, a);
-  return hipGetLastError();
 }
 
 hipError_t launch_down_small(int quant, GemmArgs a, const int32_t *topk_idx, int T, hipStream_t s,

@@ -418,50 +418,28 @@ __device__ __forceinline__ f32x4 smfma(const u32x4 &a, const u32x4 &blo, const u
   return __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(av, bv, c, 4, 0, 0, (int)sa, 0, (int)sb);
 }
 
-// Workgroup barrier without __syncthreads' release fence: the fence would make every wave wait for
-// all of its direct-to-LDS loads (vmcnt(0)) before the barrier; the pipeline orders LDS itself
-// with explicit waits. A compiler memory barrier keeps LDS accesses on their side.
-__device__ __forceinline__ void ring_barrier() { asm volatile("s_barrier" ::: "memory"); }
-
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
-__device__ __forceinline__ void lds_load16(const void *g, uint8_t *l) {
-  __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)l, 16, 0, 0);
-}
-__device__ __forceinline__ void lds_load4(const void *g, uint8_t *l) {
-  __builtin_amdgcn_global_load_lds(g, (lds_ptr_t)l, 4, 0, 0);
-}
 
-// Task ids of one workgroup of a persistent prefill kernel: τ = b, b + G, ... (G a multiple of
-// 8, so τ mod 8 is the workgroup's XCD), skipping tasks past the row tiles or the work items.
-// The 8 XCDs form P row-tile parts × 8/P work-item parts: XCD x takes row tiles of part x mod P
-// and work items of part x / P, work item by work item (each item's row tiles consecutively).
-// An expert's slice of weight rows stays in the XCD's L2 across the expert's consecutive items,
-// and an item's operand rows are fetched by the P XCDs of its item part.
-struct Mx3Tasks {
-  int b, G, RT, nwork, P, rtp, nq, lim;
-  __device__ __forceinline__ Mx3Tasks(int b_, int G_, int RT_, int nwork_, int P_)
-      : b(b_), G(G_), RT(RT_), nwork(nwork_), P(P_ == 1 || P_ == 2 || P_ == 4 ? P_ : 8) {
-    rtp = (RT + P - 1) / P;
-    nq = (nwork + 8 / P - 1) / (8 / P);
-    lim = 8 * rtp * nq;
-  }
-  __device__ __forceinline__ void tile(int tau, int &rt, int &wi) const {
+// Tasks of a prefill launch: task τ, on XCD τ mod 8 (workgroups go to the XCDs in turn), is a row tile
+// and a work item, or nothing past the row tiles or the items. The 8 XCDs form P row-tile parts ×
+// 8/P work-item parts: XCD x takes row tiles of part x mod P and work items of part x / P, work item
+// by work item (each item's row tiles consecutively). An expert's slice of weight rows stays in
+// the XCD's L2 across the expert's consecutive items, and an item's operand rows are fetched by
+// the P XCDs of its item part.
+struct PrefillTasks {
+  int RT, nwork, P, rtp, nq, lim;
+  __device__ __forceinline__ PrefillTasks(int RT_, int nwork_, int P_)
+      : RT(RT_), nwork(nwork_), P(P_), rtp((RT_ + P_ - 1) / P_), nq((nwork_ + 8 / P_ - 1) / (8 / P_)), lim(8 * rtp * nq) {}
+  __device__ __forceinline__ bool tile(int tau, int &rt, int &wi) const {
+    if (tau >= lim) return false;
     const int x = tau & 7, j = tau >> 3, q = j / rtp;
     rt = (x & (P - 1)) * rtp + (j - q * rtp);
     wi = (x / P) * nq + q;
-  }
-  __device__ __forceinline__ int first() const { return fix(b); }
-  __device__ __forceinline__ int next(int tau) const { return fix(tau + G); }
-  __device__ __forceinline__ int fix(int tau) const {
-    for (; tau < lim; tau += G) {
-      int rt, wi;
-      tile(tau, rt, wi);
-      if (rt < RT && wi < nwork) return tau;
-    }
-    return lim;
+    return rt < RT && wi < nwork;
   }
 };
 
+// At most N of the wave's loads outstanding.
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
 }  // namespace hh

@@ -7,6 +7,8 @@
 
 namespace hh {
 
+constexpr int kRowParts = 2;   // row-tile parts of the XCDs (PrefillTasks)
+
 // 16 bytes per lane from global memory straight into LDS: base (uniform) + off (per lane) to LDS
 // byte `l` + 16·lane. Written in assembly so that the compiler does not order the wave's own LDS
 // reads after its loads in flight (it would wait for all of them); the kernels wait with wait_vm.
@@ -43,7 +45,7 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // of 128 bytes. The XOR of the 16-byte segments by the row keeps the MFMA lanes' LDS reads at full rate.
 // The output tiles' arithmetic is the canonical one (chunk_mfma, prefill equals decode bit for bit).
 //
-// XCD order (Mx3Tasks): two row-tile parts × four item parts, so an item's token rows reach two
+// XCD order (PrefillTasks): two row-tile parts × four item parts, so an item's token rows reach two
 // XCDs' L2: BF16 T = 2048 gate-up 430 us with four parts, 349 with two, 359 with one.
 
 // ---- BF16 -----------------------------------------------------------------------------------------
@@ -83,11 +85,8 @@ __global__ __launch_bounds__(256 * WT_) __attribute__((amdgpu_waves_per_eu(2, 2)
   const int wave = uniform(threadIdx.x >> 6), wr = wave & 3, wt = wave >> 2;
   const int H = a.hidden, E = a.experts;
   const int nwork = *a.n_work;
-  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, a.row_tiles, nwork, a.xcd_rows);
-  if ((int)blockIdx.x >= tasks.lim) return;
   int rt, wi;
-  tasks.tile((int)blockIdx.x, rt, wi);
-  if (rt >= a.row_tiles || wi >= nwork) return;
+  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.max_work + (int)blockIdx.x, rt, wi)) return;
   const int4 it = a.work[wi];
   const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
   const ExpertGroup &grp = a.grp[e == E ? 1 : 0];
@@ -249,11 +248,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int wave = uniform(threadIdx.x >> 6);
   const int H = a.hidden, E = a.experts;
   const int nwork = *a.n_work;
-  const Mx3Tasks tasks((int)blockIdx.x, (int)gridDim.x, a.row_tiles, nwork, a.xcd_rows);
-  if ((int)blockIdx.x >= tasks.lim) return;
   int rt, wi;
-  tasks.tile((int)blockIdx.x, rt, wi);
-  if (rt >= a.row_tiles || wi >= nwork) return;
+  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.max_work + (int)blockIdx.x, rt, wi)) return;
   const int4 it = a.work[wi];
   const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
   const ExpertGroup &grp = a.grp[e == E ? 1 : 0];
@@ -454,47 +450,290 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
 }
 
-template <int PH, int BITS, int RT, int NT> static hipError_t launch_mlx(GemmArgs a, hipStream_t s, Timing tm) {
-  using C = Ml<PH, BITS, RT, NT>;
-  static std::once_flag once;
-  std::call_once(once, [] {
-    (void)hipFuncSetAttribute((const void *)prefill_mlx<PH, BITS, RT, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
-    (void)hipGetLastError();
-  });
-  const int rows = PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
-  a.row_tiles = (rows + C::ROWS - 1) / C::ROWS;
-  a.xcd_rows = 2;
-  const int P = a.xcd_rows;
-  const unsigned blocks = 8u * (unsigned)((a.row_tiles + P - 1) / P) * (unsigned)((a.max_work + 8 / P - 1) / (8 / P));
-  if (blocks == 0) return hipSuccess;
-  hipExtLaunchKernelGGL((prefill_mlx<PH, BITS, RT, NT>), dim3(blocks), dim3(256), C::LDS, s, tm.start, tm.stop, 0, a);
-  return hipGetLastError();
+// ---- MXFP4 ----------------------------------------------------------------------------------------
+// A stage is 128 columns: 16-row weight tiles of 64 bytes a row (one MFMA's K), the token rows' fp8
+// terms, and, every third stage, the scales of three stages. A wave owns 64 weight rows (32
+// intermediates of gate-up, gate and up rows interleaved) and all the item's tokens.
+// What bounds it: the weight rows' arrival. Without weight traffic the T = 2048 gate-up takes 305 of its
+// 411 us (and 224 without its MFMAs, 360 without its epilogue), so three things keep more of them in flight or
+// make them cheaper, on the 128-expert layer (H = I = 2880, Zipf load; gate-up / down us):
+//   - scales 16 bytes a row every three stages instead of 4 every stage (a row's scales lie 90
+//     bytes from the next row's, so every lane of such a load takes a cache line of its own): T = 2048
+//     447 / 312 -> 413 / 283, T = 512 212 / 135 -> 193 / 124;
+//   - a stage's weight tiles are private to a wave, which reloads their slot as soon as they are in
+//     its registers: two stages in flight from two slots, T = 512 193 / 124 -> 183 / 116;
+//   - two workgroups per compute unit: eight waves sharing a 64- or 128-token operand tile 514-540 at T = 2048.
+// Before (persistent kernels with loader waves): T = 2048 483 / 368, T = 512 222 / 148, and 102 / 55 at
+// T = 45 of the 32-expert layer, now 405 / 279, 183 / 116 and 92 / 49.
+// Gate-up items hold 64 tokens where experts average 16 or more (T = 2048 405, with 32 tokens 480;
+// T = 512 183 against 199), down items 32 (three terms: a 64-token stage leaves one slot).
+template <int PH, int NT_> struct Mx {
+  static constexpr int NT = NT_, NTERM = PH == PH_UP ? NTX : NTH;
+  static constexpr int NJ = 4;                               // 16-row tiles per wave, their 1 KiB loads per stage
+  static constexpr int ROWS = 256, TOK = 16 * NT;            // weight rows, tokens of a work item
+  static constexpr int B_INS = NTERM * TOK / 8, BPW = (B_INS + 3) / 4;   // 1 KiB operand loads per stage
+  static constexpr int BR = NTERM * TOK, BSL = (BR + 63) / 64;           // operand rows; loads of their scales
+  static constexpr int OFF_B = 16 * 1024;
+  static constexpr int STAGE = OFF_B + B_INS * 1024;
+  // Scales of three stages: 16 bytes of each weight row, then of each operand row; two such sets.
+  static constexpr int OFF_Q = 2 * STAGE, QB = 4096, QUAD = QB + BSL * 1024;
+  static constexpr int LDS = OFF_Q + 2 * QUAD;
+  static_assert(BSL <= 4 && LDS <= 80 * 1024, "two workgroups per compute unit");
+};
+
+template <int PH, int NT_>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_mx(GemmArgs a) {
+  using C = Mx<PH, NT_>;
+  constexpr int NT = C::NT, NTERM = C::NTERM, NJ = C::NJ, TOK = C::TOK;
+  extern __shared__ __align__(16) uint8_t lds[];
+  const int lane = threadIdx.x & 63, g = lane >> 4, l16 = lane & 15;
+  const int wave = uniform(threadIdx.x >> 6);
+  const int H = a.hidden;
+  const int nwork = *a.n_work;
+  int rt, wi;
+  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.max_work + (int)blockIdx.x, rt, wi)) return;
+  const int4 it = a.work[wi];
+  const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
+  const ExpertGroup &grp = a.grp[e == a.experts ? 1 : 0];
+  const uint8_t *blob = grp.blobs + (e == a.experts ? 0 : (size_t)e * grp.stride);
+  const int I = grp.inter;
+  const int K = PH == PH_UP ? H : I, out_dim = PH == PH_UP ? 2 * I : H;
+  const int nsb = K / 32, n = (K + 127) / 128;   // blocks of a row; stages
+  const int ld = PH == PH_UP ? a.xld : a.hld;
+  const uint8_t *qbase = PH == PH_UP ? a.xq : a.hq, *sbase = PH == PH_UP ? a.xs : a.hs;
+  if (rt * C::ROWS >= out_dim) return;
+  const int rw = rt * C::ROWS + 64 * wave;   // the wave's first row
+  const bool active = rw < out_dim;
+  const bool part = (K & 127) != 0;   // the last stage holds 64 columns
+  const bool last_rows = rw + 64 >= out_dim;   // holds the rows within 16 bytes of the scales' end
+
+  const int rowb = K / 2;
+  const int lr = lane >> 2, seg = (lane & 3) ^ ((lr >> 1) & 3);
+  const uint32_t aoff = (uint32_t)(lr * rowb + 16 * seg);
+  const uint32_t aoff_t = part ? (uint32_t)(lr * rowb + 16 * (seg & 1)) : aoff;   // lanes past K repeat the half before it
+  const uint8_t *abase[NJ];
+#pragma unroll
+  for (int i = 0; i < NJ; ++i) {
+    const int r0 = min(rw + 16 * i, out_dim - 16);
+    abase[i] = blob + grp.off[PH == PH_UP ? 0 : 3] + (size_t)r0 * rowb;
+  }
+  // Block scales of row rw + lane: 16 bytes from the dword that holds a stage's
+  // first, which covers three stages; moved back where they would pass the matrix's last byte.
+  const uint8_t *sbase_w = blob + grp.off[PH == PH_UP ? 1 : 4];
+  const int srow = min(rw + lane, out_dim - 1), sc_end = out_dim * nsb - 16;
+  const int ntok = (cnt + 15) & ~15;   // operand rows past the last used token tile are not loaded
+  const uint8_t *bsrc[C::BPW];
+  bool bon[C::BPW];
+#pragma unroll
+  for (int i = 0; i < C::BPW; ++i) {
+    const int j = (wave * C::BPW + i) % C::B_INS, r = 8 * j + (lane >> 3), t = r / TOK, tn = r % TOK;
+    bon[i] = (8 * j) % TOK < ntok;
+    const int sl = a.order[pos + min(tn, cnt - 1)];
+    bsrc[i] = qbase + ((size_t)(PH == PH_UP ? sl / a.slots : sl) * NTERM + t) * ld + 16 * ((lane & 7) ^ (tn & 7));
+  }
+  const uint8_t *bssrc;
+  {
+    const int d = min(min(wave, C::BSL - 1) * 64 + lane, C::BR - 1), t = d / TOK, tn = d % TOK;
+    const int sl = a.order[pos + min(tn, cnt - 1)];
+    bssrc = sbase + ((size_t)(PH == PH_UP ? sl / a.slots : sl) * NTERM + t) * (ld / 32);
+  }
+  int es[NT];
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) es[tt] = a.order[pos + min(16 * tt + l16, cnt - 1)];
+
+  const uint32_t l0 = lds_addr(lds);
+  int q = 0, qs = 0, q3 = 0, qset = 0;   // stages issued, its ring slot, stage mod 3, scale set
+  auto issue = [&]() {
+    const uint32_t st = l0 + (uint32_t)(qs * C::STAGE);
+    if (q3 == 0) {
+      const uint32_t qd = l0 + C::OFF_Q + qset * C::QUAD;
+      dma16(sbase_w + min((srow * nsb + 4 * q) & ~3, sc_end), qd + 1024 * wave);
+      if (wave < C::BSL) dma16(bssrc + 4 * q, qd + C::QB + 1024 * wave);
+      qset ^= 1;
+    }
+    q3 = q3 == 2 ? 0 : q3 + 1;
+#pragma unroll
+    for (int i = 0; i < C::BPW; ++i)
+      if (bon[i]) dma16(bsrc[i] + 128 * q, st + C::OFF_B + 1024 * ((wave * C::BPW + i) % C::B_INS));
+    ++q;
+    qs ^= 1;
+  };
+  // Weight tiles of stage s (the wave's own: only it reads them) into slot s & 1.
+  auto issue_a = [&](int s) {
+    const uint32_t ao = part && s == n - 1 ? aoff_t : aoff;
+#pragma unroll
+    for (int i = 0; i < NJ; ++i) dma16(abase[i] + 64 * s, ao, l0 + (s & 1) * C::STAGE + 1024 * (wave * NJ + i));
+  };
+  issue_a(0);
+  issue();
+  if (n > 1) issue_a(1);
+
+  f32x4 acc[NJ][NT];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) acc[j][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const int aro = 4096 * wave + 64 * l16 + 16 * (g ^ ((l16 >> 1) & 3));
+  const int bro = C::OFF_B + 128 * l16 + 16 * (g ^ (l16 & 7));   // the high half: ^ 64
+  const int sro = C::OFF_Q + 16 * (64 * wave + l16) + g + (((rw + l16) * nsb) & 3), bso = C::OFF_Q + C::QB + 16 * l16 + g;
+  int ss = 0, s3 = 0, sset = 0;
+#pragma unroll 1
+  for (int s = 0; s < n; ++s) {
+    // Stage s has landed; the weight tiles of stage s + 1, issued after it, may be in flight.
+    if (s + 1 < n) wait_vm<NJ>();
+    else wait_vm<0>();
+    step_barrier();
+    if (q < n) issue();
+    const uint8_t *stg = lds + ss * C::STAGE;
+    ss ^= 1;
+    const uint8_t *qd = lds + sset * C::QUAD + 4 * s3;   // this stage's scales in its set
+    const int sc0 = 4 * (s - s3);
+    s3 = s3 == 2 ? 0 : s3 + 1;
+    if (s3 == 0) sset ^= 1;
+    u32x4 w[NJ];
+    uint32_t sa[NJ];
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      w[j] = *(const u32x4 *)(stg + aro + 1024 * j);
+      int back = 0;   // how far the row's 16 bytes were moved back
+      if (last_rows) back = max(0, (((rw + 16 * j + l16) * nsb + sc0) & ~3) - sc_end);
+      sa[j] = qd[sro + 256 * j + back];
+    }
+    // The wave's weight tiles are in registers: their slot takes the stage after the next, two
+    // steps ahead of its use.
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if (s + 2 < n) issue_a(s + 2);
+    if (!active) continue;
+    const bool tail = part && s == n - 1;
+    // Lanes past K take zero weights and operand terms with scales 2^0 (whatever bytes they read).
+    const bool ok = !tail || g < 2;
+    if (tail) {
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        if (!ok) w[j] = u32x4{0u, 0u, 0u, 0u};
+        if (!ok) sa[j] = 127u;
+      }
+    }
+#pragma unroll
+    for (int tt = 0; tt < NT; ++tt) {
+      if (tt > 0 && 16 * tt >= cnt) break;   // token tiles wholly past the item
+#pragma unroll
+      for (int t = 0; t < NTERM; ++t) {
+        const u32x4 blo = *(const u32x4 *)(stg + bro + 128 * (TOK * t + 16 * tt));
+        u32x4 bhi = *(const u32x4 *)(stg + (bro ^ 64) + 128 * (TOK * t + 16 * tt));
+        uint32_t bs = qd[bso + 16 * (TOK * t + 16 * tt)];
+        if (tail) {
+          bhi = u32x4{0u, 0u, 0u, 0u};
+          if (!ok) bs = 127u;
+        }
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[j][tt] = smfma(w[j], blo, bhi, sa[j], bs, acc[j][tt]);
+      }
+    }
+  }
+  if (!active) return;
+  float bias[NJ][4];
+#pragma unroll
+  for (int j = 0; j < NJ; ++j)
+#pragma unroll
+    for (int ii = 0; ii < 4; ++ii) bias[j][ii] = 0.f;
+  if (a.expert_bias) {
+    const uint16_t *bp = (const uint16_t *)(blob + grp.off[PH == PH_UP ? 2 : 5]) + rw + 4 * g;
+#pragma unroll
+    for (int j = 0; j < NJ; ++j) {
+      const u32x2 bw = *(const u32x2 *)(bp + 16 * j);
+#pragma unroll
+      for (int ii = 0; ii < 4; ++ii) bias[j][ii] = bf16_bits_to_f32((bw[ii >> 1] >> (16 * (ii & 1))) & 0xFFFFu);
+    }
+  }
+#pragma unroll
+  for (int tt = 0; tt < NT; ++tt) {
+    if (16 * tt >= cnt) break;
+    const bool in = 16 * tt + l16 < cnt;
+    if constexpr (PH == PH_UP) {
+      float v[8], gv[8], uv[8];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 d = acc[j][tt];
+        gv[2 * j] = d[0] + bias[j][0];
+        uv[2 * j] = d[1] + bias[j][1];
+        gv[2 * j + 1] = d[2] + bias[j][2];
+        uv[2 * j + 1] = d[3] + bias[j][3];
+      }
+      activate_n<8>(a.act, gv, uv, v, a.alpha, a.limit);
+      uint32_t hq[NTH][2], sbq[NTH], he[NTH][2];
+      quant_block<NTH>(v, hq, sbq);
+      // Each lane's 8 contiguous bytes of every term (one store each).
+#pragma unroll
+      for (int t = 0; t < NTH; ++t) transpose_pieces(hq[t][0], hq[t][1], g, he[t][0], he[t][1]);
+      if (in) {
+        const int i0 = rw / 2;
+#pragma unroll
+        for (int t = 0; t < NTH; ++t) {
+          *(u32x2 *)(a.hq + ((size_t)es[tt] * NTH + t) * a.hld + i0 + 8 * g) = u32x2{he[t][0], he[t][1]};
+          if (g == 0) a.hs[((size_t)es[tt] * NTH + t) * (a.hld / 32) + i0 / 32] = (uint8_t)sbq[t];
+        }
+      }
+    } else if (in) {
+      const float ew = a.slot_w[es[tt]];
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        f32x4 o;
+#pragma unroll
+        for (int ii = 0; ii < 4; ++ii) o[ii] = ew * (acc[j][tt][ii] + bias[j][ii]);   // down_value's arithmetic
+        *(f32x4 *)(a.slot_out + (size_t)es[tt] * H + rw + 16 * j + 4 * g) = o;
+      }
+    }
+  }
 }
 
-template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(GemmArgs a, hipStream_t s, Timing tm) {
-  using C = Bf<PH, NT, RT, SV, WT>;
-  static std::once_flag once;
-  std::call_once(once, [] {
-    (void)hipFuncSetAttribute((const void *)prefill_bf16<PH, NT, RT, SV, WT>, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
+// One workgroup per task; launches of at most 2^22 workgroups (a launch's threads are counted in 32
+// bits), each told its first task in max_work.
+template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int threads, int rows, GemmArgs a, hipStream_t s,
+                                                  Timing tm, std::once_flag &once) {
+  std::call_once(once, [&] {
+    (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
     (void)hipGetLastError();
   });
-  const int rows = PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
   a.row_tiles = (rows + C::ROWS - 1) / C::ROWS;
-  a.xcd_rows = 2;
-  const int P = a.xcd_rows;
-  const unsigned blocks = 8u * (unsigned)((a.row_tiles + P - 1) / P) * (unsigned)((a.max_work + 8 / P - 1) / (8 / P));
-  if (blocks == 0) return hipSuccess;
-  hipExtLaunchKernelGGL((prefill_bf16<PH, NT, RT, SV, WT>), dim3(blocks), dim3(256 * WT), C::LDS, s, tm.start, tm.stop, 0, a);
-  return hipGetLastError();
+  constexpr int P = kRowParts;
+  const int64_t tasks = 8ll * ((a.row_tiles + P - 1) / P) * ((a.max_work + 8 / P - 1) / (8 / P));
+  constexpr int64_t most = 1ll << 22;
+  for (int64_t t0 = 0; t0 < tasks; t0 += most) {
+    a.max_work = (int32_t)t0;
+    hipExtLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, tasks - t0)), dim3(threads), C::LDS, s,
+                          t0 == 0 ? tm.start : nullptr, t0 + most >= tasks ? tm.stop : nullptr, 0, a);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+  }
+  return hipSuccess;
+}
+template <int PH> static int out_rows(const GemmArgs &a) {
+  return PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
+}
+template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(const GemmArgs &a, hipStream_t s, Timing tm) {
+  static std::once_flag once;
+  return launch_tasks<Bf<PH, NT, RT, SV, WT>>(prefill_bf16<PH, NT, RT, SV, WT>, 256 * WT, out_rows<PH>(a), a, s, tm, once);
+}
+template <int PH, int BITS, int RT, int NT> static hipError_t launch_mlx(const GemmArgs &a, hipStream_t s, Timing tm) {
+  static std::once_flag once;
+  return launch_tasks<Ml<PH, BITS, RT, NT>>(prefill_mlx<PH, BITS, RT, NT>, 256, out_rows<PH>(a), a, s, tm, once);
+}
+template <int PH, int NT> static hipError_t launch_mx(const GemmArgs &a, hipStream_t s, Timing tm) {
+  static std::once_flag once;
+  return launch_tasks<Mx<PH, NT>>(prefill_mx<PH, NT>, 256, (PH == PH_UP ? 2 : 1) * out_rows<PH>(a), a, s, tm, once);
 }
 
 // The tile of each call. BF16 work items hold 160 tokens (nt 10: experts averaging 40 tokens or
-// more) or 32; the MLX formats' always 32.
-hipError_t launch_prefill(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
+// more) or 32, MXFP4 gate-up items 64 (nt 4) or 32, all others 32.
+hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
   const bool up = phase == PH_UP;
   if (quant == Q_MLX4) return up ? launch_mlx<PH_UP, 4, 2, 2>(a, s, tm) : launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
   if (quant == Q_MLX8) return up ? launch_mlx<PH_UP, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
-  if (quant != Q_BF16) return hipErrorInvalidValue;
+  if (quant == Q_MXFP4) {
+    if (up) return nt == 4 ? launch_mx<PH_UP, 4>(a, s, tm) : launch_mx<PH_UP, 2>(a, s, tm);
+    return launch_mx<PH_DOWN, 2>(a, s, tm);
+  }
   if (nt == 10) return up ? launch_bf16<PH_UP, 5, 2, 2, 2>(a, s, tm) : launch_bf16<PH_DOWN, 5, 4, 2, 2>(a, s, tm);
   return up ? launch_bf16<PH_UP, 2, 1, 2, 1>(a, s, tm) : launch_bf16<PH_DOWN, 2, 2, 2, 1>(a, s, tm);
 }

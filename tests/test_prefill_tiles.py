@@ -11,8 +11,10 @@ from hydra_amd import formats as F
 from hydra_amd import synth
 
 REL = 2e-5
+REL_MX = 1.3e-4   # MXFP4: activations as three fp8 terms, 2^-13 of a value
 
 BF16 = F.GEMMA_BF16.replace(experts=3, top_k=2)
+MX = F.GPT_OSS_20B.replace(experts=3, top_k=2)
 MLX4 = F.QWEN_35B_A3B_Q4.replace(experts=3, top_k=2)
 CASES = {
     # name: (desc, tokens); 2T/3 tokens an expert
@@ -24,6 +26,10 @@ CASES = {
     "mlx4_odd_groups": (MLX4.replace(hidden=320, intermediate=192, shared_intermediate=320), 100),
     "mlx4_even_groups": (MLX4.replace(hidden=640, intermediate=384, shared_intermediate=0), 49),
     "mlx8_one_group": (MLX4.replace(quant=F.QUANT_MLX8, hidden=64, intermediate=64, shared_intermediate=0), 50),
+    "mx_half_stage": (MX.replace(hidden=64, intermediate=64), 17),           # one stage of 64 columns
+    "mx_ragged": (MX.replace(hidden=192, intermediate=320), 60),             # 40 an expert: two items of 32
+    "mx_64": (MX.replace(hidden=1088, intermediate=1024, experts=2, top_k=1), 150),   # 64-token gate-up items
+    "mx_shared": (MX.replace(hidden=448, intermediate=192, shared_intermediate=320, expert_bias=0), 90),
     "mlx8_odd_groups": (MLX4.replace(quant=F.QUANT_MLX8, hidden=448, intermediate=320, shared_intermediate=192), 70),
 }
 
@@ -41,7 +47,7 @@ def test_prefill_tiles(name):
     y, idx, _ = (t.cpu().numpy() for t in L.forward(x))
     ry, ridx, _, _ = O.moe_forward(layer, x, nthreads=8)
     assert np.array_equal(idx, ridx)
-    assert np.linalg.norm(y - ry) / np.linalg.norm(ry) < REL
+    assert np.linalg.norm(y - ry) / np.linalg.norm(ry) < (REL_MX if desc.quant == F.QUANT_MXFP4 else REL)
     for t in (0, T // 2, T - 1):
         y1 = L.forward(x[t:t + 1])[0].cpu().numpy()[0]
         assert np.array_equal(y1.view(np.uint32), y[t].view(np.uint32))
