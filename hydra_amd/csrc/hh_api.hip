@@ -154,26 +154,42 @@ struct Scratch {
   int slots, positions, ldh, max_work, tile_tokens, nt;
   int max_work_half;
   bool half_down;
+  bool products;   // the prefill products (grouped by expert) rather than the decode kernels
   int xld, hld;   // MXFP4: row lengths of the fp8 operand terms (multiples of 512)
 };
 
-constexpr int kSmallT = 16;  // batches up to this size take the decode kernels
+constexpr int kSmallT = 16;  // batches up to this size take the decode kernels, or (mid_tokens) the prefill products
 
-int token_tile_nt(const hh_moe_desc &d, int T) {
-  // Prefill work items of 16·nt tokens: MXFP4 32 or 64 (below), BF16 160 once experts
-  // average 40 tokens or more (the weight tile is then read once per 160 tokens), else 32.
-  if (d.quant == HH_QUANT_BF16 && (int64_t)T * d.top_k >= 40 * (int64_t)d.experts) return 10;
-  // MXFP4 without a shared expert, experts averaging 16 or more tokens (rows below 1024 columns: not
-  // measured): 64-token items for the gate-up (an expert's rows are read once per 64 tokens); the
-  // down product runs the same segments as 32-token items (Scratch::half_down).
-  if (d.quant == HH_QUANT_MXFP4 && d.shared_intermediate == 0 && (int64_t)T * d.top_k >= 16 * (int64_t)d.experts &&
-      d.hidden >= 1024 && d.intermediate >= 1024)
-    return 4;
-  return 2;
+// Smallest batch of at most kSmallT tokens that takes the prefill products after the decode router's logits. The
+// decode kernels read an expert's rows for each of its row tiles' workgroups with all the batch's
+// tokens staged, and down once per token; the products read them once for the expert's tokens, but
+// need a selection and dispatch launch (11 us) and a combine (4 us). Whole layer, decode kernels / products, us:
+// BF16 (H 2816, 128 experts) T = 4 101 / 101, T = 5 122 / 109, T = 8 164 / 142, T = 16 307 / 207; MLX 4-bit
+// (H 2048, 256 experts) T = 4 52 / 55, T = 5 69 / 57, T = 8 95 / 67, T = 16 198 / 96; 8-bit T = 5 75 / 65,
+// T = 16 206 / 115. MXFP4 (H 2880): T = 8 91 / 132, T = 16 148 / 147, so never.
+int mid_tokens(const hh_moe_desc &d) { return d.quant == HH_QUANT_MXFP4 ? kSmallT + 1 : 5; }
+
+// Experts must average this many tokens for the larger work items of a format (0: it has none).
+int large_item_tokens(const hh_moe_desc &d) {
+  if (d.quant == HH_QUANT_BF16) return 40;
+  if (d.quant == HH_QUANT_MXFP4 && d.shared_intermediate == 0 && d.hidden >= 1024 && d.intermediate >= 1024) return 16;
+  return 0;
 }
 
-Scratch plan(const hh_moe_desc &d, int T) {
+int token_tile_nt(const hh_moe_desc &d, int T) {
+  // Prefill work items of 16·nt tokens: 32, or where experts average enough tokens BF16 160 (the
+  // weight tile is then read once per 160 tokens), MXFP4 64 for the gate-up (without a shared expert;
+  // rows below 1024 columns: not measured), whose down product runs the same segments as 32-token items
+  // (Scratch::half_down).
+  const int avg = large_item_tokens(d);
+  if (!avg || (int64_t)T * d.top_k < (int64_t)avg * d.experts) return 2;
+  return d.quant == HH_QUANT_BF16 ? 10 : 4;
+}
+
+// `decode`: batches of at most kSmallT tokens take the decode kernels whatever mid_tokens says.
+Scratch plan(const hh_moe_desc &d, int T, bool decode = false) {
   Scratch s{};
+  s.products = T > kSmallT || (!decode && T >= mid_tokens(d));
   const int E = d.experts, K = d.top_k, H = d.hidden;
   const bool shared = d.shared_intermediate > 0;
   s.slots = K + (shared ? 1 : 0);
@@ -218,12 +234,19 @@ Scratch plan(const hh_moe_desc &d, int T) {
   s.hs = take(mx ? (size_t)s.positions * hh::NTH * (s.hld / 32) : 0);
   // Above 16 tokens the slot outputs are written only after routing, so an MLX router's fp64
   // logits [T][E+1] share their region.
-  s.slot_out = take(T > kSmallT ? std::max(sizeof(float) * (size_t)T * s.slots * H,
-                                           sizeof(double) * (size_t)T * (E + 1))
-                                : 0);
+  s.slot_out = take(s.products ? std::max(sizeof(float) * (size_t)T * s.slots * H,
+                                          sizeof(double) * (size_t)T * (E + 1))
+                               : 0);
   s.status = take(sizeof(uint32_t));
   s.total = c;
   return s;
+}
+
+// The largest batch up to T whose work items are the small ones (T where that is none): its plan, of
+// more items, can exceed that of a larger batch.
+int below_large_items(const hh_moe_desc &d, int T) {
+  const int64_t last = ((int64_t)large_item_tokens(d) * d.experts + d.top_k - 1) / d.top_k - 1;
+  return last < 1 ? T : (int)std::min<int64_t>(T, last);
 }
 
 int ensure_arena(hh_ctx *ctx, size_t bytes) {
@@ -334,7 +357,7 @@ hh::RouteArgs route_args(const hh_moe_desc &d, const hh_moe_weights *w, uint8_t 
   r.slots = s.slots;
   r.router = d.router;
   r.tile_tokens = s.tile_tokens;
-  r.want_dispatch = 1;
+  r.want_dispatch = s.products && T <= kSmallT ? 2 : 1;
   r.eps = d.router_eps;
   r.logits = nullptr;
   r.lg64 = (double *)(base + (T > kSmallT && w && w->router_bits ? s.slot_out : s.lg64));
@@ -513,7 +536,7 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
   g.hs = base + s.hs;
   g.hld = s.hld;
 
-  if (!noalloc && !resid && w->router_bits == 0 && use_fused(ctx, *d, T)) {
+  if (!s.products && !noalloc && !resid && w->router_bits == 0 && use_fused(ctx, *d, T)) {
     // Decode in one launch (decode_mx): logits and h terms in the arena, flags in the
     // context's flag buffer.
     if ((rc = ensure_flags(ctx))) return rc;
@@ -541,7 +564,7 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
   // call's flag epoch, and not for the allocation-free entry, which owns no flag buffer). In the
   // FFN block (bin) those workgroups, and the gate-up workgroups' x terms, form x from the
   // residual rows themselves.
-  const bool fr = T <= kSmallT && !noalloc && (!resid || bin) && !ctx->capturing && w->router_bits == 0 &&
+  const bool fr = !s.products && !noalloc && (!resid || bin) && !ctx->capturing && w->router_bits == 0 &&
                   decode_mode(ctx) == 2 && hh::fused_router_fits(d->quant, d->hidden, d->experts, d->router, T) &&
                   sizeof(uint32_t) * (size_t)hh::fused_router_flags(T, d->experts) <= kFlagBytes;
   if (fr) {
@@ -554,7 +577,7 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
     HH_HIP(hh::launch_route(r, ctx->stream, tm));
   }
 
-  if (T <= kSmallT) {
+  if (!s.products) {
     // Decode: exact logits → gate-up (selects the top-k itself) → down with the rank-ordered
     // combine in its epilogue.
     hh::Timing tm_down, tm_comb;
@@ -590,7 +613,7 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
   }
   if ((rc = phase_timing(ctx, &tm, noalloc))) return rc;
   HH_HIP(hh::launch_combine(g.slot_out, s.slots, d->hidden, T, y, resid, ctx->stream, tm));
-  ctx->dispatches += 6;   // route logits, select, dispatch, gate-up, down, combine
+  ctx->dispatches += T <= kSmallT ? 5 : 6;   // route logits, select, dispatch (one launch up to kSmallT), gate-up, down, combine
   return HH_OK;
 }
 
@@ -732,12 +755,8 @@ int hh_ctx_reserve(hh_ctx *ctx, const hh_moe_desc *d, int32_t max_tokens) {
   int rc = check_desc(d);
   if (rc) return rc;
   if (max_tokens <= 0 || max_tokens > kMaxTokens) return fail(HH_EINVAL, "max_tokens outside 1..65536");
-  // The plan for a batch that switches to 64-token tiles can be smaller than for a batch just
-  // below the switch; reserve the larger of the two.
   size_t need = 0;
-  // Plans just below a token-tile switch can exceed the one for max_tokens.
-  for (int t : {max_tokens, std::min(max_tokens, 63), std::min(max_tokens, 127)})
-    need = std::max(need, plan(*d, t).total);
+  for (int t : {max_tokens, below_large_items(*d, max_tokens)}) need = std::max(need, plan(*d, t).total);
   return ensure_arena(ctx, need);
 }
 
@@ -807,7 +826,8 @@ int hh_moe_forward_noalloc(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weigh
   if (rc) return rc;
   if (T == 0) return HH_OK;
   if (!ctx->scratch) return fail(HH_EHIP, "static scratch unavailable: " + ctx->scratch_error);
-  const Scratch s = plan(*d, T);
+  Scratch s = plan(*d, T);
+  if (s.total > HH_NOALLOC_SCRATCH_BYTES && T <= kSmallT) s = plan(*d, T, true);   // no slot outputs
   if (s.total > HH_NOALLOC_SCRATCH_BYTES)
     return fail(HH_ENOMEM, "the call needs " + std::to_string(s.total) +
                                " bytes of scratch; the allocation-free entry point has " +
@@ -1231,7 +1251,7 @@ int hh_runner_reserve(hh_runner *r, int32_t max_tokens) {
   for (const hh_runner::Layer &L : r->layers) {
     if (!L.set) return fail(HH_EINVAL, "a layer of the runner is not set");
     const bool gemma = L.norms.post_expert_norm != nullptr;
-    for (int t : {max_tokens, std::min(max_tokens, 63), std::min(max_tokens, 127)})
+    for (int t : {max_tokens, below_large_items(L.desc, max_tokens)})
       need = std::max(need, block_plan(L.desc, plan(L.desc, t), t, gemma).total);
   }
   return ensure_arena(r->ctx, need);

@@ -807,6 +807,34 @@ __global__ __launch_bounds__(1024) void dispatch_kernel(RouteArgs a) {
   dispatch_batch<16>(a, a.topk_idx);
 }
 
+// Selection and dispatch of a batch of at most 16 tokens, from the exact logits, for the layer's products of
+// hh_prefill.hip: wave t selects token t's experts, then workgroup 0 groups the batch's assignments
+// while workgroup 1, which has selected the same, forms their weights.
+__global__ __launch_bounds__(1024) void select_dispatch_kernel(RouteArgs a) {
+  warm_kernargs<sizeof(RouteArgs)>();
+  __shared__ int s_idx[16 * kMaxTopK];
+  __shared__ int s_ri[16][kMaxTopK];
+  __shared__ double s_rv[16][kMaxTopK];
+  __shared__ int s_ci[16][kFastCand];
+  __shared__ double s_cv[16][kFastCand];
+  const int t = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  if (t < a.tokens) {
+    const double *lg = a.lg64 + (size_t)t * (a.experts + 1);
+    TopK tk = topk_fast(lg, a.experts, a.top_k, s_ri[t], s_rv[t], s_ci[t], s_cv[t]);
+    prob_order(tk, a.top_k, a.router);
+    if (blockIdx.x == 1) {
+      finish_token(a, t, tk, a.shared_gate ? lg[a.experts] : 0.0);
+    } else {
+#pragma unroll
+      for (int r = 0; r < kMaxTopK; ++r)
+        if (lane == r && r < a.top_k) s_idx[t * a.top_k + r] = tk.i[r];
+    }
+  }
+  if (blockIdx.x == 1) return;
+  __syncthreads();
+  dispatch_batch<16>(a, s_idx);
+}
+
 // Batches above 16 tokens: one wave per 16 blocks of a token.
 __global__ __launch_bounds__(256) void quant_x_kernel(RouteArgs a) {
   const int w = blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -1365,7 +1393,7 @@ hipError_t launch_route_mlx(const RouteArgs &a, hipStream_t s, Timing tm) {
   }
   const int R = small ? 1 : MLX_RT_R;
   const int blocks = (small ? 1 : (a.tokens + MLX_RT_TILE - 1) / MLX_RT_TILE) * (((rows + R - 1) / R + 3) / 4);
-  const bool sel = !small || a.want_dispatch == 0;
+  const bool sel = !small || a.want_dispatch != 1;
   const bool disp = !small && a.want_dispatch != 0;
   const bool quant = a.xq != nullptr;
   void *kern = a.router_bits == 8 ? (small ? mlx_logits_fn<8, 1>(a.hidden) : mlx_logits_fn<8, MLX_RT_R>(a.hidden))
@@ -1386,6 +1414,10 @@ hipError_t launch_route_mlx(const RouteArgs &a, hipStream_t s, Timing tm) {
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   if (!sel) return hipSuccess;
+  if (small && a.want_dispatch) {
+    hipExtLaunchKernelGGL(select_dispatch_kernel, dim3(2), dim3(1024), 0, s, nullptr, tm.stop, 0, a);
+    return hipGetLastError();
+  }
   hipExtLaunchKernelGGL(select_lg64_kernel, dim3((a.tokens + 3) / 4), dim3(256), 0, s, nullptr,
                         disp ? nullptr : tm.stop, 0, a);
   if ((e = hipGetLastError()) != hipSuccess || !disp) return e;
@@ -1397,10 +1429,10 @@ namespace hh {
 hipError_t launch_route(const RouteArgs &a, hipStream_t s, Timing tm) {
   if (a.router_bits) return launch_route_mlx(a, s, tm);
   if (a.tokens <= RT_TOK) {
-    // The layer (want_dispatch) selects inside its gate-up kernel; the operator entry selects
-    // here.
+    // The layer's decode path (want_dispatch 1) selects inside its gate-up kernel; the operator entry
+    // (0) and a batch for the prefill products (2) select here.
     const int qwaves = a.xq ? a.tokens * ((a.hidden / 32 + 15) / 16) : 0;
-    const bool sel = a.want_dispatch == 0;
+    const bool sel = a.want_dispatch != 1;
     const bool g = a.router == R_GEMMA;
     if (a.resid) {
       // The FFN block's router (the caller admits only bf16 non-GEMMA routers, H ≤ 4096).
@@ -1423,7 +1455,10 @@ hipError_t launch_route(const RouteArgs &a, hipStream_t s, Timing tm) {
     }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || !sel) return e;
-    hipExtLaunchKernelGGL(select_small_kernel, dim3(1), dim3(256), 0, s, nullptr, tm.stop, 0, a);
+    if (a.want_dispatch)
+      hipExtLaunchKernelGGL(select_dispatch_kernel, dim3(2), dim3(1024), 0, s, nullptr, tm.stop, 0, a);
+    else
+      hipExtLaunchKernelGGL(select_small_kernel, dim3(1), dim3(256), 0, s, nullptr, tm.stop, 0, a);
     return hipGetLastError();
   }
   const int ttiles = (a.tokens + RT_TOK - 1) / RT_TOK;

@@ -1,6 +1,6 @@
-"""The prefill products (T > 16) at the edges of their tiles: row tiles past the last row, a last
+"""The expert products of hh_prefill.hip at the edges of their tiles: row tiles past the last row, a last
 stage of one step or one group, token tiles past an item's tokens, experts of more than one work
-item, both item sizes. Against the fp64 oracle, and bit for bit against one-token calls.
+item, both item sizes, batches of at most 16 tokens. Against the fp64 oracle, and bit for bit against one-token calls.
 
 Bound: activations travel as a bf16 hi + lo pair (2^-17 of the value each), fp32 sums over at most a
 few hundred columns add less, so rel-L2 stays below 2e-5."""
@@ -18,6 +18,10 @@ MX = F.GPT_OSS_20B.replace(experts=3, top_k=2)
 MLX4 = F.QWEN_35B_A3B_Q4.replace(experts=3, top_k=2)
 CASES = {
     # name: (desc, tokens); 2T/3 tokens an expert
+    "bf16_decode_5": (BF16.replace(hidden=192, intermediate=320), 5),     # smallest batch of these products
+    "bf16_decode_16": (BF16.replace(hidden=832, intermediate=192, shared_intermediate=128), 16),
+    "mlx8_decode_16": (MLX4.replace(quant=F.QUANT_MLX8, hidden=448, intermediate=320, shared_intermediate=192), 16),
+    "mlx4_decode_7": (MLX4.replace(hidden=320, intermediate=192, shared_intermediate=0, experts=300, top_k=8), 7),
     "bf16_32_small": (BF16.replace(hidden=64, intermediate=64), 17),      # one stage
     "bf16_32_ragged": (BF16.replace(hidden=192, intermediate=320), 59),   # 39 an expert: two items of 32
     "bf16_160_edge": (BF16.replace(hidden=192, intermediate=320), 60),    # 40 an expert: items of 160
