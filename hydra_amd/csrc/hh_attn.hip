@@ -20,7 +20,7 @@
 //            column reads out).
 // The waves' states merge in LDS and the workgroup writes an unnormalised partial (max, sum,
 // head_dim sums) per (query head, chunk); attn_merge_kernel combines the chunks of a head in
-// chunk order. As in the reference, every partial starts from the sink as its running maximum
+// a fixed order. As in the reference, every partial starts from the sink as its running maximum
 // and only chunk 0's wave 0 gives the sink its weight, so an empty chunk stays finite.
 #include "hh_common.hpp"
 
@@ -59,38 +59,25 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// One tile per wave up to 32768 keys (1024 workgroups), so the kernel is a chain of latencies: the
+// tile's rows are asked for first and the queries' fragments are formed, straight from global
+// memory, while they travel; the waves' outputs merge in the LDS that staged their values. Whole call, 64 / 8
+// heads of 64, before -> now: 32768 keys 21.1 -> 18.4 us (3.7 TB/s), 131072 68.6 -> 66.3, 4096 8.6 ->
+// 8.4; heads of 128, 32768 keys 52.9 -> 45.8. Three waves per SIMD: with two (205 registers) 19.8 at 32768 keys,
+// with four (128 registers, 29 spilled) 23.6.
 template <int D>
-__global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
+__global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_split_kernel(AttnArgs a) {
   warm_kernargs<sizeof(AttnArgs)>();
   constexpr int QM = kAttnQM, DG = D / 8, JG = 64 / DG, KPL = 64 / JG, NDC = D / 32, NN = D / 16;
   constexpr int VST = D + 4;   // halves per staged value row: rows 4 keys apart land 8 banks apart
-  __shared__ __align__(16) float s_q[QM][D];
-  __shared__ __align__(16) _Float16 s_v[4][64 * VST];
+  __shared__ __align__(16) _Float16 s_v[4][64 * VST];   // a wave's value tile, at the end its QM × D outputs
   __shared__ float s_m[4][QM], s_l[4][QM];
-  __shared__ float s_acc[4][QM][D];
+  static_assert(sizeof(float) * QM * D <= sizeof(_Float16) * 64 * VST, "outputs fit the tile");
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, l16 = lane & 15;
   const int kvh = blockIdx.x % a.kvh, chunk = blockIdx.x / a.kvh;
   const int qm = a.qh / a.kvh;
   const int h0 = kvh * qm;
-  for (int i = tid; i < QM * D; i += 256) {
-    const int h = i / D, c = i - h * D;
-    s_q[h][c] = h < qm ? a.q[(size_t)(h0 + h) * D + c] * a.scale : 0.f;
-  }
-  __syncthreads();
-  // The scaled queries as the B operand of the QK^T MFMAs: lane (g, l16) holds head l16's
-  // dimensions 32·dc + 8g .. +7 as an fp16 pair hi + lo (the fp32 value to ~2^-22 relative;
-  // each product with an fp16 key is exact in fp32); zero for heads ≥ qm.
-  f16x8 qhi[NDC], qlo[NDC];
-#pragma unroll
-  for (int dc = 0; dc < NDC; ++dc)
-#pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const float x = l16 < QM ? s_q[l16][32 * dc + 8 * g + e] : 0.f;
-      const _Float16 hi = (_Float16)x;
-      qhi[dc][e] = hi;
-      qlo[dc][e] = (_Float16)(x - (float)hi);
-    }
   const int first = chunk * a.per_chunk;
   const int last = min(first + a.per_chunk, a.keys);
   // Running maximum and denominator of head l16 (every lane group holds the same values).
@@ -107,12 +94,12 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
   };
   const int jg = lane / DG, dg = lane - jg * DG;
   _Float16 *sv = s_v[wave];
-  for (int base = first + 64 * wave; base < last; base += 256) {
+  f16x8 kr[4][NDC], vr[KPL];
+  auto load_tile = [&](int base) {
     // The tile's key rows (16-key subtile st, lane (g, l16): key base + 16·st + l16, dimensions
     // 32·dc + 8g .. +7) and value rows (lane (jg, dg): keys jg·KPL .. +KPL−1, dimensions
     // 8·dg .. +7) are all issued before any arithmetic: one memory latency per tile. Rows past
     // the chunk read row `first` (in bounds) and are masked (their probabilities are zero).
-    f16x8 kr[4][NDC], vr[KPL];
 #pragma unroll
     for (int st = 0; st < 4; ++st) {
       const int key = base + 16 * st + l16;
@@ -125,6 +112,26 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
       const int j = base + jg * KPL + i;
       vr[i] = *(const f16x8 *)(a.v + row_of(j < last ? j : first) * row_stride + (size_t)kvh * D + 8 * dg);
     }
+  };
+  int base = first + 64 * wave;
+  if (base < last) load_tile(base);
+  // The scaled queries as the B operand of the QK^T MFMAs: lane (g, l16) holds head l16's
+  // dimensions 32·dc + 8g .. +7 as an fp16 pair hi + lo (the fp32 value to ~2^-22 relative;
+  // each product with an fp16 key is exact in fp32); zero for heads ≥ qm.
+  f16x8 qhi[NDC], qlo[NDC];
+#pragma unroll
+  for (int dc = 0; dc < NDC; ++dc) {
+    const f32x4 *qp = (const f32x4 *)(a.q + (size_t)(h0 + min(l16, qm - 1)) * D + 32 * dc + 8 * g);
+    const f32x4 q0 = qp[0], q1 = qp[1];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = l16 < qm ? (e < 4 ? q0[e & 3] : q1[e & 3]) * a.scale : 0.f;
+      const _Float16 hi = (_Float16)x;
+      qhi[dc][e] = hi;
+      qlo[dc][e] = (_Float16)(x - (float)hi);
+    }
+  }
+  while (base < last) {
     // Phase 1: S = K·q^T on the fp16 MFMA; sc[st][i] is the logit of key base + 16·st + 4g + i
     // for head l16.
     f32x4 sc[4];
@@ -194,8 +201,11 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
         acc[n] = __builtin_amdgcn_mfma_f32_16x16x32_f16(plo[kc], vb, acc[n], 0, 0, 0);
       }
     __builtin_amdgcn_wave_barrier();   // the staged rows are rewritten by the next tile
+    base += 256;
+    if (base < last) load_tile(base);
   }
   // The waves' states merge in LDS.
+  float *so = (float *)sv;
   if (lane < QM) {   // lane h: head h's state
     s_m[wave][lane] = M;
     s_l[wave][lane] = L;
@@ -204,7 +214,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
   for (int i = 0; i < 4; ++i)
     if (4 * g + i < QM)
 #pragma unroll
-      for (int n = 0; n < NN; ++n) s_acc[wave][4 * g + i][16 * n + l16] = acc[n][i];
+      for (int n = 0; n < NN; ++n) so[(4 * g + i) * D + 16 * n + l16] = acc[n][i];
   __syncthreads();
   for (int i = tid; i < qm * D; i += 256) {
     const int h = i / D, c = i - h * D;
@@ -214,7 +224,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
     for (int w = 0; w < 4; ++w) {
       const float f = __expf(s_m[w][h] - gm);
       den += s_l[w][h] * f;
-      o += s_acc[w][h][c] * f;
+      o += ((const float *)s_v[w])[h * D + c] * f;
     }
     const size_t slot = (size_t)(h0 + h) * a.chunks + chunk;
     a.pout[slot * D + c] = o;
@@ -225,15 +235,29 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
   }
 }
 
-// One workgroup of 64 per query head. Lanes take chunks for the maximum and the denominator
-// (wave reductions), the chunk weights go to LDS, then lane i sums dimension i (and i + 64) over
-// the chunks in order, loads issued eight chunks at a time.
+// One workgroup of kMergeW waves per query head: each wave forms the maximum and the denominator (its lanes
+// take chunks) and one chunk's weight in kMergeW goes to LDS; wave w then sums chunks w, w + kMergeW, ... of every
+// dimension, sixteen loads in flight, and the waves' sums are added in wave order. (One wave summing all the
+// chunks eight at a time: 5.1 us at 128 chunks, now 4.8, most of it the launch and the first loads.)
+constexpr int kMergeW = 8;
 template <int D>
-__global__ __launch_bounds__(64) void attn_merge_kernel(AttnArgs a) {
+__global__ __launch_bounds__(64 * kMergeW) void attn_merge_kernel(AttnArgs a) {
   warm_kernargs<sizeof(AttnArgs)>();
   __shared__ float s_f[kAttnMaxChunks];
-  const int h = blockIdx.x, lane = threadIdx.x;
+  __shared__ float s_o[kMergeW][D];
+  const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float *pm = a.pmax + (size_t)h * a.chunks, *pd = a.pden + (size_t)h * a.chunks;
+  const float *po = a.pout + (size_t)h * a.chunks * D;
+  // The first round of partial sums is asked for with the chunk states.
+  constexpr int NB = 16, R = D / 64;
+  float v[NB][R];
+  auto load = [&](int c0) {
+#pragma unroll
+    for (int u = 0; u < NB; ++u)
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[u][r] = po[(size_t)min(c0 + kMergeW * u, a.chunks - 1) * D + lane + 64 * r];
+  };
+  load(wave);
   float g = -INFINITY;
   for (int c = lane; c < a.chunks; c += 64) g = fmaxf(g, pm[c]);
   g = wave_max(g);
@@ -241,33 +265,38 @@ __global__ __launch_bounds__(64) void attn_merge_kernel(AttnArgs a) {
   for (int c = lane; c < a.chunks; c += 64) den += pd[c] * __expf(pm[c] - g);
   den = wave_sum(den);
   const float inv = 1.f / den;
-  for (int c = lane; c < a.chunks; c += 64) s_f[c] = __expf(pm[c] - g) * inv;
+  for (int c = threadIdx.x; c < a.chunks; c += 64 * kMergeW) s_f[c] = __expf(pm[c] - g) * inv;
   __syncthreads();
-  const float *po = a.pout + (size_t)h * a.chunks * D;
+  float sum[R];
 #pragma unroll
-  for (int r = 0; r < D / 64; ++r) {
-    const int i = lane + 64 * r;
-    float sum = 0.f;
-    int c = 0;
-    for (; c + 8 <= a.chunks; c += 8) {
-      float v[8];
+  for (int r = 0; r < R; ++r) sum[r] = 0.f;
+  for (int c0 = wave; c0 < a.chunks; c0 += NB * kMergeW) {
+    if (c0 != wave) load(c0);
 #pragma unroll
-      for (int u = 0; u < 8; ++u) v[u] = po[(size_t)(c + u) * D + i];
+    for (int u = 0; u < NB; ++u) {
+      if (c0 + kMergeW * u >= a.chunks) break;
 #pragma unroll
-      for (int u = 0; u < 8; ++u) sum = fmaf(v[u], s_f[c + u], sum);
+      for (int r = 0; r < R; ++r) sum[r] = fmaf(v[u][r], s_f[c0 + kMergeW * u], sum[r]);
     }
-    for (; c < a.chunks; ++c) sum = fmaf(po[(size_t)c * D + i], s_f[c], sum);
-    a.out[(size_t)h * D + i] = sum;
+  }
+#pragma unroll
+  for (int r = 0; r < R; ++r) s_o[wave][lane + 64 * r] = sum[r];
+  __syncthreads();
+  if (threadIdx.x < D) {
+    float o = s_o[0][threadIdx.x];
+#pragma unroll
+    for (int w = 1; w < kMergeW; ++w) o += s_o[w][threadIdx.x];
+    a.out[(size_t)h * D + threadIdx.x] = o;
   }
 }
 
 hipError_t launch_attention_decode(const AttnArgs &a, hipStream_t s) {
   if (a.d == 64) {
     hipLaunchKernelGGL(attn_split_kernel<64>, dim3(a.kvh * a.chunks), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(attn_merge_kernel<64>, dim3(a.qh), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(attn_merge_kernel<64>, dim3(a.qh), dim3(64 * kMergeW), 0, s, a);
   } else {
     hipLaunchKernelGGL(attn_split_kernel<128>, dim3(a.kvh * a.chunks), dim3(256), 0, s, a);
-    hipLaunchKernelGGL(attn_merge_kernel<128>, dim3(a.qh), dim3(64), 0, s, a);
+    hipLaunchKernelGGL(attn_merge_kernel<128>, dim3(a.qh), dim3(64 * kMergeW), 0, s, a);
   }
   return hipGetLastError();
 }
