@@ -176,26 +176,33 @@ int large_item_tokens(const hh_moe_desc &d) {
   return 0;
 }
 
-int token_tile_nt(const hh_moe_desc &d, int T) {
-  // Prefill work items of 16·nt tokens: 32, or where experts average enough tokens BF16 160 (the
+int token_tile_nt(const hh_moe_desc &d, int T, bool compact = false) {
+  // Prefill work items of 16·nt tokens (`compact`: no more items than 32-token ones): 32, or where experts average enough tokens BF16 160 (the
   // weight tile is then read once per 160 tokens), MXFP4 64 for the gate-up (without a shared expert;
   // rows below 1024 columns: not measured), whose down product runs the same segments as 32-token items
   // (Scratch::half_down).
   const int avg = large_item_tokens(d);
+  // MXFP4, few tokens an expert and few experts: 16-token items let three workgroups share a compute unit (50 KB
+  // of LDS each), and the gate-up's 256-row tiles of every expert then run at once on 256 of them. 32 experts
+  // (736 tasks) T = 45: 168 -> 156 us the layer; 128 experts with a Zipf load T = 128: 210 -> 224.
+  if (!compact && d.quant == HH_QUANT_MXFP4 && (int64_t)T * d.top_k < 8 * (int64_t)d.experts &&
+      (int64_t)d.experts * ((2 * d.intermediate + 255) / 256) <= 3 * 256)
+    return 1;
   if (!avg || (int64_t)T * d.top_k < (int64_t)avg * d.experts) return 2;
   return d.quant == HH_QUANT_BF16 ? 10 : 4;
 }
 
-// `decode`: batches of at most kSmallT tokens take the decode kernels whatever mid_tokens says.
-Scratch plan(const hh_moe_desc &d, int T, bool decode = false) {
+// `compact`: the least scratch: batches of at most kSmallT tokens take the decode kernels (no slot
+// outputs), larger ones no 16-token items.
+Scratch plan(const hh_moe_desc &d, int T, bool compact = false) {
   Scratch s{};
-  s.products = T > kSmallT || (!decode && T >= mid_tokens(d));
+  s.products = T > kSmallT || (!compact && T >= mid_tokens(d));
   const int E = d.experts, K = d.top_k, H = d.hidden;
   const bool shared = d.shared_intermediate > 0;
   s.slots = K + (shared ? 1 : 0);
   s.positions = T * K + (shared ? T : 0);
   s.ldh = (int)align_up((size_t)std::max(d.intermediate, d.shared_intermediate), 64);
-  s.nt = token_tile_nt(d, T);
+  s.nt = token_tile_nt(d, T, compact);
   s.tile_tokens = 16 * s.nt;
   const int A = T * K;
   s.max_work = std::min(E, A) + (A + s.tile_tokens - 1) / s.tile_tokens +
@@ -827,7 +834,7 @@ int hh_moe_forward_noalloc(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weigh
   if (T == 0) return HH_OK;
   if (!ctx->scratch) return fail(HH_EHIP, "static scratch unavailable: " + ctx->scratch_error);
   Scratch s = plan(*d, T);
-  if (s.total > HH_NOALLOC_SCRATCH_BYTES && T <= kSmallT) s = plan(*d, T, true);   // no slot outputs
+  if (s.total > HH_NOALLOC_SCRATCH_BYTES) s = plan(*d, T, true);
   if (s.total > HH_NOALLOC_SCRATCH_BYTES)
     return fail(HH_ENOMEM, "the call needs " + std::to_string(s.total) +
                                " bytes of scratch; the allocation-free entry point has " +

@@ -466,7 +466,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Before (persistent kernels with loader waves): T = 2048 483 / 368, T = 512 222 / 148, and 102 / 55 at
 // T = 45 of the 32-expert layer, now 405 / 279, 183 / 116 and 92 / 49.
 // Gate-up items hold 64 tokens where experts average 16 or more (T = 2048 405, with 32 tokens 480;
-// T = 512 183 against 199), down items 32 (three terms: a 64-token stage leaves one slot).
+// T = 512 183 against 199), 16 where few experts have few tokens each (three workgroups per compute
+// unit: 92 -> 78 at T = 45), down items 32 (three terms: a 64-token stage leaves one slot).
 template <int PH, int NT_> struct Mx {
   static constexpr int NT = NT_, NTERM = PH == PH_UP ? NTX : NTH;
   static constexpr int NJ = 4;                               // 16-row tiles per wave, their 1 KiB loads per stage
@@ -482,7 +483,7 @@ template <int PH, int NT_> struct Mx {
 };
 
 template <int PH, int NT_>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_mx(GemmArgs a) {
+__global__ __launch_bounds__(256, NT_ == 1 ? 3 : 2) void prefill_mx(GemmArgs a) {
   using C = Mx<PH, NT_>;
   constexpr int NT = C::NT, NTERM = C::NTERM, NJ = C::NJ, TOK = C::TOK;
   extern __shared__ __align__(16) uint8_t lds[];
@@ -725,12 +726,14 @@ template <int PH, int NT> static hipError_t launch_mx(const GemmArgs &a, hipStre
 }
 
 // The tile of each call. BF16 work items hold 160 tokens (nt 10: experts averaging 40 tokens or
-// more) or 32, MXFP4 gate-up items 64 (nt 4) or 32, all others 32.
+// more) or 32, MXFP4 items 16 (nt 1), 32, or 64 for the gate-up
+// (nt 4), MLX items 32.
 hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
   const bool up = phase == PH_UP;
   if (quant == Q_MLX4) return up ? launch_mlx<PH_UP, 4, 2, 2>(a, s, tm) : launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
   if (quant == Q_MLX8) return up ? launch_mlx<PH_UP, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
   if (quant == Q_MXFP4) {
+    if (nt == 1) return up ? launch_mx<PH_UP, 1>(a, s, tm) : launch_mx<PH_DOWN, 1>(a, s, tm);
     if (up) return nt == 4 ? launch_mx<PH_UP, 4>(a, s, tm) : launch_mx<PH_UP, 2>(a, s, tm);
     return launch_mx<PH_DOWN, 2>(a, s, tm);
   }

@@ -32,6 +32,7 @@ CASES = {
     "mlx8_one_group": (MLX4.replace(quant=F.QUANT_MLX8, hidden=64, intermediate=64, shared_intermediate=0), 50),
     "mx_half_stage": (MX.replace(hidden=64, intermediate=64), 17),           # one stage of 64 columns
     "mx_ragged": (MX.replace(hidden=192, intermediate=320), 60),             # 40 an expert: two items of 32
+    "mx_16": (MX.replace(hidden=192, intermediate=320, experts=8, top_k=1), 60),   # 16-token items, a skewed load
     "mx_64": (MX.replace(hidden=1088, intermediate=1024, experts=2, top_k=1), 150),   # 64-token gate-up items
     "mx_shared": (MX.replace(hidden=448, intermediate=192, shared_intermediate=320, expert_bias=0), 90),
     "mlx8_odd_groups": (MLX4.replace(quant=F.QUANT_MLX8, hidden=448, intermediate=320, shared_intermediate=192), 70),
@@ -45,7 +46,7 @@ def test_prefill_tiles(name):
     from oracle import oracle as O
     desc, T = CASES[name]
     print(f"[gpu] prefill tiles {name} T={T}", flush=True)
-    layer = synth.make_layer(desc, seed=11)
+    layer = synth.make_layer(desc, seed=11, zipf=2.5 if name == "mx_16" else None)
     x = synth.make_tokens(desc.hidden, T, seed=12)
     L = MoELayer(layer, device=0)
     y, idx, _ = (t.cpu().numpy() for t in L.forward(x))
