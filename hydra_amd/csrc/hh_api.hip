@@ -177,10 +177,10 @@ int large_item_tokens(const hh_moe_desc &d) {
 }
 
 int token_tile_nt(const hh_moe_desc &d, int T, bool compact = false) {
-  // Prefill work items of 16·nt tokens (`compact`: no more items than 32-token ones): 32, or where experts average enough tokens BF16 160 (the
-  // weight tile is then read once per 160 tokens), MXFP4 64 for the gate-up (without a shared expert;
-  // rows below 1024 columns: not measured), whose down product runs the same segments as 32-token items
-  // (Scratch::half_down).
+  // Prefill work items of 16·nt tokens (`compact`: no more items than 32-token ones): 32, or where
+  // experts average enough tokens BF16 160 (the weight tile is then read once per 160 tokens), MXFP4 64
+  // for the gate-up (without a shared expert; rows below 1024 columns: not measured), whose down product
+  // runs the same segments as 32-token items (Scratch::half_down).
   const int avg = large_item_tokens(d);
   // MXFP4, few tokens an expert and few experts: 16-token items let three workgroups share a compute unit (50 KB
   // of LDS each), and the gate-up's 256-row tiles of every expert then run at once on 256 of them. 32 experts
@@ -254,6 +254,12 @@ Scratch plan(const hh_moe_desc &d, int T, bool compact = false) {
 int below_large_items(const hh_moe_desc &d, int T) {
   const int64_t last = ((int64_t)large_item_tokens(d) * d.experts + d.top_k - 1) / d.top_k - 1;
   return last < 1 ? T : (int)std::min<int64_t>(T, last);
+}
+
+// An arena that may not grow (a capture, or graphs that use it) and is too small for `bytes`: the call
+// takes the compact plan, which asks for no more than the decode kernels or 32-token items need.
+bool arena_short(const hh_ctx *ctx, size_t bytes) {
+  return ctx->arena_bytes < bytes && (ctx->capturing || ctx->live_graphs > 0);
 }
 
 int ensure_arena(hh_ctx *ctx, size_t bytes) {
@@ -774,7 +780,8 @@ int hh_moe_forward(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w,
   if (rc) return rc;
   if (T == 0) return HH_OK;
   HH_HIP(hipSetDevice(ctx->device));
-  const Scratch s = plan(*d, T);
+  Scratch s = plan(*d, T);
+  if (arena_short(ctx, s.total)) s = plan(*d, T, true);
   if ((rc = ensure_arena(ctx, s.total))) return rc;
   return forward_layer(ctx, d, w, x, x_router, T, y, topk_idx, topk_w, ctx->arena, s, false);
 }
@@ -794,7 +801,8 @@ int hh_moe_block_forward(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights
   if (dense_out && ((uintptr_t)dense_out & 15)) return fail(HH_EALIGN, "dense_out must be 16-byte aligned");
   if (T == 0) return HH_OK;
   HH_HIP(hipSetDevice(ctx->device));
-  const Scratch s = plan(*d, T);
+  Scratch s = plan(*d, T);
+  if (arena_short(ctx, block_plan(*d, s, T, gemma).total)) s = plan(*d, T, true);
   const BlockScratch bs = block_plan(*d, s, T, gemma);
   const bool router_resid = d->router == HH_ROUTER_GEMMA;
   const size_t o_xn = bs.xn, o_xr = bs.xr, o_mix = bs.mix;
@@ -1034,7 +1042,7 @@ int hh_router_topk(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w,
   if (T < 0 || T > kMaxTokens) return fail(HH_EINVAL, "token count outside 0..65536");
   if (T == 0) return HH_OK;
   HH_HIP(hipSetDevice(ctx->device));
-  const Scratch s = plan(*d, T);
+  const Scratch s = plan(*d, T, true);   // no products follow
   rc = ensure_arena(ctx, s.total);
   if (rc) return rc;
   hh::RouteArgs r = route_args(*d, w, ctx->arena, s, x_router, x_router, T);
@@ -1073,7 +1081,7 @@ int hh_permute(hh_ctx *ctx, const int32_t *topk_idx, int32_t T, int32_t K, int32
   HH_HIP(hipSetDevice(ctx->device));
   hh_moe_desc d{};
   d.hidden = 64; d.intermediate = 64; d.experts = E; d.top_k = K;
-  const Scratch s = plan(d, std::max(T, 1));
+  const Scratch s = plan(d, std::max(T, 1), true);
   int rc = ensure_arena(ctx, s.total);
   if (rc) return rc;
   hh::RouteArgs r = route_args(d, nullptr, ctx->arena, s, nullptr, nullptr, T);

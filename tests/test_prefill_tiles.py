@@ -56,3 +56,38 @@ def test_prefill_tiles(name):
     for t in (0, T // 2, T - 1):
         y1 = L.forward(x[t:t + 1])[0].cpu().numpy()[0]
         assert np.array_equal(y1.view(np.uint32), y[t].view(np.uint32))
+
+
+@pytest.mark.gpu
+def test_products_where_the_arena_may_not_grow():
+    """An arena that covers a batch's decode kernels (11 KB) and not its grouped products (44 KB), and
+    may not grow, being captured from or used by a graph: the batch still runs, with the same bits,
+    and a larger one (over 98 KB) is refused."""
+    import torch
+    from hydra_amd._lib import HydraHIPError
+    from hydra_amd.layer import Context, MoELayer
+    print("[gpu] products in a pinned arena", flush=True)
+    desc = BF16.replace(hidden=832, intermediate=192)
+    layer = synth.make_layer(desc, seed=4)
+    xs = synth.make_tokens(832, 64, seed=5)
+    want = MoELayer(layer, device=0).forward(xs[:5])[0]
+    ctx = Context(0)
+    try:
+        L = MoELayer(layer, ctx)
+        ctx.reserve(BF16.replace(hidden=64, intermediate=64), 24)   # 30 KB
+        x = torch.from_numpy(xs[:5].view(np.int16)).to("cuda:0")
+        y = torch.zeros((5, 832), dtype=torch.float32, device="cuda:0")
+        torch.cuda.synchronize()
+        graph = ctx.capture(lambda: L.forward_into(x, y))
+        assert torch.equal(L.forward(xs[:5])[0], want)
+        for _ in range(3):
+            y.zero_()
+            torch.cuda.synchronize()
+            graph.launch()
+            ctx.synchronize()
+            assert torch.equal(y, want)
+        with pytest.raises(HydraHIPError):
+            L.forward(xs)
+        graph.close()
+    finally:
+        ctx.close()
