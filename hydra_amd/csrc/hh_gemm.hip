@@ -1,5 +1,4 @@
-// hh_gemm.hip — the decode expert products on gfx950 MFMA, and the arithmetic they share with the
-// grouped ones (hh_prefill.hip).
+// hh_gemm.hip — grouped expert products on gfx950 MFMA, shared by decode and prefill.
 //
 // Two products per layer:
 //   PH_UP   : h[s][i] = act(gate_i · x_t + b, up_i · x_t + b) for every slot s = t·slots + r
@@ -27,7 +26,7 @@
 //     tokens' x rows staged in LDS. down_small computes 16 hidden rows of one token for all of
 //     its slots (one wave per slot) and sums them in rank order in the epilogue: no slot buffer,
 //     no combine launch.
-//   More tokens (MXFP4 above 16, BF16 and MLX above 4): hh_prefill.hip.
+//   T > 16: hh_prefill.hip.
 //
 // MFMA operand mapping (16x16x32, lane l, lane group g = l/16): A lane l supplies row l%16,
 // B lane l supplies token column l%16, each with 8 consecutive K values; D lane l holds rows
@@ -1570,7 +1569,7 @@ __global__ __launch_bounds__(256, 2) void decode_mx(GemmArgs a, RouteArgs ra, Fu
   }
 }
 
-#if !defined(HH_GEMM_BLOCK) && !defined(HH_GEMM_BF16) && !defined(HH_GEMM_MLX)
+#ifndef HH_GEMM_KERNELS_ONLY
 // y[t][j] = Σ_r slot[t·slots + r][j] in rank order (sum_expert_slices, dense.metal:147; the
 // shared expert's slot comes last as in QwenReferenceLayer.swift:399-404).
 __global__ __launch_bounds__(256) void combine_kernel(const float *slot_out, int slots, int H,
@@ -1615,65 +1614,44 @@ constexpr int MX_STATIC = 23;
 // MLX gate-up rows of exactly 2·MLX_NCW chunks (K = 2048: Qwen3.5-35B-A3B) take the single-round
 // stream of MLX_NCW chunks per wave.
 constexpr int MLX_NCW = 16;
-// The decode kernels come from four code objects: MXFP4's here, the FFN block's (HH_GEMM_BLOCK), the BF16
-// (HH_GEMM_BF16) and the MLX ones (HH_GEMM_MLX). A kernel's speed moves with the make-up of its code object though
-// its instructions stay the same: MXFP4 T = 4 59.4 us the layer with all formats in one object, 58.1 apart.
+#ifndef HH_GEMM_KERNELS_ONLY
+// fr: 0 none, 1 the fused router over x, 2 the fused router over the FFN block's residual.
 UpSmallKernel up_small_block_k(bool st, int T);
-UpSmallKernel up_small_bf16_k(int T);
-DownSmallKernel down_small_bf16_k(int slots);
-// `st` staged scales, `stat` the chunk count of MLX_NCW compiled in (T = 1).
-UpSmallKernel up_small_mlx_k(int quant, int T, bool st = false, bool stat = false);
-DownSmallKernel down_small_mlx_k(int quant, int slots, bool st = false);
-// BF16 and MLX split down's K by chunk parity over two waves when the workgroup has room; nine waves
-// leave a third of the register file per wave: a shallower ring.
-#if defined(HH_GEMM_BF16)
-UpSmallKernel up_small_bf16_k(int T) {
-  return T == 1 ? up_small<Q_BF16, decode_depth<Q_BF16>(), 1, 2> : up_small<Q_BF16, decode_depth<Q_BF16>(), 1, MX_XB_WIDE>;
-}
-DownSmallKernel down_small_bf16_k(int slots) {
-  return slots > 4 ? down_small<Q_BF16, decode_depth<Q_BF16>(), kMaxTopK + 1, 1> : down_small<Q_BF16, decode_depth<Q_BF16>(), 4, 2>;
-}
-#elif defined(HH_GEMM_MLX)
-template <int FMT> static UpSmallKernel up_k(int T, bool st, bool stat) {
-  constexpr int D = decode_depth<FMT>();
-  if (st && T == 1 && stat) return up_small<FMT, MLX_NCW, 1, 2, true, MLX_NCW>;
-  if (st) return T == 1 ? up_small<FMT, D, 1, 2, true> : up_small<FMT, D, 1, MX_XB_WIDE, true>;
-  return T == 1 ? up_small<FMT, D, 1, 2> : up_small<FMT, D, 1, MX_XB_WIDE>;
-}
-template <int FMT> static DownSmallKernel down_k(int slots, bool st) {
-  constexpr int D = decode_depth<FMT>();
-  if (st) return slots > 4 ? down_small<FMT, D, kMaxTopK + 1, 1, true> : down_small<FMT, D, 4, 2, true>;
-  return slots > 4 ? down_small<FMT, D, kMaxTopK + 1, 1> : down_small<FMT, D, 4, 2>;
-}
-UpSmallKernel up_small_mlx_k(int quant, int T, bool st, bool stat) {
-  return quant == Q_MLX4 ? up_k<Q_MLX4>(T, st, stat) : up_k<Q_MLX8>(T, st, stat);
-}
-DownSmallKernel down_small_mlx_k(int quant, int slots, bool st) {
-  return quant == Q_MLX4 ? down_k<Q_MLX4>(slots, st) : down_k<Q_MLX8>(slots, st);
-}
-#elif defined(HH_GEMM_BLOCK)
-UpSmallKernel up_small_block_k(bool st, int T) {
-  if (st) return T == 1 ? up_small_mx<MX_ONE, true, 2, MX_STATIC, 2> : up_small_mx<MX_ONE, true, MX_XB_WIDE, MX_STATIC, 2>;
-  return T == 1 ? up_small_mx<MX_ONE, true, 2, 0, 2> : up_small_mx<MX_ONE, true, MX_XB_WIDE, 0, 2>;
-}
-#else
-// MXFP4. fr: 0 none, 1 the fused router over x, 2 the fused router over the FFN block's residual
-// (single-round rows only).
-static UpSmallKernel up_small_mx_k(bool one, int T, bool st = false, int fr = 0) {
-  if (fr == 2) return up_small_block_k(st, T);
-  if (fr) {
-    if (st) return T == 1 ? up_small_mx<MX_ONE, true, 2, MX_STATIC, 1> : up_small_mx<MX_ONE, true, MX_XB_WIDE, MX_STATIC, 1>;
-    return T == 1 ? up_small_mx<MX_ONE, true, 2, 0, 1> : up_small_mx<MX_ONE, true, MX_XB_WIDE, 0, 1>;
+template <int FMT> static UpSmallKernel up_small_k(bool one, int T, bool st = false, bool stat = false, int fr = 0) {
+  if constexpr (FMT == Q_MXFP4) {
+    if (fr == 2) return up_small_block_k(st, T);   // the fused router: single-round rows only
+    if (fr) {
+      if (st) return T == 1 ? up_small_mx<MX_ONE, true, 2, MX_STATIC, 1> : up_small_mx<MX_ONE, true, MX_XB_WIDE, MX_STATIC, 1>;
+      return T == 1 ? up_small_mx<MX_ONE, true, 2, 0, 1> : up_small_mx<MX_ONE, true, MX_XB_WIDE, 0, 1>;
+    }
+    if (one && st) return T == 1 ? up_small_mx<MX_ONE, true, 2, MX_STATIC> : up_small_mx<MX_ONE, true, MX_XB_WIDE, MX_STATIC>;
+    if (T == 1) return one ? up_small_mx<MX_ONE, true, 2> : up_small_mx<16, false, 2>;
+    return one ? up_small_mx<MX_ONE, true, MX_XB_WIDE> : up_small_mx<16, false, MX_XB_WIDE>;
   }
-  if (one && st) return T == 1 ? up_small_mx<MX_ONE, true, 2, MX_STATIC> : up_small_mx<MX_ONE, true, MX_XB_WIDE, MX_STATIC>;
-  if (T == 1) return one ? up_small_mx<MX_ONE, true, 2> : up_small_mx<16, false, 2>;
-  return one ? up_small_mx<MX_ONE, true, MX_XB_WIDE> : up_small_mx<16, false, MX_XB_WIDE>;
+  else if constexpr (is_mlx<FMT>()) {
+    if (st && T == 1 && stat) return up_small<FMT, MLX_NCW, 1, 2, true, MLX_NCW>;
+    if (st) return T == 1 ? up_small<FMT, decode_depth<FMT>(), 1, 2, true> : up_small<FMT, decode_depth<FMT>(), 1, MX_XB_WIDE, true>;
+    return T == 1 ? up_small<FMT, decode_depth<FMT>(), 1, 2> : up_small<FMT, decode_depth<FMT>(), 1, MX_XB_WIDE>;
+  }
+  else if (T == 1) return up_small<FMT, decode_depth<FMT>(), 1, 2>;
+  else return up_small<FMT, decode_depth<FMT>(), 1, MX_XB_WIDE>;
 }
-// One chain over K, so one wave per slot; a shallower ring for more than four slots and for rows
-// longer than MX_ONE chunks.
-static DownSmallKernel down_small_mx_k(int slots, bool one) {
-  if (slots > 4 || !one) return down_small<Q_MXFP4, 8, kMaxTopK + 1, 1>;
-  return down_small<Q_MXFP4, decode_depth<Q_MXFP4>(), 4, 1>;
+// Waves per slot of down_small: MXFP4's canonical arithmetic is one chain over K (one wave per
+// slot); the others split K by chunk parity over two waves when the workgroup has room.
+template <int FMT> constexpr int down_ks(int slots) { return (FMT == Q_MXFP4 || slots > 4) ? 1 : 2; }
+
+template <int FMT> static DownSmallKernel down_small_k(int slots, bool one, bool st = false) {
+  // Nine waves leave a third of the register file per wave: a shallower ring (also the MXFP4
+  // kernel for rows longer than MX_ONE chunks).
+  constexpr int D9 = decode_depth<FMT>() > 8 ? 8 : decode_depth<FMT>();
+  if (slots > 4 || !one) {
+    if constexpr (is_mlx<FMT>())
+      if (st) return down_small<FMT, D9, kMaxTopK + 1, 1, true>;
+    return down_small<FMT, D9, kMaxTopK + 1, 1>;
+  }
+  if constexpr (is_mlx<FMT>())
+    if (st) return down_small<FMT, decode_depth<FMT>(), 4, down_ks<FMT>(4), true>;
+  return down_small<FMT, decode_depth<FMT>(), 4, down_ks<FMT>(4)>;
 }
 // MLX: whether the staged-scale variants take this layer (the rows' chunk counts fit LDS).
 static bool mlx_staged_up(int hidden) { return hidden <= 64 * kMlxSbChunks; }
@@ -1721,24 +1699,34 @@ hipError_t launch_small(int quant, GemmArgs a, const RouteArgs &ra, hipStream_t 
   UpSmallKernel up;
   switch (quant) {
   // The MXFP4 static-count variant needs every up row (over H) at MX_STATIC chunks.
-  case Q_MXFP4: up = up_small_mx_k(one_up, T, (a.hidden + 127) / 128 == MX_STATIC, !fr ? 0 : ra.resid ? 2 : 1); break;
-  case Q_BF16: up = up_small_bf16_k(T); break;
-  default: up = up_small_mlx_k(quant, T, mlx_staged_up(a.hidden), (a.hidden + 63) / 64 == 2 * MLX_NCW); break;
+  case Q_MXFP4: up = up_small_k<Q_MXFP4>(one_up, T, (a.hidden + 127) / 128 == MX_STATIC, false, !fr ? 0 : ra.resid ? 2 : 1); break;
+  case Q_BF16: up = up_small_k<Q_BF16>(true, T); break;
+  case Q_MLX4: up = up_small_k<Q_MLX4>(true, T, mlx_staged_up(a.hidden), (a.hidden + 63) / 64 == 2 * MLX_NCW); break;
+  default: up = up_small_k<Q_MLX8>(true, T, mlx_staged_up(a.hidden), (a.hidden + 63) / 64 == 2 * MLX_NCW); break;
   }
   // The decode kernels stage rows in dynamic LDS beyond the default 64 KiB window (gfx950 has
   // 160 KiB per compute unit).
   static std::once_flag lds_once;
   std::call_once(lds_once, [] {
-    std::vector<const void *> ks;
-    for (int t : {1, SMALL_T}) {
-      for (bool st : {false, true}) {
-        for (bool one : {false, true}) ks.push_back((const void *)up_small_mx_k(one, t, st));
-        for (int f : {1, 2}) ks.push_back((const void *)up_small_mx_k(true, t, st, f));
-        for (int q : {Q_MLX4, Q_MLX8})
-          for (bool stat : {false, true}) ks.push_back((const void *)up_small_mlx_k(q, t, st, stat));
-      }
-      ks.push_back((const void *)up_small_bf16_k(t));
-    }
+    const void *ks[] = {(const void *)up_small_k<Q_MXFP4>(true, 1), (const void *)up_small_k<Q_MXFP4>(false, 1),
+                        (const void *)up_small_k<Q_MXFP4>(true, SMALL_T), (const void *)up_small_k<Q_MXFP4>(false, SMALL_T),
+                        (const void *)up_small_k<Q_BF16>(true, 1), (const void *)up_small_k<Q_MLX4>(true, 1),
+                        (const void *)up_small_k<Q_MLX8>(true, 1), (const void *)up_small_k<Q_BF16>(true, SMALL_T),
+                        (const void *)up_small_k<Q_MLX4>(true, SMALL_T), (const void *)up_small_k<Q_MLX8>(true, SMALL_T),
+                        (const void *)down_small_k<Q_MXFP4>(4, true), (const void *)down_small_k<Q_BF16>(4, true),
+                        (const void *)down_small_k<Q_MLX4>(4, true), (const void *)down_small_k<Q_MLX8>(4, true),
+                        (const void *)down_small_k<Q_MXFP4>(9, true), (const void *)down_small_k<Q_BF16>(9, true),
+                        (const void *)down_small_k<Q_MLX4>(9, true), (const void *)down_small_k<Q_MLX8>(9, true),
+                        (const void *)up_small_k<Q_MXFP4>(true, 1, true), (const void *)up_small_k<Q_MXFP4>(true, SMALL_T, true),
+                        (const void *)up_small_k<Q_MLX4>(true, 1, true), (const void *)up_small_k<Q_MLX4>(true, SMALL_T, true),
+                        (const void *)up_small_k<Q_MLX8>(true, 1, true), (const void *)up_small_k<Q_MLX8>(true, SMALL_T, true),
+                        (const void *)up_small_k<Q_MLX4>(true, 1, true, true), (const void *)up_small_k<Q_MLX8>(true, 1, true, true),
+                        (const void *)down_small_k<Q_MLX4>(4, true, true), (const void *)down_small_k<Q_MLX4>(9, true, true),
+                        (const void *)down_small_k<Q_MLX8>(4, true, true), (const void *)down_small_k<Q_MLX8>(9, true, true),
+                        (const void *)up_small_k<Q_MXFP4>(true, 1, true, false, true), (const void *)up_small_k<Q_MXFP4>(true, SMALL_T, true, false, true),
+                        (const void *)up_small_k<Q_MXFP4>(true, 1, false, false, true), (const void *)up_small_k<Q_MXFP4>(true, SMALL_T, false, false, true),
+                        (const void *)up_small_k<Q_MXFP4>(true, 1, true, false, 2), (const void *)up_small_k<Q_MXFP4>(true, SMALL_T, true, false, 2),
+                        (const void *)up_small_k<Q_MXFP4>(true, 1, false, false, 2), (const void *)up_small_k<Q_MXFP4>(true, SMALL_T, false, false, 2)};
     // Best effort: HIP on gfx950 accepts launches up to the hardware LDS size without it, and
     // a runtime that rejects the attribute must not leave its error for the launch check below.
     for (const void *k : ks) {
@@ -1794,17 +1782,18 @@ hipError_t launch_down_small(int quant, GemmArgs a, const int32_t *topk_idx, int
   const bool one_down = !mx || (imax + 127) / 128 <= MX_ONE;
   DownSmallKernel down;
   switch (quant) {
-  case Q_MXFP4: down = down_small_mx_k(S, one_down); break;
-  case Q_BF16: down = down_small_bf16_k(S); break;
-  default: down = down_small_mlx_k(quant, S, mlx_staged_down(S, imax)); break;
+  case Q_MXFP4: down = down_small_k<Q_MXFP4>(S, one_down); break;
+  case Q_BF16: down = down_small_k<Q_BF16>(S, true); break;
+  case Q_MLX4: down = down_small_k<Q_MLX4>(S, true, mlx_staged_down(S, imax)); break;
+  default: down = down_small_k<Q_MLX8>(S, true, mlx_staged_down(S, imax)); break;
   }
   static std::once_flag lds_once;
   std::call_once(lds_once, [] {
-    for (int sl : {4, 9})
-      for (const void *k : {(const void *)down_small_mx_k(sl, true), (const void *)down_small_mx_k(sl, false),
-                            (const void *)down_small_bf16_k(sl), (const void *)down_small_mlx_k(Q_MLX4, sl),
-                            (const void *)down_small_mlx_k(Q_MLX8, sl), (const void *)down_small_mlx_k(Q_MLX4, sl, true),
-                            (const void *)down_small_mlx_k(Q_MLX8, sl, true)}) {
+    for (int sl : {1, 2, 3, 4, 5, 6, 7, 8, 9})
+      for (const void *k : {(const void *)down_small_k<Q_MXFP4>(sl, true), (const void *)down_small_k<Q_MXFP4>(sl, false),
+                            (const void *)down_small_k<Q_BF16>(sl, true), (const void *)down_small_k<Q_MLX4>(sl, true),
+                            (const void *)down_small_k<Q_MLX8>(sl, true), (const void *)down_small_k<Q_MLX4>(sl, true, true),
+                            (const void *)down_small_k<Q_MLX8>(sl, true, true)}) {
         (void)hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
         (void)hipGetLastError();
       }
@@ -1887,6 +1876,15 @@ hipError_t launch_combine(const float *slot_out, int slots, int H, int T, float 
   hipExtLaunchKernelGGL(combine_kernel, dim3(blocks), dim3(256), 0, s, tm.start, tm.stop, 0,
                         slot_out, slots, H, T, y, resid);
   return hipGetLastError();
+}
+
+#else
+// The FFN block's MXFP4 gate-up kernels with the fused router, compiled in a translation unit of
+// their own (hh_gemm_block.hip): adding them leaves the code object of the other kernels as it
+// was (the decode kernels' speed had moved with it).
+UpSmallKernel up_small_block_k(bool st, int T) {
+  if (st) return T == 1 ? up_small_mx<MX_ONE, true, 2, MX_STATIC, 2> : up_small_mx<MX_ONE, true, MX_XB_WIDE, MX_STATIC, 2>;
+  return T == 1 ? up_small_mx<MX_ONE, true, 2, 0, 2> : up_small_mx<MX_ONE, true, MX_XB_WIDE, 0, 2>;
 }
 
 #endif
