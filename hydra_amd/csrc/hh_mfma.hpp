@@ -439,6 +439,22 @@ struct PrefillTasks {
   }
 };
 
+// Where an MXFP4 prefill wave finds its row scales in LDS. A row's three stages of scales come as the 16
+// bytes from the dword that holds block sc0 of the row, moved back where they would pass the
+// matrix's last byte: mx_scale_src is their offset in the matrix (rows of nsb blocks),
+// mx_scale_back how far they were moved. Only a wave that holds the matrix's last rows has any that
+// were (mx_last_rows, rw its first row): a wave wholly past them loads the last row's bytes, uses none,
+// and must not form a distance from rows that do not exist.
+__host__ __device__ constexpr bool mx_last_rows(int rw, int out_dim) { return rw < out_dim && rw + 64 >= out_dim; }
+__host__ __device__ constexpr int mx_scale_src(int row, int out_dim, int nsb, int sc0) {
+  const int at = (row * nsb + sc0) & ~3, end = out_dim * nsb - 16;
+  return at < end ? at : end;
+}
+__host__ __device__ constexpr int mx_scale_back(int row, int out_dim, int nsb, int sc0) {
+  const int past = ((row * nsb + sc0) & ~3) - (out_dim * nsb - 16);
+  return past > 0 ? past : 0;
+}
+
 // At most N of the wave's loads outstanding.
 template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 

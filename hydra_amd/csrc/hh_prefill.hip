@@ -506,7 +506,7 @@ __global__ __launch_bounds__(256, NT_ == 1 ? 3 : 2) void prefill_mx(GemmArgs a) 
   const int rw = rt * C::ROWS + 64 * wave;   // the wave's first row
   const bool active = rw < out_dim;
   const bool part = (K & 127) != 0;   // the last stage holds 64 columns
-  const bool last_rows = rw + 64 >= out_dim;   // holds the rows within 16 bytes of the scales' end
+  const bool last_rows = mx_last_rows(rw, out_dim);   // holds the rows within 16 bytes of the scales' end
 
   const int rowb = K / 2;
   const int lr = lane >> 2, seg = (lane & 3) ^ ((lr >> 1) & 3);
@@ -521,7 +521,7 @@ __global__ __launch_bounds__(256, NT_ == 1 ? 3 : 2) void prefill_mx(GemmArgs a) 
   // Block scales of row rw + lane: 16 bytes from the dword that holds a stage's
   // first, which covers three stages; moved back where they would pass the matrix's last byte.
   const uint8_t *sbase_w = blob + grp.off[PH == PH_UP ? 1 : 4];
-  const int srow = min(rw + lane, out_dim - 1), sc_end = out_dim * nsb - 16;
+  const int srow = min(rw + lane, out_dim - 1);
   const int ntok = (cnt + 15) & ~15;   // operand rows past the last used token tile are not loaded
   const uint8_t *bsrc[C::BPW];
   bool bon[C::BPW];
@@ -548,7 +548,7 @@ __global__ __launch_bounds__(256, NT_ == 1 ? 3 : 2) void prefill_mx(GemmArgs a) 
     const uint32_t st = l0 + (uint32_t)(qs * C::STAGE);
     if (q3 == 0) {
       const uint32_t qd = l0 + C::OFF_Q + qset * C::QUAD;
-      dma16(sbase_w + min((srow * nsb + 4 * q) & ~3, sc_end), qd + 1024 * wave);
+      dma16(sbase_w + mx_scale_src(srow, out_dim, nsb, 4 * q), qd + 1024 * wave);
       if (wave < C::BSL) dma16(bssrc + 4 * q, qd + C::QB + 1024 * wave);
       qset ^= 1;
     }
@@ -597,7 +597,7 @@ __global__ __launch_bounds__(256, NT_ == 1 ? 3 : 2) void prefill_mx(GemmArgs a) 
     for (int j = 0; j < NJ; ++j) {
       w[j] = *(const u32x4 *)(stg + aro + 1024 * j);
       int back = 0;   // how far the row's 16 bytes were moved back
-      if (last_rows) back = max(0, (((rw + 16 * j + l16) * nsb + sc0) & ~3) - sc_end);
+      if (last_rows) back = mx_scale_back(rw + 16 * j + l16, out_dim, nsb, sc0);
       sa[j] = qd[sro + 256 * j + back];
     }
     // The wave's weight tiles are in registers: their slot takes the stage after the next, two
