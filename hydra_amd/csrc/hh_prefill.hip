@@ -12,20 +12,20 @@ constexpr int kRowParts = 2;   // row-tile parts of the XCDs (PrefillTasks)
 // 16 bytes per lane from global memory straight into LDS: base (uniform) + off (per lane) to LDS
 // byte `l` + 16·lane. Written in assembly so that the compiler does not order the wave's own LDS
 // reads after its loads in flight (it would wait for all of them); the kernels wait with wait_vm.
-// The instruction has no register result.
+// The instruction has no register result; its LDS address goes through m0.
 __device__ __forceinline__ void dma16(const void *base, uint32_t off, uint32_t l) {
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(l), "v"(off), "s"(base)
-               : "memory");
+               : "memory", "m0");
 }
 __device__ __forceinline__ void dma16(const void *p, uint32_t l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(p) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(l), "v"(p) : "memory", "m0");
 }
 // 4 (2) bytes per lane to LDS byte `l` + 4·lane.
 __device__ __forceinline__ void dma4(const void *p, uint32_t l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(l), "v"(p) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, off" ::"s"(l), "v"(p) : "memory", "m0");
 }
 __device__ __forceinline__ void dma2(const void *p, uint32_t l) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" ::"s"(l), "v"(p) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, off" ::"s"(l), "v"(p) : "memory", "m0");
 }
 // Barrier after the wave's own LDS reads have returned: the next stage may overwrite what they read.
 __device__ __forceinline__ void step_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
