@@ -463,8 +463,10 @@ __device__ __forceinline__ TokenScreen screen_token(const RouteArgs &a, int t, L
     if (e < E) {
       const float l = (float)(fscale * (double)lgf(e));
       const float err = cb * wnf(e) + 2.384185791015625e-07f * fabsf(l) + 1e-30f;
-      lb[j] = l - err;
-      ub[j] = l + err;
+      // A bound that is NaN (infinities in the row or the fp32 sum) says nothing: the expert is a
+      // candidate, so at least K experts always are.
+      lb[j] = fmaxf(l - err, -INFINITY);
+      ub[j] = fminf(l + err, INFINITY);
     } else {
       lb[j] = -INFINITY;
       ub[j] = -INFINITY;
