@@ -262,6 +262,15 @@ bool arena_short(const hh_ctx *ctx, size_t bytes) {
   return ctx->arena_bytes < bytes && (ctx->capturing || ctx->live_graphs > 0);
 }
 
+// Bytes that every batch of up to T tokens fits: `bytes(t, compact)` gives those of one batch.
+// Where the arena may not grow, a reservation asks for what its calls would then take.
+template <class Bytes> size_t reserve_bytes(const hh_ctx *ctx, const hh_moe_desc &d, int T, Bytes bytes) {
+  size_t need[2] = {0, 0};   // as planned, compact
+  for (int t : {T, below_large_items(d, T)})
+    for (int c : {0, 1}) need[c] = std::max(need[c], bytes(t, c != 0));
+  return need[arena_short(ctx, need[0]) ? 1 : 0];
+}
+
 int ensure_arena(hh_ctx *ctx, size_t bytes) {
   if (ctx->arena_bytes >= bytes) return HH_OK;
   if (ctx->capturing)
@@ -768,9 +777,7 @@ int hh_ctx_reserve(hh_ctx *ctx, const hh_moe_desc *d, int32_t max_tokens) {
   int rc = check_desc(d);
   if (rc) return rc;
   if (max_tokens <= 0 || max_tokens > kMaxTokens) return fail(HH_EINVAL, "max_tokens outside 1..65536");
-  size_t need = 0;
-  for (int t : {max_tokens, below_large_items(*d, max_tokens)}) need = std::max(need, plan(*d, t).total);
-  return ensure_arena(ctx, need);
+  return ensure_arena(ctx, reserve_bytes(ctx, *d, max_tokens, [&](int t, bool c) { return plan(*d, t, c).total; }));
 }
 
 int hh_moe_forward(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w,
@@ -1266,8 +1273,9 @@ int hh_runner_reserve(hh_runner *r, int32_t max_tokens) {
   for (const hh_runner::Layer &L : r->layers) {
     if (!L.set) return fail(HH_EINVAL, "a layer of the runner is not set");
     const bool gemma = L.norms.post_expert_norm != nullptr;
-    for (int t : {max_tokens, below_large_items(L.desc, max_tokens)})
-      need = std::max(need, block_plan(L.desc, plan(L.desc, t), t, gemma).total);
+    need = std::max(need, reserve_bytes(r->ctx, L.desc, max_tokens, [&](int t, bool c) {
+                      return block_plan(L.desc, plan(L.desc, t, c), t, gemma).total;
+                    }));
   }
   return ensure_arena(r->ctx, need);
 }

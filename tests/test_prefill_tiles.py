@@ -91,3 +91,33 @@ def test_products_where_the_arena_may_not_grow():
         graph.close()
     finally:
         ctx.close()
+
+
+@pytest.mark.gpu
+def test_reservation_where_the_arena_may_not_grow():
+    """While a graph pins the arena, a reservation that the calls' fallback fits is granted (the
+    context's and a runner's), and one that it does not fit is refused."""
+    import torch
+    from hydra_amd._lib import HydraHIPError
+    from hydra_amd.layer import Context, MoELayer, Runner, to_device
+    print("[gpu] reservation in a pinned arena", flush=True)
+    desc = BF16.replace(hidden=832, intermediate=192, router=F.ROUTER_SOFTMAX_TOPK_RENORM)
+    ctx = Context(0)
+    try:
+        L = MoELayer(synth.make_layer(desc, seed=4), ctx)
+        runner = Runner(ctx, [(L, {"pre_norm": to_device(synth.f32_to_bf16(np.ones(832, np.float32)), "cuda:0")}, None)])
+        ctx.reserve(BF16.replace(hidden=64, intermediate=64), 24)   # 30 KB: as above
+        x = torch.zeros((1, 832), dtype=torch.int16, device="cuda:0")
+        y = torch.zeros((1, 832), dtype=torch.float32, device="cuda:0")
+        torch.cuda.synchronize()
+        graph = ctx.capture(lambda: L.forward_into(x, y))
+        ctx.reserve(desc, 5)
+        runner.reserve(5)
+        for reserve in (lambda: ctx.reserve(desc, 64), lambda: runner.reserve(64)):
+            with pytest.raises(HydraHIPError):
+                reserve()
+        graph.close()
+        runner.reserve(64)
+        runner.close()
+    finally:
+        ctx.close()
