@@ -158,16 +158,27 @@ struct Scratch {
   int xld, hld;   // MXFP4: row lengths of the fp8 operand terms (multiples of 512)
 };
 
-constexpr int kSmallT = 16;  // batches up to this size take the decode kernels, or (mid_tokens) the prefill products
+constexpr int kSmallT = 16;  // batches up to this size take the decode kernels, or (mid_batch) the prefill products
 
-// Smallest batch of at most kSmallT tokens that takes the prefill products after the decode router's logits. The
+// Whether a batch of at most kSmallT tokens takes the prefill products after the decode router's logits. The
 // decode kernels read an expert's rows for each of its row tiles' workgroups with all the batch's
 // tokens staged, and down once per token; the products read them once for the expert's tokens, but
 // need a selection and dispatch launch (11 us) and a combine (4 us). Whole layer, decode kernels / products, us:
-// BF16 (H 2816, 128 experts) T = 4 101 / 101, T = 5 122 / 109, T = 8 164 / 142, T = 16 307 / 207; MLX 4-bit
-// (H 2048, 256 experts) T = 4 52 / 55, T = 5 69 / 57, T = 8 95 / 67, T = 16 198 / 96; 8-bit T = 5 75 / 65,
-// T = 16 206 / 115. MXFP4 (H 2880): T = 8 91 / 132, T = 16 148 / 147, so never.
-int mid_tokens(const hh_moe_desc &d) { return d.quant == HH_QUANT_MXFP4 ? kSmallT + 1 : 5; }
+// BF16 (H 2816, I 704, 128 experts) T = 4 101 / 101, T = 5 122 / 109, T = 16 307 / 207; MLX 4-bit
+// (H 2048, I 512, 256 experts) T = 4 52 / 55, T = 5 69 / 57, T = 16 198 / 96; 8-bit T = 5 75 / 65. Small layers
+// do not earn the launches back: MLX 4-bit (H 1024, I 1024, 8 experts, K 1) T = 5 24 / 44, BF16 (H 512, I 256,
+// 8 experts, K 2) T = 8 21 / 28. The decode kernels' time grows with the elements read once per token and slot and
+// with the distinct experts; the line over both was fitted on 99 layers of H 384-4096, I 192-2048, 4 to 256 experts, at
+// T = 5, 8, 11, 16: the form it picks is 0.8 % slower than the faster one on average (worst 25 %).
+// MXFP4 (H 2880): T = 8 91 / 132, T = 16 148 / 147, so never.
+bool mid_batch(const hh_moe_desc &d, int T) {
+  if (T < 5 || d.quant == HH_QUANT_MXFP4) return false;
+  const double row = 3.0 * d.hidden;   // an expert's elements per intermediate
+  const double read = T * row * ((double)d.top_k * d.intermediate + d.shared_intermediate);
+  const double distinct = std::min(d.experts, T * d.top_k) + (d.shared_intermediate > 0);
+  if (d.quant == HH_QUANT_BF16) return read / 120e6 + distinct / 28 >= 1;
+  return d.quant == HH_QUANT_MLX4 ? read / 160e6 + distinct / 40 >= 1 : read / 100e6 + distinct / 48 >= 1;
+}
 
 // Experts must average this many tokens for the larger work items of a format (0: it has none).
 int large_item_tokens(const hh_moe_desc &d) {
@@ -196,7 +207,7 @@ int token_tile_nt(const hh_moe_desc &d, int T, bool compact = false) {
 // outputs), larger ones no 16-token items.
 Scratch plan(const hh_moe_desc &d, int T, bool compact = false) {
   Scratch s{};
-  s.products = T > kSmallT || (!compact && T >= mid_tokens(d));
+  s.products = T > kSmallT || (!compact && mid_batch(d, T));
   const int E = d.experts, K = d.top_k, H = d.hidden;
   const bool shared = d.shared_intermediate > 0;
   s.slots = K + (shared ? 1 : 0);
