@@ -187,6 +187,14 @@ int large_item_tokens(const hh_moe_desc &d) {
   return 0;
 }
 
+// Work items of `tokens` tokens that a call has, about: one of every expert that is reached, and half of the
+// experts one more that is partly filled.
+int64_t item_estimate(const hh_moe_desc &d, int T, int tokens) {
+  const int64_t A = (int64_t)T * d.top_k;
+  return std::max<int64_t>(std::min<int64_t>(d.experts, A), A / tokens + d.experts / 2) +
+         (d.shared_intermediate > 0 ? (T + tokens - 1) / tokens : 0);
+}
+
 int token_tile_nt(const hh_moe_desc &d, int T, bool compact = false) {
   // Prefill work items of 16·nt tokens (`compact`: no more items than 32-token ones): 32, or where
   // experts average enough tokens BF16 160 (the weight tile is then read once per 160 tokens), MXFP4 64
@@ -200,12 +208,21 @@ int token_tile_nt(const hh_moe_desc &d, int T, bool compact = false) {
       (int64_t)d.experts * ((2 * d.intermediate + 255) / 256) <= 3 * 256)
     return 1;
   if (!avg || (int64_t)T * d.top_k < (int64_t)avg * d.experts) return 2;
-  return d.quant == HH_QUANT_BF16 ? 10 : 4;
+  if (d.quant != HH_QUANT_BF16) return 4;
+  // BF16: the 160-token items' tiles (128 intermediates, 256 hidden rows) leave the chip idle where a call has few
+  // of them. The products' time goes with 1 / tasks then; the line is where 32-token items took over, us the layer,
+  // 160 / 32 (1 / (1/up + 1/down) of the tasks at 160): H 512, I 2880, 1 expert T = 300 128 / 62 (2), T = 2000 175 / 117
+  // (22); H 2048, I 1024, 8 experts K 2 T = 300 92 / 63 (32), T = 1000 127 / 127 (64), T = 2000 141 / 191 (116); H 2816,
+  // I 704, 16 experts K 8 T = 100 118 / 109 (62); H 512, I 192, 8 experts K 4 T = 2000 73 / 64 (54); H 384, I 1024,
+  // 16 experts K 8 T = 1000 115 / 125 (93); H 4096, I 1408, 8 experts K 2 T = 1000 194 / 285 (104).
+  const double items = (double)item_estimate(d, T, 160), up = items * ((d.intermediate + 127) / 128),
+               down = items * ((d.hidden + 255) / 256);
+  return compact || up * down >= 70 * (up + down) ? 10 : 2;
 }
 
 // `compact`: the least scratch: batches of at most kSmallT tokens take the decode kernels (no slot
-// outputs), larger ones no 16-token items.
-Scratch plan(const hh_moe_desc &d, int T, bool compact = false) {
+// outputs), larger ones no 16-token items. `nt`: work items of 16·nt tokens, whatever the call's own choice.
+Scratch plan(const hh_moe_desc &d, int T, bool compact = false, int nt = 0) {
   Scratch s{};
   s.products = T > kSmallT || (!compact && mid_batch(d, T));
   const int E = d.experts, K = d.top_k, H = d.hidden;
@@ -213,7 +230,7 @@ Scratch plan(const hh_moe_desc &d, int T, bool compact = false) {
   s.slots = K + (shared ? 1 : 0);
   s.positions = T * K + (shared ? T : 0);
   s.ldh = (int)align_up((size_t)std::max(d.intermediate, d.shared_intermediate), 64);
-  s.nt = token_tile_nt(d, T, compact);
+  s.nt = nt ? nt : token_tile_nt(d, T, compact);
   s.tile_tokens = 16 * s.nt;
   const int A = T * K;
   s.max_work = std::min(E, A) + (A + s.tile_tokens - 1) / s.tile_tokens +
@@ -260,26 +277,21 @@ Scratch plan(const hh_moe_desc &d, int T, bool compact = false) {
   return s;
 }
 
-// The largest batch up to T whose work items are the small ones (T where that is none): its plan, of
-// more items, can exceed that of a larger batch.
-int below_large_items(const hh_moe_desc &d, int T) {
-  const int64_t last = ((int64_t)large_item_tokens(d) * d.experts + d.top_k - 1) / d.top_k - 1;
-  return last < 1 ? T : (int)std::min<int64_t>(T, last);
-}
-
 // An arena that may not grow (a capture, or graphs that use it) and is too small for `bytes`: the call
 // takes the compact plan, which asks for no more than the decode kernels or 32-token items need.
 bool arena_short(const hh_ctx *ctx, size_t bytes) {
   return ctx->arena_bytes < bytes && (ctx->capturing || ctx->live_graphs > 0);
 }
 
-// Bytes that every batch of up to T tokens fits: `bytes(t, compact)` gives those of one batch.
-// Where the arena may not grow, a reservation asks for what its calls would then take.
+// Bytes that every batch of up to T tokens fits: those of T tokens (`bytes(scratch)`), the most over the
+// work items that a smaller batch may choose. Where the arena may not grow, a reservation asks for
+// what its calls would then take.
 template <class Bytes> size_t reserve_bytes(const hh_ctx *ctx, const hh_moe_desc &d, int T, Bytes bytes) {
-  size_t need[2] = {0, 0};   // as planned, compact
-  for (int t : {T, below_large_items(d, T)})
-    for (int c : {0, 1}) need[c] = std::max(need[c], bytes(t, c != 0));
-  return need[arena_short(ctx, need[0]) ? 1 : 0];
+  size_t need = 0;
+  for (int nt : {1, 2, 4}) {
+    if (nt == 2 || d.quant == HH_QUANT_MXFP4) need = std::max(need, bytes(plan(d, T, false, nt)));
+  }
+  return arena_short(ctx, need) ? std::max(bytes(plan(d, T, true)), bytes(plan(d, T, true, 2))) : need;
 }
 
 int ensure_arena(hh_ctx *ctx, size_t bytes) {
@@ -788,7 +800,7 @@ int hh_ctx_reserve(hh_ctx *ctx, const hh_moe_desc *d, int32_t max_tokens) {
   int rc = check_desc(d);
   if (rc) return rc;
   if (max_tokens <= 0 || max_tokens > kMaxTokens) return fail(HH_EINVAL, "max_tokens outside 1..65536");
-  return ensure_arena(ctx, reserve_bytes(ctx, *d, max_tokens, [&](int t, bool c) { return plan(*d, t, c).total; }));
+  return ensure_arena(ctx, reserve_bytes(ctx, *d, max_tokens, [](const Scratch &s) { return s.total; }));
 }
 
 int hh_moe_forward(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w,
@@ -1284,8 +1296,8 @@ int hh_runner_reserve(hh_runner *r, int32_t max_tokens) {
   for (const hh_runner::Layer &L : r->layers) {
     if (!L.set) return fail(HH_EINVAL, "a layer of the runner is not set");
     const bool gemma = L.norms.post_expert_norm != nullptr;
-    need = std::max(need, reserve_bytes(r->ctx, L.desc, max_tokens, [&](int t, bool c) {
-                      return block_plan(L.desc, plan(L.desc, t, c), t, gemma).total;
+    need = std::max(need, reserve_bytes(r->ctx, L.desc, max_tokens, [&](const Scratch &s) {
+                      return block_plan(L.desc, s, max_tokens, gemma).total;
                     }));
   }
   return ensure_arena(r->ctx, need);

@@ -28,8 +28,10 @@ CASES = {
     "mlx4_decode_7": (MLX4.replace(hidden=320, intermediate=192, shared_intermediate=0, experts=300, top_k=8), 7),
     "bf16_32_small": (BF16.replace(hidden=64, intermediate=64), 17),      # one stage
     "bf16_32_ragged": (BF16.replace(hidden=192, intermediate=320), 59),   # 39 an expert: two items of 32
-    "bf16_160_edge": (BF16.replace(hidden=192, intermediate=320), 60),    # 40 an expert: items of 160
-    "bf16_160_two": (BF16.replace(hidden=832, intermediate=192), 300),    # 200 an expert: 160 + 40
+    "bf16_160_edge": (BF16.replace(hidden=192, intermediate=320), 60),    # 40 an expert, too few tasks for items of 160
+    "bf16_160_two": (BF16.replace(hidden=832, intermediate=192), 300),
+    "bf16_160": (BF16.replace(hidden=832, intermediate=320, experts=48), 960),      # 40 an expert: items of 160
+    "bf16_160_over": (BF16.replace(hidden=832, intermediate=320, experts=24), 2500),   # 208 an expert: 160 + 48
     "mlx4_one_group": (MLX4.replace(hidden=64, intermediate=64, shared_intermediate=64), 17),
     "mlx4_odd_groups": (MLX4.replace(hidden=320, intermediate=192, shared_intermediate=320), 100),
     "mlx4_even_groups": (MLX4.replace(hidden=640, intermediate=384, shared_intermediate=0), 49),
