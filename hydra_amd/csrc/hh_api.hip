@@ -201,12 +201,22 @@ int token_tile_nt(const hh_moe_desc &d, int T, bool compact = false) {
   // for the gate-up (without a shared expert; rows below 1024 columns: not measured), whose down product
   // runs the same segments as 32-token items (Scratch::half_down).
   const int avg = large_item_tokens(d);
-  // MXFP4, few tokens an expert and few experts: 16-token items let three workgroups share a compute unit (50 KB
-  // of LDS each), and the gate-up's 256-row tiles of every expert then run at once on 256 of them. 32 experts
-  // (736 tasks) T = 45: 168 -> 156 us the layer; 128 experts with a Zipf load T = 128: 210 -> 224.
-  if (!compact && d.quant == HH_QUANT_MXFP4 && (int64_t)T * d.top_k < 8 * (int64_t)d.experts &&
-      (int64_t)d.experts * ((2 * d.intermediate + 255) / 256) <= 3 * 256)
-    return 1;
+  // MXFP4: 16-token items let three gate-up workgroups share a compute unit (50 KB of LDS each).
+  // With few tokens an expert and few experts the gate-up's 256-row tiles of every expert then run at once on
+  // 256 of them: 32 experts (736 tasks) T = 45: 168 -> 156 us the layer; 128 experts with a Zipf load
+  // T = 128: 210 -> 224. With more tokens they pay while their tasks (`tasks(16)`) still run at once, and
+  // 32-token items before 64-token ones likewise; us the layer with items of 16 / 32 / 64 tokens: 1 expert of
+  // H 4096, I 2880 T = 100 67 / 83 / 100 (138 tasks of 16 tokens), T = 300 82 / 93 / 104 (414), T = 1000 173 / 140 / 134
+  // (1426); 4 experts of H 1536, I 704 (K 1) T = 300 41 / 47 / 55 (120); 8 experts of H 4096, I 1536 (K 4) T = 100
+  // 78 / 79 / 94 (348; 192 of 32), T = 200 105 / 93 / 101 (648; 348), T = 300 128 / 133 / 121 (948; 492); 8 experts of
+  // H = I = 2880 (K 2) T = 200 92 / 89 / 97 (667; 368).
+  if (d.quant == HH_QUANT_MXFP4 && !compact) {
+    const int64_t tiles = (2 * d.intermediate + 255) / 256;
+    auto tasks = [&](int tokens) { return item_estimate(d, T, tokens) * tiles; };
+    if ((int64_t)T * d.top_k < 8 * (int64_t)d.experts && d.experts * tiles <= 3 * 256) return 1;
+    if (tasks(16) <= 600) return 1;
+    if (tasks(32) <= 400) return 2;
+  }
   if (!avg || (int64_t)T * d.top_k < (int64_t)avg * d.experts) return 2;
   if (d.quant != HH_QUANT_BF16) return 4;
   // BF16: the 160-token items' tiles (128 intermediates, 256 hidden rows) leave the chip idle where a call has few

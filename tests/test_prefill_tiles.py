@@ -37,9 +37,13 @@ CASES = {
     "mlx4_even_groups": (MLX4.replace(hidden=640, intermediate=384, shared_intermediate=0), 49),
     "mlx8_one_group": (MLX4.replace(quant=F.QUANT_MLX8, hidden=64, intermediate=64, shared_intermediate=0), 50),
     "mx_half_stage": (MX.replace(hidden=64, intermediate=64), 17),           # one stage of 64 columns
-    "mx_ragged": (MX.replace(hidden=192, intermediate=320), 60),             # 40 an expert: two items of 32
+    "mx_ragged": (MX.replace(hidden=192, intermediate=320), 60),             # 40 an expert, few tasks: items of 16
+    "mx_32": (MX.replace(hidden=192, intermediate=448, experts=256, top_k=4), 60),   # items of 32
+    "mx_32_full": (MX.replace(hidden=192, intermediate=832, experts=40, top_k=8), 300),   # 60 an expert: items of 32
     "mx_16": (MX.replace(hidden=192, intermediate=320, experts=8, top_k=1), 60),   # 16-token items, a skewed load
-    "mx_64": (MX.replace(hidden=1088, intermediate=1024, experts=2, top_k=1), 150),   # 64-token gate-up items
+    "mx_16_full": (MX.replace(hidden=1088, intermediate=1024, experts=2, top_k=1), 150),   # 75 an expert: items of 16
+    "mx_64": (MX.replace(hidden=1088, intermediate=1024, experts=64, top_k=1), 1100),      # 64-token gate-up items
+    "mx_32_long": (MX.replace(hidden=1088, intermediate=1024, experts=8, top_k=4), 300),   # 150 an expert: items of 32
     "mx_shared": (MX.replace(hidden=448, intermediate=192, shared_intermediate=320, expert_bias=0), 90),
     "mlx8_odd_groups": (MLX4.replace(quant=F.QUANT_MLX8, hidden=448, intermediate=320, shared_intermediate=192), 70),
 }
