@@ -709,6 +709,8 @@ template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int 
   }
   return hipSuccess;
 }
+// Tasks of a launch at most, with `rows` output rows each.
+static int64_t tasks(const GemmArgs &a, int out, int rows) { return (int64_t)a.max_work * ((out + rows - 1) / rows); }
 template <int PH> static int out_rows(const GemmArgs &a) {
   return PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
 }
@@ -730,7 +732,15 @@ template <int PH, int NT> static hipError_t launch_mx(const GemmArgs &a, hipStre
 // (nt 4), MLX items 32.
 hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
   const bool up = phase == PH_UP;
-  if (quant == Q_MLX4) return up ? launch_mlx<PH_UP, 4, 2, 2>(a, s, tm) : launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
+  if (quant == Q_MLX4) {
+    // Tiles of 64 rows where even they do not fill the two workgroups a compute unit holds (tasks counted at the
+    // wide tiles, of twice and three times the rows). Gate-up, us, wide / 64 (tasks): 1 expert of H 2880, I 512 T = 100
+    // 40 / 28 (20), 16 experts of H 2048, I 768 (K 4) T = 100 29 / 21 (174), 256 experts of H 2048, I 512 (K 8)
+    // T = 8 26 / 24 (268), T = 12 36 / 37 (400). Down: 4 experts of H 2048, I 1536 (K 2) T = 100 24 / 17 (121), T = 300
+    // 24 / 32 (253).
+    if (up) return tasks(a, a.grp[0].inter, 128) <= 300 ? launch_mlx<PH_UP, 4, 1, 2>(a, s, tm) : launch_mlx<PH_UP, 4, 2, 2>(a, s, tm);
+    return tasks(a, a.hidden, 192) <= 130 ? launch_mlx<PH_DOWN, 4, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
+  }
   if (quant == Q_MLX8) return up ? launch_mlx<PH_UP, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
   if (quant == Q_MXFP4) {
     if (nt == 1) return up ? launch_mx<PH_UP, 1>(a, s, tm) : launch_mx<PH_DOWN, 1>(a, s, tm);

@@ -35,6 +35,9 @@ CASES = {
     "mlx4_one_group": (MLX4.replace(hidden=64, intermediate=64, shared_intermediate=64), 17),
     "mlx4_odd_groups": (MLX4.replace(hidden=320, intermediate=192, shared_intermediate=320), 100),
     "mlx4_even_groups": (MLX4.replace(hidden=640, intermediate=384, shared_intermediate=0), 49),
+    # tiles of 64 rows for the few tasks of the layers above, wide ones for these (ragged: 320 of 3 x 128, 832 of 5 x 192)
+    "mlx4_wide": (MLX4.replace(hidden=832, intermediate=320, shared_intermediate=192, experts=128, top_k=8), 40),
+    "mlx4_wide_odd": (MLX4.replace(hidden=320, intermediate=832, shared_intermediate=0, experts=128, top_k=4), 130),
     "mlx8_one_group": (MLX4.replace(quant=F.QUANT_MLX8, hidden=64, intermediate=64, shared_intermediate=0), 50),
     "mx_half_stage": (MX.replace(hidden=64, intermediate=64), 17),           # one stage of 64 columns
     "mx_ragged": (MX.replace(hidden=192, intermediate=320), 60),             # 40 an expert, few tasks: items of 16
