@@ -63,8 +63,9 @@ __device__ __forceinline__ float wave_sum(float v) {
 // tile's rows are asked for first and the queries' fragments are formed, straight from global
 // memory, while they travel; the waves' outputs merge in the LDS that staged their values. Whole call, 64 / 8
 // heads of 64, before -> now: 32768 keys 21.1 -> 18.4 us (3.7 TB/s), 131072 68.6 -> 66.3, 4096 8.6 ->
-// 8.4; heads of 128, 32768 keys 52.9 -> 45.8. Three waves per SIMD: with two (205 registers) 19.8 at 32768 keys,
-// with four (128 registers, 29 spilled) 23.6.
+// 8.4; heads of 128, 32768 keys 52.9 -> 45.8 (before the merge below). Heads of 64: three waves per SIMD, with two (205
+// registers) 19.8 at 32768 keys, with four (128 registers, 29 spilled) 23.6; heads of 128 take two, and all of
+// their 256 registers.
 template <int D>
 __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_split_kernel(AttnArgs a) {
   warm_kernargs<sizeof(AttnArgs)>();
@@ -235,16 +236,20 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_split_kernel(AttnAr
   }
 }
 
-// One workgroup of kMergeW waves per query head: each wave forms the maximum and the denominator (its lanes
-// take chunks) and one chunk's weight in kMergeW goes to LDS; wave w then sums chunks w, w + kMergeW, ... of every
-// dimension, sixteen loads in flight, and the waves' sums are added in wave order. (One wave summing all the
-// chunks eight at a time: 5.1 us at 128 chunks, now 4.8, most of it the launch and the first loads.)
+// One workgroup of kMergeW waves per query head. Its threads take the chunk states in one round of loads (up to 64
+// chunks every wave all of them, so that no barrier is needed for them): the waves' maxima and denominators meet in
+// LDS, added in wave order, and every chunk's weight goes there; wave w then sums chunks w, w + kMergeW, ... of every
+// dimension, sixteen loads in flight, and the waves' sums are added in wave order. Bound by the rounds of loads
+// and the barriers between them. Whole call, 8 / 1 heads of 64, 512 / 976 chunks: 27.1 / 57.0 us with every wave walking
+// all the chunk states, 24.4 / 49.3 with one wave for the whole head, now 23.3 / 49.4; 64 / 8 heads, 128 chunks 18.5,
+// 20.9, now 18.0.
 constexpr int kMergeW = 8;
 template <int D>
 __global__ __launch_bounds__(64 * kMergeW) void attn_merge_kernel(AttnArgs a) {
   warm_kernargs<sizeof(AttnArgs)>();
   __shared__ float s_f[kAttnMaxChunks];
   __shared__ float s_o[kMergeW][D];
+  __shared__ float s_g[kMergeW], s_den[kMergeW];
   const int h = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const float *pm = a.pmax + (size_t)h * a.chunks, *pd = a.pden + (size_t)h * a.chunks;
   const float *po = a.pout + (size_t)h * a.chunks * D;
@@ -258,14 +263,43 @@ __global__ __launch_bounds__(64 * kMergeW) void attn_merge_kernel(AttnArgs a) {
       for (int r = 0; r < R; ++r) v[u][r] = po[(size_t)min(c0 + kMergeW * u, a.chunks - 1) * D + lane + 64 * r];
   };
   load(wave);
+  constexpr int NT = 64 * kMergeW, PC = kAttnMaxChunks / NT;
+  const bool few = a.chunks <= 64;
+  const int c_first = few ? lane : (int)threadIdx.x;
+  float m[PC], d[PC], e[PC];
   float g = -INFINITY;
-  for (int c = lane; c < a.chunks; c += 64) g = fmaxf(g, pm[c]);
+#pragma unroll
+  for (int i = 0; i < PC; ++i) {
+    const int c = c_first + NT * i;
+    m[i] = c < a.chunks ? pm[c] : -INFINITY;
+    d[i] = c < a.chunks ? pd[c] : 0.f;
+    g = fmaxf(g, m[i]);
+  }
   g = wave_max(g);
+  if (!few) {
+    if (lane == 0) s_g[wave] = g;
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kMergeW; ++w) g = fmaxf(g, s_g[w]);
+  }
   float den = 0.f;
-  for (int c = lane; c < a.chunks; c += 64) den += pd[c] * __expf(pm[c] - g);
+#pragma unroll
+  for (int i = 0; i < PC; ++i) {
+    e[i] = c_first + NT * i < a.chunks ? __expf(m[i] - g) : 0.f;
+    den += d[i] * e[i];
+  }
   den = wave_sum(den);
+  if (!few) {
+    if (lane == 0) s_den[wave] = den;
+    __syncthreads();
+    den = s_den[0];
+#pragma unroll
+    for (int w = 1; w < kMergeW; ++w) den += s_den[w];
+  }
   const float inv = 1.f / den;
-  for (int c = threadIdx.x; c < a.chunks; c += 64 * kMergeW) s_f[c] = __expf(pm[c] - g) * inv;
+  if (!few || wave == 0)
+#pragma unroll
+    for (int i = 0; i < PC; ++i) s_f[c_first + NT * i] = e[i] * inv;
   __syncthreads();
   float sum[R];
 #pragma unroll

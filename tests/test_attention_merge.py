@@ -7,7 +7,7 @@ from oracle import oracle as O
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("qh,d,keys", [(8, 64, 33100), (5, 128, 70000)])   # 129 and 273 chunks
+@pytest.mark.parametrize("qh,d,keys", [(8, 64, 33100), (5, 128, 70000), (2, 64, 131072), (1, 64, 262400)])   # 129, 273, 512, 1024 chunks
 def test_attention_many_chunks(qh, d, keys):
     import torch
     from hydra_amd import synth
