@@ -1153,17 +1153,23 @@ int hh_expert_gemm(hh_ctx *ctx, const hh_matrix *m, const float *x, int32_t T, f
   if (T == 0) return HH_OK;
   HH_HIP(hipSetDevice(ctx->device));
   // Scratch: the activation operand of T rows, routing (topk, weights, order) and the work list.
-  const int tile = 32;
+  // Work items of 32 tokens; MXFP4 16 while their tasks (256 rows each) run at once: a stage of the K loop is then
+  // shorter, and its latency is all there is. us with 32 / 16: 4096 x 4096 T = 17 40 / 29, T = 300 45 / 38 (304 tasks),
+  // T = 1000 60 / 59 (1008); 512 x 2880 T = 2000 39 / 31 (250); 64 x 256 T = 8000 15 / 17 (500).
+  const bool small = q == HH_QUANT_MXFP4 && (int64_t)((T + 15) / 16) * ((R + 255) / 256) <= 400;
+  int tile = small ? 16 : 32;
   const size_t ldh = align_up((size_t)Kc, 64), hld = align_up(ldh, 512);
   const bool mx = q == HH_QUANT_MXFP4;
-  const int items = (T + tile - 1) / tile;
   size_t c = 0;
   auto take = [&](size_t bytes) { size_t o = c; c = align_up(c + bytes, 256); return o; };
   const size_t o_hi = take(mx ? 0 : 2 * (size_t)T * ldh), o_lo = take(mx ? 0 : 2 * (size_t)T * ldh);
   const size_t o_hq = take(mx ? (size_t)T * hh::NTH * hld : 0), o_hs = take(mx ? (size_t)T * hh::NTH * (hld / 32) : 0);
   const size_t o_w = take(4 * (size_t)T), o_k = take(4 * (size_t)T), o_ord = take(4 * (size_t)T);
-  const size_t o_work = take(sizeof(int4) * (size_t)items), o_nw = take(4);
-  int rc = ensure_arena(ctx, c);
+  const size_t o_nw = take(4), o_work = c;   // the work list last: the one part that depends on `tile`
+  auto total = [&](int t) { return align_up(c + sizeof(int4) * (size_t)((T + t - 1) / t), 256); };
+  if (arena_short(ctx, total(tile))) tile = 32;
+  const int items = (T + tile - 1) / tile;
+  int rc = ensure_arena(ctx, total(tile));
   if (rc) return rc;
   uint8_t *base = ctx->arena;
   // The matrix as the down tensors of a one-expert blob: offsets from the lowest pointer.
@@ -1214,7 +1220,7 @@ int hh_expert_gemm(hh_ctx *ctx, const hh_matrix *m, const float *x, int32_t T, f
     HH_HIP(hh::launch_down_small(q, g, topk, T, ctx->stream, hh::Timing{}));
   } else {
     g.max_work = items;
-    HH_HIP(hh::launch_gemm(1, q, 2, g, ctx->stream, hh::Timing{}));
+    HH_HIP(hh::launch_gemm(1, q, tile / 16, g, ctx->stream, hh::Timing{}));
   }
   ctx->dispatches += 2;
   return HH_OK;

@@ -119,6 +119,34 @@ def test_projection_against_oracle(name):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T", [500, 560])   # 384 tasks of 16-token items; 32-token items
+def test_mxfp4_projection_item_sizes(T):
+    """gemm row t equals gemv of x[t] bit for bit with either size of work items."""
+    import torch
+    from hydra_amd._lib import MatrixC, check, lib
+    from hydra_amd.layer import Context, to_device
+    print(f"[gpu] projection items T={T}", flush=True)
+    m = make_matrix(F.QUANT_MXFP4, 2880, 192, seed=8, bias=True)
+    w, sc, bias = (to_device(m[k], "cuda:0") for k in ("weights", "scales", "bias"))
+    p = lambda t: C.c_void_p(t.data_ptr())
+    mc = MatrixC(F.QUANT_MXFP4, 2880, 192, 64, p(w), p(sc), None, p(bias))
+    x = torch.from_numpy(np.random.default_rng(9).standard_normal((T, 192)).astype(np.float32)).to("cuda:0")
+    y = torch.full((T, 2880), float("nan"), dtype=torch.float32, device="cuda:0")
+    y1 = torch.empty(2880, dtype=torch.float32, device="cuda:0")
+    ctx = Context(0)
+    try:
+        torch.cuda.synchronize()
+        check(lib().hh_expert_gemm(ctx.handle, C.byref(mc), p(x), T, p(y)))
+        for t in (0, 15, 16, T // 2, T - 1):
+            check(lib().hh_expert_gemv(ctx.handle, C.byref(mc), p(x[t]), p(y1)))
+            ctx.synchronize()
+            assert torch.equal(y[t], y1)
+        assert torch.isfinite(y).all()
+    finally:
+        ctx.close()
+
+
+@pytest.mark.gpu
 def test_combine_bit_exact():
     import torch
     from hydra_amd._lib import check, lib
