@@ -737,11 +737,21 @@ hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStrea
     // wide tiles, of twice and three times the rows). Gate-up, us, wide / 64 (tasks): 1 expert of H 2880, I 512 T = 100
     // 40 / 28 (20), 16 experts of H 2048, I 768 (K 4) T = 100 29 / 21 (174), 256 experts of H 2048, I 512 (K 8)
     // T = 8 26 / 24 (268), T = 12 36 / 37 (400). Down: 4 experts of H 2048, I 1536 (K 2) T = 100 24 / 17 (121), T = 300
-    // 24 / 32 (253).
+    // 24 / 32 (253). Down tiles of 128 rows where those of 192 would be a tenth padding, with up to two tasks a
+    // compute unit: 512 x 2880 T = 2000 55 / 48 (189), 1024 x 1024 T = 2000 33 / 30 (378), T = 8000 77 / 82 (1500).
     if (up) return tasks(a, a.grp[0].inter, 128) <= 300 ? launch_mlx<PH_UP, 4, 1, 2>(a, s, tm) : launch_mlx<PH_UP, 4, 2, 2>(a, s, tm);
-    return tasks(a, a.hidden, 192) <= 130 ? launch_mlx<PH_DOWN, 4, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
+    const int64_t wide = tasks(a, a.hidden, 192);
+    if (wide <= 130) return launch_mlx<PH_DOWN, 4, 1, 2>(a, s, tm);
+    const int pad128 = (a.hidden + 127) / 128 * 128, pad192 = (a.hidden + 191) / 192 * 192;
+    if (wide <= 512 && 10 * pad192 > 11 * pad128) return launch_mlx<PH_DOWN, 4, 2, 2>(a, s, tm);
+    return launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
   }
-  if (quant == Q_MLX8) return up ? launch_mlx<PH_UP, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
+  if (quant == Q_MLX8) {
+    // The same for 8-bit down tiles: 4 experts of H 2048, I 1536 (K 2) T = 40 the layer 60 / 55 (tasks of 128 rows: 112),
+    // 1 expert of H 2880, I 512 T = 300 61 / 65 (253).
+    if (up) return launch_mlx<PH_UP, 8, 1, 2>(a, s, tm);
+    return tasks(a, a.hidden, 128) <= 200 ? launch_mlx<PH_DOWN, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
+  }
   if (quant == Q_MXFP4) {
     if (nt == 1) return up ? launch_mx<PH_UP, 1>(a, s, tm) : launch_mx<PH_DOWN, 1>(a, s, tm);
     if (up) return nt == 4 ? launch_mx<PH_UP, 4>(a, s, tm) : launch_mx<PH_UP, 2>(a, s, tm);

@@ -38,6 +38,8 @@ CASES = {
     # tiles of 64 rows for the few tasks of the layers above, wide ones for these (ragged: 320 of 3 x 128, 832 of 5 x 192)
     "mlx4_wide": (MLX4.replace(hidden=832, intermediate=320, shared_intermediate=192, experts=128, top_k=8), 40),
     "mlx4_wide_odd": (MLX4.replace(hidden=320, intermediate=832, shared_intermediate=0, experts=128, top_k=4), 130),
+    "mlx4_down_128": (MLX4.replace(hidden=256, intermediate=192, shared_intermediate=64, experts=80, top_k=2), 70),   # 176 tasks, 192-row tiles a third padding
+    "mlx8_wide": (MLX4.replace(quant=F.QUANT_MLX8, hidden=320, intermediate=192, shared_intermediate=64, experts=80, top_k=2), 70),   # 8-bit down tiles of 128 rows
     "mlx8_one_group": (MLX4.replace(quant=F.QUANT_MLX8, hidden=64, intermediate=64, shared_intermediate=0), 50),
     "mx_half_stage": (MX.replace(hidden=64, intermediate=64), 17),           # one stage of 64 columns
     "mx_ragged": (MX.replace(hidden=192, intermediate=320), 60),             # 40 an expert, few tasks: items of 16
