@@ -59,6 +59,9 @@ __device__ __forceinline__ float wave_sum(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// The outputs that take over the LDS of a wave's value tile (halves): a float that may alias them.
+typedef float __attribute__((may_alias)) outputs_t;
+
 // One tile per wave up to 32768 keys (1024 workgroups), so the kernel is a chain of latencies: the
 // tile's rows are asked for first and the queries' fragments are formed, straight from global
 // memory, while they travel; the waves' outputs merge in the LDS that staged their values. Whole call, 64 / 8
@@ -206,7 +209,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_split_kernel(AttnAr
     if (base < last) load_tile(base);
   }
   // The waves' states merge in LDS.
-  float *so = (float *)sv;
+  outputs_t *so = (outputs_t *)sv;
   if (lane < QM) {   // lane h: head h's state
     s_m[wave][lane] = M;
     s_l[wave][lane] = L;
@@ -225,7 +228,7 @@ __global__ __launch_bounds__(256, D == 64 ? 3 : 2) void attn_split_kernel(AttnAr
     for (int w = 0; w < 4; ++w) {
       const float f = __expf(s_m[w][h] - gm);
       den += s_l[w][h] * f;
-      o += ((const float *)s_v[w])[h * D + c] * f;
+      o += ((const outputs_t *)s_v[w])[h * D + c] * f;
     }
     const size_t slot = (size_t)(h0 + h) * a.chunks + chunk;
     a.pout[slot * D + c] = o;
