@@ -22,8 +22,8 @@ CASES = {
     "mxfp4-shared": (F.MoEDesc(hidden=640, intermediate=128, experts=6, top_k=2, quant=F.QUANT_MXFP4,
                                activation=F.ACT_SWIGLU_OAI, router=F.ROUTER_SOFTMAX_TOPK_RENORM,
                                shared_intermediate=128, expert_bias=1), [1, 2, 5]),
-    "qwen-q4": (F.QWEN_35B_A3B_Q4, [1, 24]),
-    "gemma-bf16": (F.GEMMA_BF16, [1, 40]),
+    "qwen-q4": (F.QWEN_35B_A3B_Q4, [1, 8, 24]),   # 8: the grouped products after the decode router
+    "gemma-bf16": (F.GEMMA_BF16, [1, 8, 40]),
 }
 
 

@@ -21,30 +21,34 @@ STACK = [
 ]
 
 
+# Experts enough for the MLX and BF16 layers' batches of 5 to 16 tokens to take the grouped products.
+MANY = [STACK[0]] + [d.replace(experts=64, top_k=8) for d in STACK[1:]]
+
+
 @pytest.mark.gpu
-@pytest.mark.parametrize("T", [1, 40])
-def test_graph_replays_equal_eager_calls(T):
+@pytest.mark.parametrize("T,stack,launches", [(1, STACK, 9), (40, STACK, 18), (8, STACK, 9), (8, MANY, 13)],
+                         ids=["1", "40", "8", "8-many"])
+def test_graph_replays_equal_eager_calls(T, stack, launches):
     import torch
     from hydra_amd.layer import Context, MoELayer, to_device
     print(f"[gpu] graph stack T={T}", flush=True)
     ctx = Context(0)
     try:
-        layers = [MoELayer(synth.make_layer(d, seed=50 + i), ctx) for i, d in enumerate(STACK)]
-        for d in STACK:
+        layers = [MoELayer(synth.make_layer(d, seed=50 + i), ctx) for i, d in enumerate(stack)]
+        for d in stack:
             ctx.reserve(d, T)
         dev = "cuda:0"
-        xs = [torch.empty((T, d.hidden), dtype=torch.int16, device=dev) for d in STACK]
-        ys = [torch.empty((T, d.hidden), dtype=torch.float32, device=dev) for d in STACK]
-        ids = [torch.empty((T, d.top_k), dtype=torch.int32, device=dev) for d in STACK]
-        ws = [torch.empty((T, d.top_k), dtype=torch.float32, device=dev) for d in STACK]
+        xs = [torch.empty((T, d.hidden), dtype=torch.int16, device=dev) for d in stack]
+        ys = [torch.empty((T, d.hidden), dtype=torch.float32, device=dev) for d in stack]
+        ids = [torch.empty((T, d.top_k), dtype=torch.int32, device=dev) for d in stack]
+        ws = [torch.empty((T, d.top_k), dtype=torch.float32, device=dev) for d in stack]
         torch.cuda.synchronize()
         before = ctx.dispatches
         graph = ctx.capture(lambda: [l.forward_into(x, y, i, w)
                                      for l, x, y, i, w in zip(layers, xs, ys, ids, ws)])
         assert ctx.dispatches == before            # recording runs nothing
-        per_replay = None
         for rep in range(3):
-            host = [synth.make_tokens(d.hidden, T, seed=700 + 10 * rep + j) for j, d in enumerate(STACK)]
+            host = [synth.make_tokens(d.hidden, T, seed=700 + 10 * rep + j) for j, d in enumerate(stack)]
             eager = [l.forward(h) for l, h in zip(layers, host)]   # eager work between replays
             for x, h in zip(xs, host):
                 x.copy_(to_device(h, dev))
@@ -56,8 +60,7 @@ def test_graph_replays_equal_eager_calls(T):
             d0 = ctx.dispatches
             graph.launch()
             ctx.synchronize()
-            per_replay = ctx.dispatches - d0 if per_replay is None else per_replay
-            assert ctx.dispatches - d0 == per_replay > 0
+            assert ctx.dispatches - d0 == launches
             for (ey, ei, ew), y, i, w in zip(eager, ys, ids, ws):
                 assert torch.equal(i, ei) and torch.equal(w, ew) and torch.equal(y, ey), f"replay {rep}"
         graph.close()

@@ -26,6 +26,9 @@ DESCS = [
     (F.MoEDesc(hidden=H, intermediate=128, experts=5, top_k=2, quant=F.QUANT_BF16,
                activation=F.ACT_GELU_TANH, router=F.ROUTER_GEMMA), 0),
 ]
+# Experts enough for the MLX (both routers) and BF16 layers' batches of 5 to 16 tokens to take the grouped products.
+MANY = [DESCS[0]] + [(d.replace(experts=64, top_k=8), rb) for d, rb in DESCS[1:]] + \
+       [(DESCS[1][0].replace(experts=64, top_k=8), 0)]
 
 
 def _norms(rng, gemma):
@@ -37,8 +40,8 @@ def _norms(rng, gemma):
     return n
 
 
-@pytest.mark.parametrize("T", [1, 24])
-def test_runner_equals_calls_one_by_one(T):
+@pytest.mark.parametrize("T,descs", [(1, DESCS), (24, DESCS), (8, DESCS), (8, MANY)], ids=["1", "24", "8", "8-many"])
+def test_runner_equals_calls_one_by_one(T, descs):
     import torch
     from hydra_amd._lib import MatrixC, check, lib
     from hydra_amd.layer import Context, MoELayer, Runner, to_device
@@ -49,7 +52,7 @@ def test_runner_equals_calls_one_by_one(T):
         rng = np.random.default_rng(71)
         layers, mats, probes = [], [], []
         dense = torch.zeros((T, H), dtype=torch.float32, device=dev)
-        for i, (d, rb) in enumerate(DESCS):
+        for i, (d, rb) in enumerate(descs):
             ml = MoELayer(synth.make_layer(d, seed=72 + i, router_bits=rb), ctx)
             gemma = d.router == F.ROUTER_GEMMA
             norms = {k: (v if k == "eps" else to_device(v, dev)) for k, v in _norms(rng, gemma).items()}
@@ -87,7 +90,7 @@ def test_runner_equals_calls_one_by_one(T):
         seen = []
         runner.forward(hid2, hook=lambda l: (seen.append(l), hook(l, hid2)))
         ctx.synchronize()
-        assert seen == [0, 1, 2]
+        assert seen == list(range(len(descs)))
         for a, b in zip(snapshot(hid2), ref):
             assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
         # one graph for the stack, replayed on new inputs
