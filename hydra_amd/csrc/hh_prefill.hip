@@ -466,8 +466,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // Before (persistent kernels with loader waves): T = 2048 483 / 368, T = 512 222 / 148, and 102 / 55 at
 // T = 45 of the 32-expert layer, now 405 / 279, 183 / 116 and 92 / 49.
 // Gate-up items hold 64 tokens where experts average 16 or more (T = 2048 405, with 32 tokens 480;
-// T = 512 183 against 199), 16 where few experts have few tokens each (three workgroups per compute
-// unit: 92 -> 78 at T = 45), down items 32 (three terms: a 64-token stage leaves one slot).
+// T = 512 183 against 199), 16 where few experts have few tokens each (three gate-up workgroups per
+// compute unit: 92 -> 78 at T = 45; the down product's three terms leave room for two), down items otherwise 32
+// (a 64-token stage leaves one slot).
 template <int PH, int NT_> struct Mx {
   static constexpr int NT = NT_, NTERM = PH == PH_UP ? NTX : NTH;
   static constexpr int NJ = 4;                               // 16-row tiles per wave, their 1 KiB loads per stage
@@ -479,11 +480,13 @@ template <int PH, int NT_> struct Mx {
   // Scales of three stages: 16 bytes of each weight row, then of each operand row; two such sets.
   static constexpr int OFF_Q = 2 * STAGE, QB = 4096, QUAD = QB + BSL * 1024;
   static constexpr int LDS = OFF_Q + 2 * QUAD;
+  static constexpr int WGS = LDS <= 160 * 1024 / 3 ? 3 : 2;   // workgroups per compute unit
   static_assert(BSL <= 4 && LDS <= 80 * 1024, "two workgroups per compute unit");
 };
+static_assert(Mx<PH_UP, 1>::WGS == 3 && Mx<PH_DOWN, 1>::WGS == 2, "16-token items: 50 KB, and 54 KB with three terms");
 
 template <int PH, int NT_>
-__global__ __launch_bounds__(256, NT_ == 1 ? 3 : 2) void prefill_mx(GemmArgs a) {
+__global__ __launch_bounds__(256, (Mx<PH, NT_>::WGS)) void prefill_mx(GemmArgs a) {
   using C = Mx<PH, NT_>;
   constexpr int NT = C::NT, NTERM = C::NTERM, NJ = C::NJ, TOK = C::TOK;
   extern __shared__ __align__(16) uint8_t lds[];
