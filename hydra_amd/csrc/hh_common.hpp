@@ -241,11 +241,12 @@ struct GemmArgs {
   int32_t quant, act, expert_bias, group;
   float alpha, limit;
   int32_t ldh;                  // row stride (elements) of h_hi / h_lo; multiple of 64
-  int32_t max_work;             // most work items (host); prefill kernels: the launch's first task
+  int32_t max_work;             // grouped products, on the host: most work items
+  int32_t first_task;           // grouped products: the launch's first task
   int32_t row_tiles;            // workgroup row tiles along the output dimension
-  int32_t reserved;
+  int32_t tokens;               // decode down product: tokens of the batch
   const uint16_t *x;            // bf16 [T][H]
-  const int32_t *order;         // [positions] slot id (t·slots + r) of each permuted position (T > 16)
+  const int32_t *order;         // [positions] slot id (t·slots + r) of each permuted position (grouped products)
   const int4 *work;             // [max_work] {expert (E = shared), pos0, n, 0}
   const int32_t *n_work;        // device count of valid work items
   uint16_t *h_hi, *h_lo;        // bf16 [T·slots][ldh]: activation of each slot, hi + lo split
@@ -254,7 +255,7 @@ struct GemmArgs {
   uint8_t *hq, *hs;             // h: [T·slots][NTH][hld] bytes, scales [T·slots][NTH][hld/32]
   int32_t xld, hld;             // row lengths (multiples of 128)
   const float *slot_w;          // fp32 [T·slots] routing weight of each slot
-  float *slot_out;              // fp32 [T·slots][H] (T > 16)
+  float *slot_out;              // fp32 [T·slots][H] (grouped products)
   float *y;                     // fp32 [T][H] layer output (written directly by the decode path)
   const float *resid;           // fp32 [T][H] residual added to the mixture (y = resid + Σ slots), or null
 };

@@ -1,41 +1,40 @@
-// hh_gemm.hip — grouped expert products on gfx950 MFMA, shared by decode and prefill.
+// hh_gemm.hip — decode's expert products on gfx950 MFMA, and the combine of the grouped products (hh_prefill.hip).
 //
 // Two products per layer:
 //   PH_UP   : h[s][i] = act(gate_i · x_t + b, up_i · x_t + b) for every slot s = t·slots + r
-//             (token t, rank r; rank `top_k` is the shared expert), stored as bf16 hi + lo so
-//             the down product sees the fp32 activation to ~2^-17 relative;
+//             (token t, rank r; rank `top_k` is the shared expert), stored as bf16 hi + lo (MXFP4 layers:
+//             as three fp8 terms) so the down product sees the fp32 activation to ~2^-17 (2^-13) relative;
 //   PH_DOWN : slot value w(t, r) · (down_j · h[s] + b_j); the slots of a token are summed in rank
 //             order into y.
 //
-// Canonical arithmetic. Every output element (row j, slot s) is TWO accumulation chains over the
-// K dimension, summed at the end (acc_even + acc_odd): chain p takes the chunks c ≡ p (mod 2) in
-// increasing order, each chunk a fixed sequence of v_mfma_f32_16x16x32_bf16 steps (MXFP4/BF16:
+// Canonical arithmetic, shared with hh_prefill.hip. BF16 and MLX: every output element (row j, slot s) is TWO
+// accumulation chains over the K dimension, summed at the end (acc_even + acc_odd): chain p takes the chunks
+// c ≡ p (mod 2) in increasing order, each chunk a fixed sequence of v_mfma_f32_16x16x32_bf16 steps (BF16:
 // 128-column chunks, 4 steps; MLX: one 64-column affine group, 2 steps into a group partial P,
 // then acc = fma(s, P, acc), acc = fma(b, Σx, acc)). Two chains halve the dependent-MFMA latency
-// of a decode wave, which owns a single 16-row tile. Decode and prefill kernels differ only in
+// of a decode wave, which owns a single 16-row tile. MXFP4: one chain of v_mfma_scale_f32_16x16x128_f8f6f4 over the
+// 128-column chunks, the operand's terms of a chunk in order. Decode and grouped kernels differ only in
 // how rows and tokens are tiled over waves and how the B operand reaches the registers; each
 // output element sees the same MFMA sequence with the same operands, so a T-token call equals
 // T one-token calls bit for bit. No split-K across waves, no atomics.
 //
-// Kernels:
-//   up_small / down_small (T ≤ 16, decode): up_small selects the top-k itself from the exact
-//     fp64 logits (every workgroup redundantly, hh_select.hpp), takes the u-th distinct expert of
-//     the batch (in order of first appearance in the (token, rank) table), and computes 32
-//     intermediates of it for all its tokens: 4 waves = {gate, up} × 2 tiles of 16 rows, each
-//     wave issuing its whole weight stream at once (one 16-byte load per lane per chunk), the
-//     tokens' x rows staged in LDS. down_small computes 16 hidden rows of one token for all of
-//     its slots (one wave per slot) and sums them in rank order in the epilogue: no slot buffer,
-//     no combine launch.
-//   T > 16: hh_prefill.hip.
+// Kernels (T ≤ 16; on BF16 and MLX layers the batches that hh_api.hip:mid_batch leaves):
+//   up_small / up_small_mx select the top-k themselves from the exact fp64 logits (every workgroup
+//     redundantly, hh_select.hpp), take the u-th distinct expert of the batch (in order of first appearance in
+//     the (token, rank) table), and compute 16 (MXFP4: 32) intermediates of it for all its tokens, a wave's
+//     weight stream in flight at once or in a register ring, the tokens' x rows staged in LDS.
+//   down_small computes 16 hidden rows of one token for all of its slots (one wave per slot, or two) and
+//     sums them in rank order in the epilogue: no slot buffer, no combine launch.
+//   decode_mx runs the whole MXFP4 layer in one launch (opt-in).
 //
 // MFMA operand mapping (16x16x32, lane l, lane group g = l/16): A lane l supplies row l%16,
 // B lane l supplies token column l%16, each with 8 consecutive K values; D lane l holds rows
 // 4g..4g+3 of column l%16. The K slots are assigned per format:
-//   MXFP4, BF16: chunk c of 128 columns; MFMA step v∈0..3 takes lane group g's columns
-//                128c + 32g + 8v .. +8 (g's 16-byte MXFP4 block 4c+g, or its 64 bytes of bf16)
+//   BF16       : chunk c of 128 columns; step v∈0..3 takes lane group g's columns 128c + 32v + 8g .. +8
 //   MLX4/MLX8  : chunk c = affine group c (64 columns); step v∈0..1 takes columns
 //                64c + 16g + 8v .. +8, so both steps stay inside one group and the affine
 //                factorisation s·Σq·x + b·Σx applies per group.
+//   MXFP4      : see smfma (hh_mfma.hpp): lane group g's 16-byte block 4c + g.
 //
 // Reference kernels replaced: mxfp4_gemv_vectorized (mxfp4.metal:119), mxfp4_gemm_gathered /
 // mxfp4_gemm_tiled (batch.metal:96, tiled.metal:127), bf16_gemv (dense.metal:14),
@@ -521,8 +520,8 @@ __global__ __launch_bounds__(256 * TPW) void up_small(GemmArgs a, RouteArgs ra, 
     if (it == (int)blockIdx.x) HH_TR(1, 3);
     if (slot_of_part == 0 && l16 < ntok) {
       const int r = rank_of(s_idx, my_t, e, K, sh);
-      up_epilogue<FMT>(a, blob, grp, rb + 4 * g, my_t * S + r, sum_chains(acc[0][0], s_part[0][q][lane]),
-                       sum_chains(s_part[1][q][lane], s_part[2][q][lane]));
+      up_epilogue(a, rb + 4 * g, my_t * S + r, sum_chains(acc[0][0], s_part[0][q][lane]),
+                  sum_chains(s_part[1][q][lane], s_part[2][q][lane]));
     }
     if (it == (int)blockIdx.x) HH_TR(1, 4);
   }
@@ -560,7 +559,7 @@ __device__ __forceinline__ MxOps<NTERM> mx_ops(const uint8_t *brow, int RS, int 
 template <int NTERM>
 __device__ __forceinline__ void chunk_mx1(f32x4 &acc, const u32x4 &w, const MxOps<NTERM> &o, int c, int g, int K,
                                           bool full = false) {
-  const u32x4 wv = (full || Fmt<Q_MXFP4>::lane_valid(c, g, K)) ? w : u32x4{0u, 0u, 0u, 0u};
+  const u32x4 wv = (full || Fmt<Q_MXFP4_W>::lane_valid(c, g, K)) ? w : u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
   for (int t = 0; t < NTERM; ++t) acc = smfma(wv, o.b[t].lo, o.b[t].hi, o.sa & 0xFFu, o.b[t].s, acc);
 }
@@ -1155,7 +1154,7 @@ __device__ __forceinline__ void down_small_item(int it, int T, int &rt, int &t) 
 template <int FMT, int DA, int SMAX, int KS, bool SBS = false>
 __global__ __launch_bounds__(64 * SMAX * KS) void down_small(GemmArgs a, const int32_t *topk_idx) {
   warm_kernargs<sizeof(GemmArgs) + sizeof(void *)>();
-  constexpr int NM = 1;
+  constexpr int NM = 1, WF = FMT == Q_MXFP4 ? Q_MXFP4_W : FMT;
   extern __shared__ __align__(16) uint16_t s_h[];   // [slots][2][ldh + LDS_PAD]
   __shared__ f32x4 s_odd[KS > 1 ? SMAX : 1][4];     // odd chain, lanes l16 == 0
   constexpr bool SB = SBS && is_mlx<FMT>();         // MLX: each slot's scales and biases staged
@@ -1166,7 +1165,7 @@ __global__ __launch_bounds__(64 * SMAX * KS) void down_small(GemmArgs a, const i
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int g = lane >> 4, l16 = lane & 15;
   const int S = a.slots, K = a.top_k, H = a.hidden, E = a.experts;
-  const int T = a.max_work;              // tokens of the batch
+  const int T = a.tokens;
   const int nitems = down_small_items(a.row_tiles, T);
   const int r = wave % S, par = wave / S;
   HH_TR(2, 0);
@@ -1185,9 +1184,7 @@ __global__ __launch_bounds__(64 * SMAX * KS) void down_small(GemmArgs a, const i
   // The residual of the item's 16 rows (FFN block), loaded ahead of the weight stream.
   const float rv = (a.resid && tid < 16) ? a.resid[(size_t)t * H + rb + tid] : 0.f;
 
-  ATile<FMT> at[NM];
-  wave_tiles<PH_DOWN, FMT, 1>(at, blob, grp, rb, H, I, l16);
-  const int nch = (I + Fmt<FMT>::CHUNK - 1) / Fmt<FMT>::CHUNK;
+  const int nch = (I + Fmt<WF>::CHUNK - 1) / Fmt<WF>::CHUNK;
   f32x4 acc[2][NM][1];
 #pragma unroll
   for (int p = 0; p < 2; ++p) acc[p][0][0] = f32x4{0.f, 0.f, 0.f, 0.f};
@@ -1259,6 +1256,7 @@ __global__ __launch_bounds__(64 * SMAX * KS) void down_small(GemmArgs a, const i
   };
   u32x4 sbr[kMlxSbNB];
   if constexpr (SB) mlx_sb_load<1>(sbr, nch, sid, sth, sb_src);
+  const ATile<FMT> at[NM] = {tile_of<PH_DOWN, FMT>(blob, grp, min(rb, H - 16), false, I, l16)};
   AStream<FMT, NM, DA, SB> as(KS > 1 ? par : 0, KS, nch);
   as.fill(at, nch, g, I);
 #pragma unroll
@@ -1808,7 +1806,7 @@ hipError_t launch_down_small(int quant, GemmArgs a, const int32_t *topk_idx, int
   // MXFP4: per slot the activation terms and 16 rows of weight scales (of the larger group).
   const size_t lds_down = mx ? (size_t)S * (NTH * mx_row_bytes(a.hld) + 16 * ((16 * (imax / 32) + 15) / 16))
                              : (size_t)S * 2 * (a.ldh + LDS_PAD) * 2;
-  a.max_work = T;
+  a.tokens = T;
   const int ks = (mx || S > 4 || !one_down) ? 1 : 2;
   // Persistent, a multiple of 8 workgroups: up to two per compute unit, as many as are co-resident.
   const int down_per_cu = std::min(2, resident_per_cu((const void *)down, 64 * S * ks, lds_down));

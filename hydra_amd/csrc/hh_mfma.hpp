@@ -1,5 +1,5 @@
-// hh_mfma.hpp — device code shared by the expert products' translation units (hh_gemm.hip,
-// hh_prefill.hip): weight formats, the canonical arithmetic of one chunk, epilogue values, and the
+// hh_mfma.hpp — device code shared by the expert products' translation units (hh_gemm.hip and
+// hh_gemm_block.hip, hh_prefill.hip): weight formats, the canonical arithmetic of one chunk, epilogue values, and the
 // task order and direct-to-LDS loads of the prefill kernels.
 #pragma once
 #include "hh_common.hpp"
@@ -20,15 +20,6 @@ __device__ __forceinline__ uint32_t u8pair_to_bf16x2(uint32_t lo, uint32_t hi) {
   return __builtin_amdgcn_perm(b, a, 0x07060302u);   // the upper halves
 }
 
-// 8 4-bit MLX values of one word (low-order first) → bf16 integers.
-__device__ __forceinline__ bf16x8 mlx4_to_bf16(uint32_t w) {
-  u32x4 r;
-#pragma unroll
-  for (int k = 0; k < 4; ++k)
-    r[k] = u8pair_to_bf16x2((w >> (8 * k)) & 0xF, (w >> (8 * k + 4)) & 0xF);
-  return as_bf16x8(r);
-}
-
 // 8 8-bit MLX values of two words → bf16 integers.
 __device__ __forceinline__ bf16x8 mlx8_to_bf16(uint32_t w0, uint32_t w1) {
   u32x4 r = {u8pair_to_bf16x2(w0 & 0xFF, (w0 >> 8) & 0xFF),
@@ -40,24 +31,8 @@ __device__ __forceinline__ bf16x8 mlx8_to_bf16(uint32_t w0, uint32_t w1) {
 
 template <int FMT> struct Fmt;
 
-// ---- MXFP4: 128-column chunks, one 16-byte block per lane -----------------------------------
-template <> struct Fmt<Q_MXFP4> {
-  static constexpr int CHUNK = 128, NB = 4;  // B vectors (16 B) per lane per chunk
-  struct A { u32x4 w; uint32_t s; };
-  struct Row { const uint8_t *w; const uint8_t *s; };
-  __device__ static Row row(const uint8_t *blocks, const uint8_t *scales, int r, int K) {
-    return {blocks + (size_t)r * (K / 2), scales + (size_t)r * (K / 32)};
-  }
-  __device__ static void load(A &a, const Row &rw, int c, int g, int K) {
-    int kb = min(4 * c + g, K / 32 - 1);
-    a.w = *(const u32x4 *)(rw.w + kb * 16);
-    a.s = rw.s[kb];
-  }
-  __device__ static int bcol(int c, int g, int K) { return min(128 * c + 32 * g, K - 32); }
-  __device__ static bool lane_valid(int c, int g, int K) { return 128 * c + 32 * g < K; }
-};
-
-// ---- MXFP4 blocks without their scales (decode kernels stage a tile's scales in LDS) ----------
+// ---- MXFP4 blocks without their scales (decode kernels stage a tile's scales in LDS): 128-column
+// chunks, one 16-byte block per lane
 constexpr int Q_MXFP4_W = 4;
 // Rows are read through a buffer resource over the whole weight matrix of the expert: the lane's
 // row offset is computed once and a chunk's offset (64 bytes per chunk) goes into the
@@ -135,10 +110,6 @@ template <int BITS> struct FmtMLX {
     }
     a.sb = 0u;
   }
-  __device__ static bf16x8 decode(const A &a, int j) {
-    if constexpr (BITS == 4) return mlx4_to_bf16(a.w[j]);
-    else return mlx8_to_bf16(a.w[2 * j], a.w[2 * j + 1]);
-  }
   __device__ static int bcol(int c, int g, int) { return 64 * c + 16 * g; }
 };
 template <> struct Fmt<Q_MLX4> : FmtMLX<4> {};
@@ -148,25 +119,11 @@ template <int FMT> constexpr bool is_mlx() { return FMT == Q_MLX4 || FMT == Q_ML
 
 // ---- shared pieces of the canonical arithmetic -------------------------------------------------
 
-// Sum of 8 bf16 values of one 16-byte vector, in index order.
-__device__ __forceinline__ float sum8_bf16(const u32x4 &v) {
-  float s = 0.f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    s += bf16_bits_to_f32(v[k] & 0xFFFF);
-    s += bf16_bits_to_f32(v[k] >> 16);
-  }
-  return s;
-}
-
 // One 16-row A tile of a wave: the lane's weight row.
 template <int FMT> struct ATile {
   typename Fmt<FMT>::Row row;
 };
 
-// Tiles of a wave whose first output row is rb: PH_UP takes RT gate tiles then RT up tiles of
-// intermediates rb + 16q, PH_DOWN RT tiles of hidden rows rb + 16q. Rows past out_dim are
-// clamped into the matrix (their results are never stored).
 // One 16-row A tile: output rows r0 .. r0+15 (lane l16 takes r0 + l16); PH_UP picks the gate
 // (is_up false) or the up matrix.
 template <int PH, int FMT>
@@ -175,12 +132,9 @@ __device__ __forceinline__ ATile<FMT> tile_of(const uint8_t *blob, const ExpertG
   ATile<FMT> t;
   const int orow = r0 + l16;
   const int I = grp.inter;
-  if constexpr (FMT == Q_MXFP4) {
-    // GPT-OSS gate_up rows interleave gate and up (ReferenceLayer.swift:11).
-    if (PH == PH_UP) t.row = Fmt<FMT>::row(blob + grp.off[0], blob + grp.off[1], 2 * orow + (is_up ? 1 : 0), K);
-    else t.row = Fmt<FMT>::row(blob + grp.off[3], blob + grp.off[4], orow, K);
-  } else if constexpr (FMT == Q_MXFP4_W) {
-    // The matrix extends to the next sub-tensor of the blob (its scales).
+  if constexpr (FMT == Q_MXFP4_W) {
+    // GPT-OSS gate_up rows interleave gate and up (ReferenceLayer.swift:11). The matrix extends to the next
+    // sub-tensor of the blob (its scales).
     if (PH == PH_UP) t.row = Fmt<FMT>::row(blob + grp.off[0], grp.off[1] - grp.off[0], 2 * orow + (is_up ? 1 : 0), K);
     else t.row = Fmt<FMT>::row(blob + grp.off[3], grp.down_bytes ? grp.down_bytes : grp.off[4] - grp.off[3], orow, K);
   } else if constexpr (FMT == Q_BF16) {
@@ -193,16 +147,6 @@ __device__ __forceinline__ ATile<FMT> tile_of(const uint8_t *blob, const ExpertG
                           orow, K);
   }
   return t;
-}
-
-template <int PH, int FMT, int RT>
-__device__ __forceinline__ void wave_tiles(ATile<FMT> (&t)[(PH == PH_UP ? 2 : 1) * RT],
-                                           const uint8_t *blob, const ExpertGroup &grp, int rb,
-                                           int out_dim, int K, int l16) {
-  constexpr int NM = (PH == PH_UP ? 2 : 1) * RT;
-#pragma unroll
-  for (int m = 0; m < NM; ++m)
-    t[m] = tile_of<PH, FMT>(blob, grp, min(rb + 16 * (m % RT), out_dim - 16), (PH == PH_UP) && (m >= RT), K, l16);
 }
 
 // The MFMA sequence of chunk c for NM A tiles × NT token tiles. `bv(st, hh, v)` returns the
@@ -230,25 +174,6 @@ __device__ __forceinline__ void chunk_mfma(f32x4 (&acc)[NM][NT], const typename 
         for (int st = 0; st < NT; ++st)
 #pragma unroll
           for (int hh = 0; hh < NH; ++hh) acc[m][st] = mfma(as_bf16x8(w[m].w[v]), as_bf16x8(b[st][hh]), acc[m][st]);
-    }
-  } else if constexpr (!is_mlx<FMT>()) {
-    const bool ok = F::lane_valid(c, g, K);
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      u32x4 b[NT][NH];
-#pragma unroll
-      for (int st = 0; st < NT; ++st)
-#pragma unroll
-        for (int hh = 0; hh < NH; ++hh) b[st][hh] = bv(st, hh, v);
-#pragma unroll
-      for (int m = 0; m < NM; ++m) {
-        bf16x8 av;
-        av = mxfp4_to_bf16(ok ? w[m].w[v] : 0u, e8m0_to_f32(w[m].s));
-#pragma unroll
-        for (int st = 0; st < NT; ++st)
-#pragma unroll
-          for (int hh = 0; hh < NH; ++hh) acc[m][st] = mfma(av, as_bf16x8(b[st][hh]), acc[m][st]);
-      }
     }
   } else {
     // MLX affine, one 64-column group: P = Σ q·x on the bf16 MFMA (steps v = 0, 1: word v of the
@@ -300,7 +225,7 @@ __device__ __forceinline__ void chunk_mfma(f32x4 (&acc)[NM][NT], const typename 
           for (int k = 0; k < 4; ++k) r[k] = ((wv >> (4 * k)) & 0x000F000Fu) | 0x43004300u;
           av = as_bf16x8(r);
         } else {
-          av = F::decode(w[m], v);
+          av = mlx8_to_bf16(w[m].w[2 * v], w[m].w[2 * v + 1]);
         }
 #pragma unroll
         for (int st = 0; st < NT; ++st)
@@ -346,31 +271,19 @@ __device__ __forceinline__ f32x4 sum_chains(const f32x4 &p0, const f32x4 &p1) {
   return r;
 }
 
-// Activations of 4 intermediates i0..i0+3: bias (GPT-OSS gate_up bias, interleaved like the
-// rows) and the gated activation.
-template <int FMT>
-__device__ __forceinline__ f32x4 up_values(const GemmArgs &a, const uint8_t *blob, const ExpertGroup &grp,
-                                           int i0, const f32x4 &gate, const f32x4 &up) {
-  float gb[4] = {0.f, 0.f, 0.f, 0.f}, ub[4] = {0.f, 0.f, 0.f, 0.f};
-  if (FMT == Q_MXFP4 && a.expert_bias) {
-    const uint16_t *bias = (const uint16_t *)(blob + grp.off[2]);
-#pragma unroll
-    for (int ii = 0; ii < 4; ++ii) {
-      gb[ii] = bf16_bits_to_f32(bias[2 * (i0 + ii)]);
-      ub[ii] = bf16_bits_to_f32(bias[2 * (i0 + ii) + 1]);
-    }
-  }
+// Gated activations of 4 intermediates (BF16 and MLX layers, which have no expert bias).
+__device__ __forceinline__ f32x4 up_values(const GemmArgs &a, const f32x4 &gate, const f32x4 &up) {
   float gv[4], uv[4], yv[4];
 #pragma unroll
   for (int ii = 0; ii < 4; ++ii) {
-    gv[ii] = gate[ii] + gb[ii];
-    uv[ii] = up[ii] + ub[ii];
+    gv[ii] = gate[ii] + 0.f;
+    uv[ii] = up[ii] + 0.f;
   }
   activate_n<4>(a.act, gv, uv, yv, a.alpha, a.limit);
   return f32x4{yv[0], yv[1], yv[2], yv[3]};
 }
 
-// up_values with the GPT-OSS bias of the 4 intermediates already loaded: 16 bytes from the bias
+// The same with the GPT-OSS bias of the 4 intermediates, already loaded: 16 bytes from the bias
 // row at element 2·i0, (gate, up) bf16 pairs in order.
 __device__ __forceinline__ f32x4 up_values_mx(const GemmArgs &a, const u32x4 &bias, const f32x4 &gate,
                                               const f32x4 &up) {
@@ -384,12 +297,9 @@ __device__ __forceinline__ f32x4 up_values_mx(const GemmArgs &a, const u32x4 &bi
   return f32x4{yv[0], yv[1], yv[2], yv[3]};
 }
 
-// Gate-up epilogue of 4 intermediates i0..i0+3 of slot `slot`: bias, activation, bf16 hi/lo.
-template <int FMT>
-__device__ __forceinline__ void up_epilogue(const GemmArgs &a, const uint8_t *blob,
-                                            const ExpertGroup &grp, int i0, int slot,
-                                            const f32x4 &gate, const f32x4 &up) {
-  const f32x4 yv = up_values<FMT>(a, blob, grp, i0, gate, up);
+// Gate-up epilogue of 4 intermediates i0..i0+3 of slot `slot` (BF16 and MLX layers): activation, bf16 hi/lo.
+__device__ __forceinline__ void up_epilogue(const GemmArgs &a, int i0, int slot, const f32x4 &gate, const f32x4 &up) {
+  const f32x4 yv = up_values(a, gate, up);
   uint32_t hi[4], lo[4];
 #pragma unroll
   for (int ii = 0; ii < 4; ++ii) {

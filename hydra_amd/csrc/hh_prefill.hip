@@ -1,5 +1,5 @@
-// hh_prefill.hip — grouped expert products of the prefill path (T > 16) on gfx950 MFMA: one
-// four-wave workgroup per task (a row tile × a work item), two workgroups per compute unit.
+// hh_prefill.hip — expert products grouped by expert, on gfx950 MFMA: batches above 16 tokens, and of 5 to 16
+// tokens on BF16 and MLX layers large enough for it (hh_api.hip:mid_batch). One four-wave workgroup per task (a row tile × a work item), two workgroups per compute unit.
 #include "hh_mfma.hpp"
 
 #include <algorithm>
@@ -86,7 +86,7 @@ __global__ __launch_bounds__(256 * WT_) __attribute__((amdgpu_waves_per_eu(2, 2)
   const int H = a.hidden, E = a.experts;
   const int nwork = *a.n_work;
   int rt, wi;
-  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.max_work + (int)blockIdx.x, rt, wi)) return;
+  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.first_task + (int)blockIdx.x, rt, wi)) return;
   const int4 it = a.work[wi];
   const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
   const ExpertGroup &grp = a.grp[e == E ? 1 : 0];
@@ -198,8 +198,8 @@ __global__ __launch_bounds__(256 * WT_) __attribute__((amdgpu_waves_per_eu(2, 2)
       const int r0 = rb + 16 * r;
       if (r0 >= out_dim) continue;
       if constexpr (PH == PH_UP) {
-        up_epilogue<Q_BF16>(a, nullptr, grp, r0 + 4 * g, es[st], sum_chains(acc[0][r][st], acc[1][r][st]),
-                            sum_chains(acc[0][RT + r][st], acc[1][RT + r][st]));
+        up_epilogue(a, r0 + 4 * g, es[st], sum_chains(acc[0][r][st], acc[1][r][st]),
+                    sum_chains(acc[0][RT + r][st], acc[1][RT + r][st]));
       } else {
         const f32x4 v = sum_chains(acc[0][r][st], acc[1][r][st]);
         f32x4 o;
@@ -249,7 +249,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   const int H = a.hidden, E = a.experts;
   const int nwork = *a.n_work;
   int rt, wi;
-  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.max_work + (int)blockIdx.x, rt, wi)) return;
+  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.first_task + (int)blockIdx.x, rt, wi)) return;
   const int4 it = a.work[wi];
   const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
   const ExpertGroup &grp = a.grp[e == E ? 1 : 0];
@@ -437,8 +437,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
       const int r0 = rb + 16 * r;
       if (r0 >= out_dim) continue;
       if constexpr (PH == PH_UP) {
-        up_epilogue<Q_BF16>(a, nullptr, grp, r0 + 4 * g, es[st], sum_chains(acc[0][r][st], acc[1][r][st]),
-                            sum_chains(acc[0][RT + r][st], acc[1][RT + r][st]));
+        up_epilogue(a, r0 + 4 * g, es[st], sum_chains(acc[0][r][st], acc[1][r][st]),
+                    sum_chains(acc[0][RT + r][st], acc[1][RT + r][st]));
       } else {
         const f32x4 v = sum_chains(acc[0][r][st], acc[1][r][st]);
         f32x4 o;
@@ -495,7 +495,7 @@ __global__ __launch_bounds__(256, (Mx<PH, NT_>::WGS)) void prefill_mx(GemmArgs a
   const int H = a.hidden;
   const int nwork = *a.n_work;
   int rt, wi;
-  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.max_work + (int)blockIdx.x, rt, wi)) return;
+  if (!PrefillTasks(a.row_tiles, nwork, kRowParts).tile(a.first_task + (int)blockIdx.x, rt, wi)) return;
   const int4 it = a.work[wi];
   const int e = uniform(it.x), pos = uniform(it.y), cnt = uniform(it.z);
   const ExpertGroup &grp = a.grp[e == a.experts ? 1 : 0];
@@ -692,7 +692,7 @@ __global__ __launch_bounds__(256, (Mx<PH, NT_>::WGS)) void prefill_mx(GemmArgs a
 }
 
 // One workgroup per task; launches of at most 2^22 workgroups (a launch's threads are counted in 32
-// bits), each told its first task in max_work.
+// bits), each told its first task.
 template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int threads, int rows, GemmArgs a, hipStream_t s,
                                                   Timing tm, std::once_flag &once) {
   std::call_once(once, [&] {
@@ -704,7 +704,7 @@ template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int 
   const int64_t tasks = 8ll * ((a.row_tiles + P - 1) / P) * ((a.max_work + 8 / P - 1) / (8 / P));
   constexpr int64_t most = 1ll << 22;
   for (int64_t t0 = 0; t0 < tasks; t0 += most) {
-    a.max_work = (int32_t)t0;
+    a.first_task = (int32_t)t0;
     hipExtLaunchKernelGGL(kernel, dim3((unsigned)std::min(most, tasks - t0)), dim3(threads), C::LDS, s,
                           t0 == 0 ? tm.start : nullptr, t0 + most >= tasks ? tm.stop : nullptr, 0, a);
     const hipError_t e = hipGetLastError();

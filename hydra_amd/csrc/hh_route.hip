@@ -1370,7 +1370,7 @@ static hipError_t launch_dispatch(const RouteArgs &a, hipStream_t s, hipEvent_t 
 }
 
 // The MLX-router sequence: exact logits, x terms (MXFP4 layers), selection (unless the layer's
-// decode gate-up kernel selects), dispatch (layers above 16 tokens).
+// decode gate-up kernel selects), dispatch (the grouped products; up to 16 tokens in the selection's launch).
 hipError_t launch_route_mlx(const RouteArgs &a, hipStream_t s, Timing tm) {
   const int rows = a.experts + (a.shared_gate ? 1 : 0);
   const bool small = a.tokens <= RT_TOK;

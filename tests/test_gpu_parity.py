@@ -236,7 +236,7 @@ TINY = {
     "mxfp4-narrow": F.MoEDesc(hidden=192, intermediate=64, experts=4, top_k=2,
                               quant=F.QUANT_MXFP4, activation=F.ACT_SWIGLU_OAI,
                               router=F.ROUTER_TOPK_SOFTMAX, expert_bias=1),
-    # Rows of ≥ 8 chunks in both products: the persistent LDS-ring prefill kernel.
+    # Rows of 8 chunks in both products.
     "mxfp4-wide": F.MoEDesc(hidden=1024, intermediate=1024, experts=8, top_k=4,
                             quant=F.QUANT_MXFP4, activation=F.ACT_SWIGLU_OAI,
                             router=F.ROUTER_TOPK_SOFTMAX, expert_bias=1),
@@ -283,7 +283,7 @@ def test_prefill_equals_token_by_token_bit_for_bit(torch_dev, ctx, name):
     desc = TINY[name]
     say(f"prefill==decode {name}")
     layer = synth.make_layer(desc, seed=41)
-    T = 80                                   # crosses the 64-token tile switch
+    T = 80                                   # several work items an expert
     x = synth.make_tokens(desc.hidden, T, seed=42)
     L = MoELayer(layer, ctx)
     y_all, idx_all, w_all = L.forward(x)
@@ -321,12 +321,10 @@ def test_large_batch_equals_token_by_token_bit_for_bit(torch_dev, ctx, name):
 
 WIDE = {
     "mxfp4-wide": TINY["mxfp4-wide"],
-    # Gate-up rows of ≥ 12 chunks: the register-ring gate-up kernel (64-token items at T=300: the
-    # experts average 150 tokens).
+    # Gate-up rows of 16 chunks, 150 tokens an expert at T=300; 32-token items, of few tasks as above.
     "mxfp4-deep": F.MoEDesc(hidden=2048, intermediate=1024, experts=8, top_k=4, quant=F.QUANT_MXFP4,
                             activation=F.ACT_SWIGLU_OAI, router=F.ROUTER_TOPK_SOFTMAX, expert_bias=1),
-    # Many experts (≈ 19 tokens each at T=300): 32-token items, the register-ring gate-up kernel's
-    # 32-token tiles and the 128-row down tiles.
+    # Many experts (≈ 19 tokens each at T=300): 64-token gate-up items, 32-token down items.
     "mxfp4-many": F.MoEDesc(hidden=2048, intermediate=1024, experts=64, top_k=4, quant=F.QUANT_MXFP4,
                             activation=F.ACT_SWIGLU_OAI, router=F.ROUTER_TOPK_SOFTMAX, expert_bias=1),
 }
