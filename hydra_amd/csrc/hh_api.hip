@@ -16,7 +16,7 @@
 namespace hh {
 hipError_t launch_route(const RouteArgs &a, hipStream_t s, Timing tm = {});
 hipError_t launch_permute(const RouteArgs &a, hipStream_t s);
-hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm);
+hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, int max_work, hipStream_t s, Timing tm);
 hipError_t launch_small(int quant, GemmArgs a, const RouteArgs &ra, hipStream_t s, Timing tm_up,
                         Timing tm_down, const FuseArgs *fr = nullptr);
 bool fused_router_fits(int quant, int H, int E, int router, int T);
@@ -573,7 +573,6 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
   g.alpha = d->swiglu_alpha;
   g.limit = d->swiglu_limit;
   g.ldh = s.ldh;
-  g.max_work = s.max_work;
   g.x = x;
   g.order = r.order;
   g.work = r.work;
@@ -655,16 +654,15 @@ int forward_layer(hh_ctx *ctx, const hh_moe_desc *d, const hh_moe_weights *w, co
     return HH_OK;
   }
   if ((rc = phase_timing(ctx, &tm, noalloc))) return rc;
-  HH_HIP(hh::launch_gemm(0, d->quant, s.nt, g, ctx->stream, tm));
+  HH_HIP(hh::launch_gemm(0, d->quant, s.nt, g, s.max_work, ctx->stream, tm));
   if ((rc = phase_timing(ctx, &tm, noalloc))) return rc;
   if (s.half_down) {
     hh::GemmArgs gd = g;
     gd.work = r.work_half;
     gd.n_work = r.n_work_half;
-    gd.max_work = s.max_work_half;
-    HH_HIP(hh::launch_gemm(1, d->quant, s.nt / 2, gd, ctx->stream, tm));
+    HH_HIP(hh::launch_gemm(1, d->quant, s.nt / 2, gd, s.max_work_half, ctx->stream, tm));
   } else {
-    HH_HIP(hh::launch_gemm(1, d->quant, s.nt, g, ctx->stream, tm));
+    HH_HIP(hh::launch_gemm(1, d->quant, s.nt, g, s.max_work, ctx->stream, tm));
   }
   if ((rc = phase_timing(ctx, &tm, noalloc))) return rc;
   HH_HIP(hh::launch_combine(g.slot_out, s.slots, d->hidden, T, y, resid, ctx->stream, tm));
@@ -1219,8 +1217,7 @@ int hh_expert_gemm(hh_ctx *ctx, const hh_matrix *m, const float *x, int32_t T, f
   if (T <= kSmallT) {
     HH_HIP(hh::launch_down_small(q, g, topk, T, ctx->stream, hh::Timing{}));
   } else {
-    g.max_work = items;
-    HH_HIP(hh::launch_gemm(1, q, tile / 16, g, ctx->stream, hh::Timing{}));
+    HH_HIP(hh::launch_gemm(1, q, tile / 16, g, items, ctx->stream, hh::Timing{}));
   }
   ctx->dispatches += 2;
   return HH_OK;

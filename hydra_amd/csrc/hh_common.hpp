@@ -241,13 +241,12 @@ struct GemmArgs {
   int32_t quant, act, expert_bias, group;
   float alpha, limit;
   int32_t ldh;                  // row stride (elements) of h_hi / h_lo; multiple of 64
-  int32_t max_work;             // grouped products, on the host: most work items
-  int32_t first_task;           // grouped products: the launch's first task
-  int32_t row_tiles;            // workgroup row tiles along the output dimension
   int32_t tokens;               // decode down product: tokens of the batch
+  int32_t row_tiles;            // workgroup row tiles along the output dimension
+  int32_t first_task;           // grouped products: the launch's first task
   const uint16_t *x;            // bf16 [T][H]
   const int32_t *order;         // [positions] slot id (t·slots + r) of each permuted position (grouped products)
-  const int4 *work;             // [max_work] {expert (E = shared), pos0, n, 0}
+  const int4 *work;             // work items {expert (E = shared), pos0, n, 0}
   const int32_t *n_work;        // device count of valid work items
   uint16_t *h_hi, *h_lo;        // bf16 [T·slots][ldh]: activation of each slot, hi + lo split
   // MXFP4 (scaled fp4 × fp8 products): the operands as fp8 e4m3 terms with e8m0 block scales.

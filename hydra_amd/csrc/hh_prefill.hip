@@ -693,15 +693,15 @@ __global__ __launch_bounds__(256, (Mx<PH, NT_>::WGS)) void prefill_mx(GemmArgs a
 
 // One workgroup per task; launches of at most 2^22 workgroups (a launch's threads are counted in 32
 // bits), each told its first task.
-template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int threads, int rows, GemmArgs a, hipStream_t s,
-                                                  Timing tm, std::once_flag &once) {
+template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int threads, int rows, GemmArgs a, int max_work,
+                                                  hipStream_t s, Timing tm, std::once_flag &once) {
   std::call_once(once, [&] {
     (void)hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, C::LDS);
     (void)hipGetLastError();
   });
   a.row_tiles = (rows + C::ROWS - 1) / C::ROWS;
   constexpr int P = kRowParts;
-  const int64_t tasks = 8ll * ((a.row_tiles + P - 1) / P) * ((a.max_work + 8 / P - 1) / (8 / P));
+  const int64_t tasks = 8ll * ((a.row_tiles + P - 1) / P) * ((max_work + 8 / P - 1) / (8 / P));
   constexpr int64_t most = 1ll << 22;
   for (int64_t t0 = 0; t0 < tasks; t0 += most) {
     a.first_task = (int32_t)t0;
@@ -713,27 +713,27 @@ template <class C> static hipError_t launch_tasks(void (*kernel)(GemmArgs), int 
   return hipSuccess;
 }
 // Tasks of a launch at most, with `rows` output rows each.
-static int64_t tasks(const GemmArgs &a, int out, int rows) { return (int64_t)a.max_work * ((out + rows - 1) / rows); }
+static int64_t tasks(int max_work, int out, int rows) { return (int64_t)max_work * ((out + rows - 1) / rows); }
 template <int PH> static int out_rows(const GemmArgs &a) {
   return PH == PH_UP ? std::max(a.grp[0].inter, a.grp[1].inter) : a.hidden;
 }
-template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(const GemmArgs &a, hipStream_t s, Timing tm) {
+template <int PH, int NT, int RT, int SV, int WT> static hipError_t launch_bf16(const GemmArgs &a, int max_work, hipStream_t s, Timing tm) {
   static std::once_flag once;
-  return launch_tasks<Bf<PH, NT, RT, SV, WT>>(prefill_bf16<PH, NT, RT, SV, WT>, 256 * WT, out_rows<PH>(a), a, s, tm, once);
+  return launch_tasks<Bf<PH, NT, RT, SV, WT>>(prefill_bf16<PH, NT, RT, SV, WT>, 256 * WT, out_rows<PH>(a), a, max_work, s, tm, once);
 }
-template <int PH, int BITS, int RT, int NT> static hipError_t launch_mlx(const GemmArgs &a, hipStream_t s, Timing tm) {
+template <int PH, int BITS, int RT, int NT> static hipError_t launch_mlx(const GemmArgs &a, int max_work, hipStream_t s, Timing tm) {
   static std::once_flag once;
-  return launch_tasks<Ml<PH, BITS, RT, NT>>(prefill_mlx<PH, BITS, RT, NT>, 256, out_rows<PH>(a), a, s, tm, once);
+  return launch_tasks<Ml<PH, BITS, RT, NT>>(prefill_mlx<PH, BITS, RT, NT>, 256, out_rows<PH>(a), a, max_work, s, tm, once);
 }
-template <int PH, int NT> static hipError_t launch_mx(const GemmArgs &a, hipStream_t s, Timing tm) {
+template <int PH, int NT> static hipError_t launch_mx(const GemmArgs &a, int max_work, hipStream_t s, Timing tm) {
   static std::once_flag once;
-  return launch_tasks<Mx<PH, NT>>(prefill_mx<PH, NT>, 256, (PH == PH_UP ? 2 : 1) * out_rows<PH>(a), a, s, tm, once);
+  return launch_tasks<Mx<PH, NT>>(prefill_mx<PH, NT>, 256, (PH == PH_UP ? 2 : 1) * out_rows<PH>(a), a, max_work, s, tm, once);
 }
 
-// The tile of each call. BF16 work items hold 160 tokens (nt 10: experts averaging 40 tokens or
+// The tile of each call (`max_work`: its work items at most). BF16 work items hold 160 tokens (nt 10: experts averaging 40 tokens or
 // more) or 32, MXFP4 items 16 (nt 1), 32, or 64 for the gate-up
 // (nt 4), MLX items 32.
-hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStream_t s, Timing tm) {
+hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, int max_work, hipStream_t s, Timing tm) {
   const bool up = phase == PH_UP;
   if (quant == Q_MLX4) {
     // Tiles of 64 rows where even they do not fill the two workgroups a compute unit holds (tasks counted at the
@@ -742,26 +742,26 @@ hipError_t launch_gemm(int phase, int quant, int nt, const GemmArgs &a, hipStrea
     // T = 8 26 / 24 (268), T = 12 36 / 37 (400). Down: 4 experts of H 2048, I 1536 (K 2) T = 100 24 / 17 (121), T = 300
     // 24 / 32 (253). Down tiles of 128 rows where those of 192 would be a tenth padding, with up to two tasks a
     // compute unit: 512 x 2880 T = 2000 55 / 48 (189), 1024 x 1024 T = 2000 33 / 30 (378), T = 8000 77 / 82 (1500).
-    if (up) return tasks(a, a.grp[0].inter, 128) <= 300 ? launch_mlx<PH_UP, 4, 1, 2>(a, s, tm) : launch_mlx<PH_UP, 4, 2, 2>(a, s, tm);
-    const int64_t wide = tasks(a, a.hidden, 192);
-    if (wide <= 130) return launch_mlx<PH_DOWN, 4, 1, 2>(a, s, tm);
+    if (up) return tasks(max_work, a.grp[0].inter, 128) <= 300 ? launch_mlx<PH_UP, 4, 1, 2>(a, max_work, s, tm) : launch_mlx<PH_UP, 4, 2, 2>(a, max_work, s, tm);
+    const int64_t wide = tasks(max_work, a.hidden, 192);
+    if (wide <= 130) return launch_mlx<PH_DOWN, 4, 1, 2>(a, max_work, s, tm);
     const int pad128 = (a.hidden + 127) / 128 * 128, pad192 = (a.hidden + 191) / 192 * 192;
-    if (wide <= 512 && 10 * pad192 > 11 * pad128) return launch_mlx<PH_DOWN, 4, 2, 2>(a, s, tm);
-    return launch_mlx<PH_DOWN, 4, 3, 2>(a, s, tm);
+    if (wide <= 512 && 10 * pad192 > 11 * pad128) return launch_mlx<PH_DOWN, 4, 2, 2>(a, max_work, s, tm);
+    return launch_mlx<PH_DOWN, 4, 3, 2>(a, max_work, s, tm);
   }
   if (quant == Q_MLX8) {
     // The same for 8-bit down tiles: 4 experts of H 2048, I 1536 (K 2) T = 40 the layer 60 / 55 (tasks of 128 rows: 112),
     // 1 expert of H 2880, I 512 T = 300 61 / 65 (253).
-    if (up) return launch_mlx<PH_UP, 8, 1, 2>(a, s, tm);
-    return tasks(a, a.hidden, 128) <= 200 ? launch_mlx<PH_DOWN, 8, 1, 2>(a, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, s, tm);
+    if (up) return launch_mlx<PH_UP, 8, 1, 2>(a, max_work, s, tm);
+    return tasks(max_work, a.hidden, 128) <= 200 ? launch_mlx<PH_DOWN, 8, 1, 2>(a, max_work, s, tm) : launch_mlx<PH_DOWN, 8, 2, 2>(a, max_work, s, tm);
   }
   if (quant == Q_MXFP4) {
-    if (nt == 1) return up ? launch_mx<PH_UP, 1>(a, s, tm) : launch_mx<PH_DOWN, 1>(a, s, tm);
-    if (up) return nt == 4 ? launch_mx<PH_UP, 4>(a, s, tm) : launch_mx<PH_UP, 2>(a, s, tm);
-    return launch_mx<PH_DOWN, 2>(a, s, tm);
+    if (nt == 1) return up ? launch_mx<PH_UP, 1>(a, max_work, s, tm) : launch_mx<PH_DOWN, 1>(a, max_work, s, tm);
+    if (up) return nt == 4 ? launch_mx<PH_UP, 4>(a, max_work, s, tm) : launch_mx<PH_UP, 2>(a, max_work, s, tm);
+    return launch_mx<PH_DOWN, 2>(a, max_work, s, tm);
   }
-  if (nt == 10) return up ? launch_bf16<PH_UP, 5, 2, 2, 2>(a, s, tm) : launch_bf16<PH_DOWN, 5, 4, 2, 2>(a, s, tm);
-  return up ? launch_bf16<PH_UP, 2, 1, 2, 1>(a, s, tm) : launch_bf16<PH_DOWN, 2, 2, 2, 1>(a, s, tm);
+  if (nt == 10) return up ? launch_bf16<PH_UP, 5, 2, 2, 2>(a, max_work, s, tm) : launch_bf16<PH_DOWN, 5, 4, 2, 2>(a, max_work, s, tm);
+  return up ? launch_bf16<PH_UP, 2, 1, 2, 1>(a, max_work, s, tm) : launch_bf16<PH_DOWN, 2, 2, 2, 1>(a, max_work, s, tm);
 }
 
 }  // namespace hh

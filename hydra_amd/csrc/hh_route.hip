@@ -899,7 +899,7 @@ __global__ __launch_bounds__(256) void logits_small_kernel(RouteArgs a) {
   const int t = p / E1, e = p - t * E1;
   if (e == E && !a.shared_gate) return;
   const double v = pair_logit<gemma>(a, t, e);
-  if (lane == 0) a.lg64[(size_t)t * E1 + e] = v;
+  if (lane == 0) a.lg64[(size_t)t * E1 + e] = e < E ? ranked(v) : v;
   if (wave == 0) HH_RT(1);
 }
 
@@ -930,7 +930,7 @@ __global__ __launch_bounds__(256) void logits_split_kernel(RouteArgs a) {
   const int t = blockIdx.x / E1, e = blockIdx.x - t * E1;
   if (e == E && !a.shared_gate) return;   // uniform over the workgroup
   const double v = split_pair_logit<gemma>(a, t, e, s_acc, s_px);
-  if (wave == 0 && lane == 0) a.lg64[(size_t)t * E1 + e] = v;
+  if (wave == 0 && lane == 0) a.lg64[(size_t)t * E1 + e] = e < E ? ranked(v) : v;
   if (wave == 0) HH_RT(1);
 }
 
@@ -1044,7 +1044,7 @@ __global__ __launch_bounds__(64 * BLK_W) void logits_block_kernel(RouteArgs a) {
   }
   double v = wave_sum_f64((acc[0] + acc[1]) + (acc[2] + acc[3]));
   if (e < E && a.router_b) v += (double)bf16_bits_to_f32(a.router_b[e]);
-  if (lane == 0) a.lg64[(size_t)t * E1 + e] = v;
+  if (lane == 0) a.lg64[(size_t)t * E1 + e] = e < E ? ranked(v) : v;
   if (wave == 0) HH_RT(1);
 }
 
@@ -1186,7 +1186,7 @@ __global__ __launch_bounds__(256) void mlx_router_logits_kernel(RouteArgs a) {
   const int t0 = tile * tsz, t1 = min(T, t0 + tsz);
   const int r0 = wid * R;
   mlx_rows_logits<BITS, R, J, 4>(a, [&](int r) { return min(r0 + r, rows - 1); }, rows - r0, t0, t1,
-                                 [&](double v, int r, int tp) { a.lg64[(size_t)tp * (E + 1) + r0 + r] = v; });
+                                 [&](double v, int r, int tp) { a.lg64[(size_t)tp * (E + 1) + r0 + r] = r0 + r < E ? ranked(v) : v; });
 }
 
 // ---- MLX-affine router above 16 tokens: screen on the MFMA, exact logits of the candidates ----

@@ -41,6 +41,8 @@ __device__ __forceinline__ int block_exclusive_scan(int *data, int n, int *s_wav
 // A logit as the selections rank it: NaN (a token or router row with NaN, or infinities that cancel)
 // as −∞, so that any K logits give K distinct experts, each below E: the ids index LDS tables,
 // segment counts and weights. Comparisons with NaN are all false, which would leave ranks unfilled.
+// Applied where an expert's logit is written (or inserted), so the selections read none that is NaN; the shared
+// gate's, which is ranked with none, keeps its NaN.
 __device__ __forceinline__ double ranked(double logit) { return fmax(logit, -INFINITY); }
 
 // Running exact top-k, descending, ties to the smaller index. Every lane of a wave holds the
@@ -124,7 +126,7 @@ __device__ __forceinline__ TopK topk_exact(const double *lg, int E, int K) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
     const int e = lane + 64 * j;
-    v[j] = e < E ? ranked(lg[e]) : -INFINITY;
+    v[j] = e < E ? lg[e] : -INFINITY;
   }
   TopK tk;
   uint32_t taken = 0;
@@ -188,7 +190,7 @@ template <int NW = 1>
 __device__ __forceinline__ TopK topk_rank64(const double *lg, int E, int K, double *s_lg, int *s_ri,
                                             int (*s_part)[64] = nullptr) {
   const int lane = threadIdx.x & 63;
-  const double v = lane < E ? ranked(lg[lane]) : -INFINITY;
+  const double v = lane < E ? lg[lane] : -INFINITY;
   s_lg[lane] = v;
   __builtin_amdgcn_wave_barrier();
   int j0, j1;
@@ -229,8 +231,7 @@ __device__ __forceinline__ double readlane_f64(double v, int l) {
 // (larger, or equal with a smaller index) from registers by readlane, so ties resolve exactly as
 // topk_exact's. s_ri / s_rv[kMaxTopK] and s_ci[kFastCand] / s_cv[kFastCand] are the wave's LDS
 // scratch; more candidates than 64 (heavy ties) rank from LDS, more than kFastCand take
-// topk_exact. NaN is no candidate: fewer than K candidates (fewer than K other logits) take
-// topk_exact, which ranks it, so no logit pays for a test here.
+// topk_exact.
 // NW > 1: groups of NW waves share the 64 lane maxima's ranking (one barrier pair for every
 // group, whatever its token); NWC > 1 also splits the candidates' ranking, whose barrier count
 // depends on the candidate count: only when every wave of the workgroup ranks the same token.
@@ -262,7 +263,7 @@ __device__ __forceinline__ TopK topk_fast(const double *lg, int E, int K, int *s
   int nc = 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) nc += __popcll(__ballot(lane + 64 * j < E && v[j] >= tau));
-  if (nc < K || nc > kFastCand) return topk_exact(lg, E, K);
+  if (nc > kFastCand) return topk_exact(lg, E, K);
   nc = 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
