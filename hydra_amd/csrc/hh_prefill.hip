@@ -42,7 +42,8 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // Weight loads take whole 128-byte (4-bit MLX: 64-byte) pieces of a row with consecutive lanes: 50 B/clk
 // per compute unit from L2, against 15.5 for the MFMA lane order (16 rows × 64 bytes, consecutive
 // lanes on different rows), which the L1 serves a row at a time when the row stride is a multiple
-// of 128 bytes. The XOR of the 16-byte segments by the row keeps the MFMA lanes' LDS reads at full rate.
+// of 128 bytes. The XOR of the 16-byte segments by the row keeps the MFMA lanes' LDS reads at full rate for BF16
+// and 8-bit MLX (no conflict cycles counted; a fifth of MXFP4's and 4-bit MLX's LDS cycles are conflicts).
 // The output tiles' arithmetic is the canonical one (chunk_mfma, prefill equals decode bit for bit).
 //
 // XCD order (PrefillTasks): two row-tile parts × four item parts, so an item's token rows reach two
@@ -53,7 +54,8 @@ __device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirs
 // 32 columns per stage.
 // Tiles, timed on the 128-expert layer (H 2816, I 704; gate-up / down us at T tokens):
 //   T = 2048 (128 tokens an expert): 64-token items of 128 intermediates 300 / 222, 128-token items
-//     285 / 217, 160-token items 278 / 194 (an expert's weights are read 2.5, 1.5, 1.0 times);
+//     285 / 217, 160-token items 278 / 194 (an expert's weights are in 2.5, 1.5, 1.0 items; at 160 the
+//     counters show 1.18 / 1.11 times the bytes needed);
 //     with 32-column stages (64-byte pieces) 349 for the 64-token gate-up;
 //   T = 700 (44 an expert): 160-token 206 / 144, 32-token 243 / 141;
 //   T = 400 (25 an expert): 160-token 195 / 133, 32-token 196 / 112, hence the line at 40;
@@ -455,8 +457,8 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 // terms, and, every third stage, the scales of three stages. A wave owns 64 weight rows (32
 // intermediates of gate-up, gate and up rows interleaved) and all the item's tokens.
 // What bounds it: the weight rows' arrival. Without weight traffic the T = 2048 gate-up takes 305 of its
-// 411 us (and 224 without its MFMAs, 360 without its epilogue), so three things keep more of them in flight or
-// make them cheaper, on the 128-expert layer (H = I = 2880, Zipf load; gate-up / down us):
+// 411 us (and 224 without its MFMAs, 360 without its epilogue; the MFMA pipes are busy a third of the time, and 2.1 times the
+// bytes needed are fetched, 1.4 at T = 512), so three things keep more of them in flight or make them cheaper, on the 128-expert layer (H = I = 2880, Zipf load; gate-up / down us):
 //   - scales 16 bytes a row every three stages instead of 4 every stage (a row's scales lie 90
 //     bytes from the next row's, so every lane of such a load takes a cache line of its own): T = 2048
 //     447 / 312 -> 413 / 283, T = 512 212 / 135 -> 193 / 124;

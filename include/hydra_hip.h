@@ -136,7 +136,10 @@ void *hh_ctx_stream(hh_ctx *ctx);
 int hh_ctx_synchronize(hh_ctx *ctx);
 /* Pre-sizes the scratch arena for up to max_tokens tokens of layers shaped like `desc`, so
  * that later hh_moe_forward calls within that bound allocate nothing (the reference's
- * preallocated scratch, LayerRunner.swift:6-10).                                             */
+ * preallocated scratch, LayerRunner.swift:6-10). While graphs of the context live, the arena
+ * cannot grow and calls that do not fit their preferred plan take one with less scratch, with
+ * the same results; a reservation is then granted if the arena covers what every call up to
+ * max_tokens would take, and HH_EINVAL otherwise. hh_runner_reserve follows the same rule.   */
 int hh_ctx_reserve(hh_ctx *ctx, const hh_moe_desc *desc, int32_t max_tokens);
 /* Kernel launches issued through this context since creation (the DispatchCounter analogue,
  * ForwardEncoder.swift:34-68).                                                               */
