@@ -2,17 +2,17 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W]
 
-Headline (`value`): GPT-OSS-20B-shaped MXFP4 MoE layer in decode at T=1 (BASELINE.json
-configs[1]), whole-layer tokens/s (router + top-k + dispatch + gate-up + SwiGLU + down +
+Headline (`value`): GPT-OSS-20B-shaped MXFP4 MoE layer (hidden and intermediate 2880, 32 experts,
+top-4) in decode at T=1, whole-layer tokens/s (router + top-k + dispatch + gate-up + SwiGLU + down +
 combine) with inputs already in HBM. A step is one layer over one token batch; steps cycle over
 several resident copies of the layer (> 256 MB Infinity Cache) and over a bank of inputs, so
 every step streams its experts from HBM as consecutive layers of a model would.
 
 Also reported: decode at T=2, 4, 8; the GPT-OSS-120B-shaped Zipf-skewed chunked prefill at
-T=512 and T=2048 (configs[2]); the Qwen-shaped MLX 4-bit and 8-bit layers (configs[3]) and the
-BF16 GELU layer at T=1 and in chunked prefill; the roofline of the dominant kernel (the gate-up expert
+T=512 and T=2048; the Qwen-shaped MLX 4-bit and 8-bit layers and the
+BF16 GELU layer at T=1, T=8 and in chunked prefill; the roofline of the dominant kernel (the gate-up expert
 product) from HIP events on the library's stream; and the fp64 CPU restatement of the
-reference path timed on this host (configs[0]).
+reference path timed on this host.
 
 Prints one JSON line.
 """
@@ -289,9 +289,8 @@ def measure_prefill(wl, T, steps, warmup):
     }
 
 
-OTHER = [  # (name, desc, copies, prefill T, router bits): BASELINE configs[3] (both bit
-    # widths; the router and shared gate 8-bit MLX-affine as the published Qwen checkpoints
-    # store them, Qwen35MoeConfig.swift:340-342) and [4]
+OTHER = [  # (name, desc, copies, prefill T, router bits); the Qwen router and shared gate are 8-bit
+    # MLX-affine as the published checkpoints store them (Qwen35MoeConfig.swift:340-342)
     ("qwen-35b-a3b-mlx4", F.QWEN_35B_A3B_Q4, 2, 1024, 8),
     ("qwen-35b-a3b-mlx8", F.QWEN_35B_A3B_Q8, 2, 1024, 8),
     ("gemma-bf16", F.GEMMA_BF16, 2, 2048, 0),
@@ -324,8 +323,8 @@ def measure_other(torch, name, desc, copies, T_prefill, steps, prefill=True, dec
 
 
 def cpu_baseline(runs=5, seconds=2.5):
-    """The fp64 restatement of the reference's CPU path (oracle/), GPT-OSS-20B shape
-    (configs[0]), timed on this host: `runs` timed runs of T=16 tokens per call with OpenMP over
+    """The fp64 restatement of the reference's CPU path (oracle/), GPT-OSS-20B shape,
+    timed on this host: `runs` timed runs of T=16 tokens per call with OpenMP over
     rows (each about `seconds` long) and `runs` single-thread T=1 calls; the medians are
     reported."""
     from oracle import oracle as O
@@ -351,7 +350,7 @@ def cpu_baseline(runs=5, seconds=2.5):
             "runs": runs, "openmp_tokens_per_s": omp, "openmp_threads": threads,
             "single_thread_tokens_per_s": float(np.median(single)),
             "single_thread_runs": single,
-            "sample": f"gpt-oss-20b MXFP4 MoE layer (BASELINE configs[0]), fp64 oracle: median of "
+            "sample": f"gpt-oss-20b MXFP4 MoE layer, fp64 oracle: median of "
                       f"{runs} runs of T=16 calls with OpenMP over rows on {threads} threads "
                       f"({total} tokens in ~{runs * seconds:.0f}s), and median of {runs} "
                       f"single-thread T=1 calls"}
@@ -481,7 +480,7 @@ def main():
         "vs_baseline": None,
         "dtype": "mxfp4 weights x fp8-e4m3 activation terms (x: 2 terms, h: 3), fp32 accumulation",
         "data": "synthetic",
-        "config": {"workload": "gpt-oss-20b-shaped MXFP4 MoE layer, decode T=1 (BASELINE configs[1])",
+        "config": {"workload": "gpt-oss-20b-shaped MXFP4 MoE layer, decode T=1",
                    "hidden": 2880, "intermediate": 2880, "experts": 32, "top_k": 4,
                    "weights": "mxfp4 e2m1 + e8m0/32", "layer_copies": args.copies},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -96,7 +96,7 @@ def streamed_expert_bytes(desc: MoEDesc, intermediate: int | None = None) -> int
     return total
 
 
-# ---- named configurations --------------------------------------------
+# ---- named configurations --------------------------------------------------------------------
 
 GPT_OSS_20B = MoEDesc(hidden=2880, intermediate=2880, experts=32, top_k=4, quant=QUANT_MXFP4,
                       activation=ACT_SWIGLU_OAI, router=ROUTER_TOPK_SOFTMAX, expert_bias=1)

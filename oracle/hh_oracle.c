@@ -1,7 +1,7 @@
 /*
  * hh_oracle.c — fp64 CPU restatement of Hydra's HydraReference MoE path.
  *
- * TEST INFRASTRUCTURE ONLY: the checker for the HIP kernels and the timed CPU baseline.
+ * TEST INFRASTRUCTURE ONLY: what the HIP kernels are compared with, and the timed CPU baseline.
  * The product never links or loads this file.
  *
  * Every function follows a reference routine, cited file:line relative to the Hydra

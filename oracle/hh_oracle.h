@@ -3,7 +3,7 @@
  *
  * TEST INFRASTRUCTURE ONLY. Nothing in the product (hydra_amd/, include/) links, loads or
  * calls this. Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg use it,
- * and only as the checker / the timed CPU baseline.
+ * and only for comparison or as the timed CPU baseline.
  *
  * Enumerations use the numeric values of include/hydra_hip.h so a description can be handed
  * to both sides unchanged.

@@ -1,7 +1,7 @@
 """ctypes front end of oracle/liboracle.so (fp64 restatement of HydraReference).
 
 TEST INFRASTRUCTURE ONLY: used by tests/, __graft_entry__.smoke() and the cpu_baseline leg of
-bench.py as the checker / CPU baseline. Build with `make -C oracle`.
+bench.py, for comparison or as the CPU baseline. Build with `make -C oracle`.
 """
 from __future__ import annotations
 

@@ -1,6 +1,6 @@
 """GPU parity: the HIP path against the fp64 oracle and against itself.
 
-Bars (BASELINE.json north_star): dequantisation and top-k indices bit-exact; layer output
+Bars: dequantisation and top-k indices bit-exact; layer output
 within rel-L2 1e-3 of the oracle (fp32 accumulation); a T-token call bit-identical to T
 one-token calls. Every test calls the library through its C ABI.
 """

@@ -117,7 +117,7 @@ def test_gpu_mlx_router_topk_exact(bits):
 @pytest.mark.gpu
 @pytest.mark.parametrize("bits", [4, 8])
 def test_gpu_qwen_layer_with_mlx_router(bits):
-    """The Qwen-shaped layer (MLX-4 experts) with its router and shared
+    """The Qwen-shaped layer (hidden 2048, 256 experts, MLX-4) with its router and shared
     gate in MLX-affine form, decode and prefill, against the oracle and token-by-token."""
     import torch
     from hydra_amd.layer import Context, MoELayer
